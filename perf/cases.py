@@ -34,7 +34,7 @@ from mfixdem.ensemble import Ensemble  # noqa: E402
 from mfixdem.system import DemSystem  # noqa: E402
 
 _D = 1.0e-3      # sphere diameter scale (m)
-_DT = 1.0e-5     # solid time step (s)
+_DT = 2.0e-6     # solid time step (s): a fiftieth of the shortest collision, about
 _GRAV = -9.81
 _RLM = float(np.float32(1.2))
 
@@ -195,6 +195,7 @@ def _bed(c, seed):
             p.desgridsearch_imax, p.desgridsearch_jmax, p.desgridsearch_kmax = 26, 52, 26
         p.imax, p.jmax, p.kmax = cells
         p.coupled = 1
+        p.des_epg_clip = 0.35
         p.drag_type = abi.DRAG_WEN_YU if c.get("drag") == "WEN_YU" else abi.DRAG_GIDASPOW
         if c.get("scheme") == "HAT":
             p.interp_scheme = abi.INTERP_LINEAR_HAT
@@ -660,7 +661,7 @@ class _Dem64:
                 rop[m] = np.where(self.fluid, a, a * self.cvol)
         eps = sum(rop[m] / p.ro_s0[m] for m in range(p.nphases))
         self.rop = rop
-        self.ep[self.fluid] = 1.0 - np.minimum(1.0, eps[self.fluid])
+        self.ep[self.fluid] = 1.0 - np.minimum(1.0 - p.des_epg_clip, eps[self.fluid])
 
     def _drag_coefficient(self):
         """F_GP, the gas velocity at the particles, P_FORCE there."""
