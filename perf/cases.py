@@ -41,17 +41,17 @@ _RLM = float(np.float32(1.2))
 
 def listed():
     return [
-        # a few spheres, as the reference's small test cases: launches and
-        # latency only (Adams-Bashforth, two phases)
+        # a few spheres without gravity, as the reference's small impact
+        # tests: launches and latency only (Adams-Bashforth, two phases)
         {"name": "impacts_93", "kind": "march", "n": 93, "phi": 0.25, "model": "LSD", "ab2": True,
-         "phases": 2, "mixed": False, "steps": 100},
-        # the smallest system of a parameter sweep
-        {"name": "bed_2k", "kind": "march", "n": 2003, "phi": 0.30, "model": "LSD", "ab2": False,
+         "phases": 2, "mixed": False, "steps": 100, "gravity": False},
+        # the smallest system of a parameter sweep, settled
+        {"name": "bed_2k", "kind": "march", "n": 2003, "phi": 0.60, "model": "LSD", "ab2": False,
          "phases": 1, "mixed": False, "steps": 100},
-        # the plain settling bed of 20,000 spheres
-        {"name": "bed_20k", "kind": "march", "n": 20000, "phi": 0.30, "model": "LSD", "ab2": False,
+        # the plain bed of 20,000 spheres, settled
+        {"name": "bed_20k", "kind": "march", "n": 20000, "phi": 0.60, "model": "LSD", "ab2": False,
          "phases": 1, "mixed": False, "steps": 250},
-        # a dense bed at rest: most listed pairs touch (Hertz, two phases,
+        # a large dense bed: most listed pairs touch (Hertz, two phases,
         # Adams-Bashforth)
         {"name": "dense_300k", "kind": "march", "n": 301057, "phi": 0.60, "model": "HERTZ",
          "ab2": True, "phases": 2, "mixed": False, "steps": 100},
@@ -186,6 +186,8 @@ def _bed(c, seed):
     _collisions(p, c.get("model", "HERTZ"), c.get("ab2", False), phases, c.get("mixed", False))
     p.max_pip = n
     p.max_radius = 0.5 * float(d.max())
+    if not c.get("gravity", True):
+        p.grav[:] = [0.0, 0.0, 0.0]
     phase = rng.integers(1, phases + 1, n).astype(np.int32)
     rho = 2500.0 - 500.0 * (phase - 1)
     if coupled:   # cubic gas cells of two diameters
