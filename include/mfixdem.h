@@ -79,11 +79,9 @@ enum {
   MFIXDEM_DEBUG_REFERENCE_DEPOSITION = 4, /* eps_s deposition summed in the reference's
                                      serial order (PIC lists, node gather) instead
                                      of order-independent fixed-point sums */
-  MFIXDEM_DEBUG_NO_GRAPH = 8      /* launch every step eagerly, no hipGraph capture:
-                                     for hosts that drive several handles from
-                                     different threads (a capture in progress on
-                                     one thread makes the HIP runtime refuse
-                                     legacy-stream copies and frees on others) */
+  MFIXDEM_DEBUG_NO_GRAPH = 8      /* accepted, without effect: every step is launched
+                                     eagerly and no hipGraph is captured, so hosts may
+                                     drive several handles from different threads */
 };
 /* kernel groups reported by mfixdem_get_kernel_times */
 enum { MFIXDEM_TIME_STEP = 0, MFIXDEM_TIME_REBUILD = 1, MFIXDEM_TIME_GAS = 2,
@@ -302,7 +300,7 @@ int32_t mfixdem_init(mfixdem_handle* h);
    COMP_MEAN_FIELDS when coupled.  Runs the fused kernels. */
 int32_t mfixdem_step(mfixdem_handle* h, int32_t nn);
 /* nsteps consecutive DES_TIME_STEP calls, NN = nn_first .. nn_first+nsteps-1;
-   the runs of steps between rebuilds are replayed from a captured hipGraph. */
+   all launches are queued on the handle's stream. */
 int32_t mfixdem_run(mfixdem_handle* h, int32_t nn_first, int32_t nsteps);
 /* Waits for the handle's stream.  Conditions the reference treats as fatal
    that arise on the device (a coincident contact pair, calc_force_dem.f:
@@ -423,10 +421,9 @@ int32_t mfixdem_get_device_bytes(mfixdem_handle* h, int64_t* bytes);
    parameter sweeps and ensembles of pure-DEM systems of uneven size.  One
    handle holds nsys systems, p[s] giving each its own parameters, box,
    capacity (max_pip) and time step; every launch -- the step kernel and
-   each rebuild stage -- covers all systems at once, and the runs of steps
-   between rebuilds are replayed from one captured hipGraph.  Each system
-   evolves exactly as it would in its own handle.  All systems must share
-   precision, neighbor_search_n and remove_rogue, use the grid search and be
+   each rebuild stage -- covers all systems at once.  Each system evolves
+   exactly as it would in its own handle.  All systems must share precision,
+   neighbor_search_n and remove_rogue, use the grid search and be
    uncoupled (else MFIXDEM_ERR_UNSUPPORTED).  mfixdem_init / step / run /
    synchronize / get_status / destroy work on the ensemble handle; the
    single-system state calls return MFIXDEM_ERR_ARG on it. */

@@ -4,8 +4,11 @@
 // one stream.  The time step is a fused particle kernel (walls, pairs, drag,
 // integrator, fluid-cell locate) plus, when gas-coupled, the deposition
 // kernels; every NEIGHBOR_SEARCH_N steps the particles are re-sorted and the
-// neighbour list rebuilt.  Runs of steps between rebuilds are replayed from
-// captured hipGraphs.
+// neighbour list rebuilt.  Steps are launched eagerly: one launch costs the
+// host 4 us (3 KB of arguments) and a chain of kernels longer than that runs
+// back to back, while replaying a one-step hipGraph cost 13 us a step and each
+// rebuild new captures (93 spheres: 21.9 -> 13.8 us a step; 120,000: 46 -> 42;
+// the coupled 1M-sphere bed: 227 -> 216).
 #include <hip/hip_runtime.h>
 #include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
@@ -159,11 +162,6 @@ struct mfixdem_handle {
   mfixdem_status st{};
   bool inited = false, gas_set = false, first_pass = true, binned = false;
   int debug = 0;
-  // graphs: [cur parity][deposition buffer]
-  hipGraphExec_t graph[2][2]{};
-  // executable graphs replaced while launches of them may still be queued on
-  // the stream; destroyed once the stream has drained (reap_graphs)
-  std::vector<hipGraphExec_t> retired;
   // kernel timing
   // kernel timing: a pool of events recorded around each timed launch and
   // read back in one go, so launches queue back to back while timed
@@ -278,27 +276,8 @@ StepPtrs step_ptrs(mfixdem_handle* h) {
   return a;
 }
 
-// The captured graphs no longer match the handle's buffers: they are
-// retired, not destroyed, because launches of them may still be queued on
-// the handle's stream; sync_stream destroys them once the stream has drained.
-void invalidate_graphs(mfixdem_handle* h) {
-  for (auto& row : h->graph)
-    for (auto& g : row)
-      if (g) {
-        h->retired.push_back(g);
-        g = nullptr;
-      }
-}
-void reap_graphs(mfixdem_handle* h) {
-  for (hipGraphExec_t g : h->retired) (void)hipGraphExecDestroy(g);
-  h->retired.clear();
-}
 // Waits for the handle's stream; every wait goes through here.
-hipError_t sync_stream(mfixdem_handle* h) {
-  const hipError_t e = hipStreamSynchronize(h->stream);
-  if (e == hipSuccess) reap_graphs(h);
-  return e;
-}
+hipError_t sync_stream(mfixdem_handle* h) { return hipStreamSynchronize(h->stream); }
 
 // New particle state: deposition restarts from buffer 0 with both
 // fixed-point node-sum buffers zero (the last step left its sums in one of
@@ -530,7 +509,6 @@ int32_t do_bin(mfixdem_handle* h) {
     HIPOK(hipGetLastError());
   }
   h->binned = true;
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 
@@ -729,7 +707,6 @@ int32_t do_neighbour(mfixdem_handle* h) {
   }
   h->binned = false;
   h->st.rebuilds++;
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 
@@ -856,15 +833,6 @@ bool rebin_each_step(const mfixdem_handle* h) {
   return h->S.p.coupled && !h->S.p.des_explicitly_coupled;
 }
 
-// the part of a step that is identical between rebuilds (graph-capturable)
-int32_t plain_step_body(mfixdem_handle* h) {
-  CHECKRC(launch_step<kModeFused>(h));
-  h->cur = 1 - h->cur;
-  h->pcur = 1 - h->pcur;
-  if (rebin_each_step(h)) CHECKRC(gas_tail(h));
-  return MFIXDEM_OK;
-}
-
 // The free global ids, from the particle states (at init, and after rogue
 // particles have been removed).
 int32_t refresh_free_gids(mfixdem_handle* h) {
@@ -948,50 +916,26 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
 int32_t one_step(mfixdem_handle* h, int32_t nn) {
   if (h->P.nbc) return bc_step(h, nn);
   const bool rebuild = (nn == 1) || (nn % h->S.p.neighbor_search_n == 0);
-  const bool use_graph = !rebuild && !h->first_pass && !timing(h) &&
-                         !(h->debug & (MFIXDEM_DEBUG_STORE_FORCES | MFIXDEM_DEBUG_NO_GRAPH));
-  if (use_graph) {
-    hipGraphExec_t& g = h->graph[h->cur][h->fb];
-    if (!g) {
-      const int c0 = h->cur, p0 = h->pcur, f0 = h->fb;
-      HIPOK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-      int32_t rc = plain_step_body(h);
-      hipGraph_t graph = nullptr;
-      hipError_t e = hipStreamEndCapture(h->stream, &graph);
-      h->cur = c0;
-      h->pcur = p0;
-      h->fb = f0;
-      if (rc != MFIXDEM_OK) return rc;
-      HIPOK(e);
-      HIPOK(hipGraphInstantiate(&g, graph, nullptr, nullptr, 0));
-      (void)hipGraphDestroy(graph);
-    }
-    HIPOK(hipGraphLaunch(g, h->stream));
-    h->cur = 1 - h->cur;
-    h->pcur = 1 - h->pcur;
-    if (h->S.p.coupled) h->fb = 1 - h->fb;
-  } else {
+  t_begin(h);
+  CHECKRC(launch_step<kModeFused>(h));
+  t_end(h, kTimeStep);
+  h->cur = 1 - h->cur;
+  h->pcur = 1 - h->pcur;
+  if (rebuild) {
     t_begin(h);
-    CHECKRC(launch_step<kModeFused>(h));
-    t_end(h, kTimeStep);
-    h->cur = 1 - h->cur;
-    h->pcur = 1 - h->pcur;
-    if (rebuild) {
-      t_begin(h);
-      if (fused_dep(h)) {  // the rebuild reorders the slots the removal queue names
-        hipLaunchKernelGGL(k_apply_removals, dim3(1), dim3(kBS), 0, h->stream, h->rm_cnt + h->fb,
-                           h->rm_list, h->state[h->tw], h->radius[h->tw]);
-        HIPOK(hipGetLastError());
-      }
-      CHECKRC(do_bin(h));
-      CHECKRC(do_neighbour(h));
-      t_end(h, kTimeRebuild);
+    if (fused_dep(h)) {  // the rebuild reorders the slots the removal queue names
+      hipLaunchKernelGGL(k_apply_removals, dim3(1), dim3(kBS), 0, h->stream, h->rm_cnt + h->fb,
+                         h->rm_list, h->state[h->tw], h->radius[h->tw]);
+      HIPOK(hipGetLastError());
     }
-    if (rebin_each_step(h)) {
-      t_begin(h);
-      CHECKRC(gas_tail(h));
-      t_end(h, kTimeGas);
-    }
+    CHECKRC(do_bin(h));
+    CHECKRC(do_neighbour(h));
+    t_end(h, kTimeRebuild);
+  }
+  if (rebin_each_step(h)) {
+    t_begin(h);
+    CHECKRC(gas_tail(h));
+    t_end(h, kTimeGas);
   }
   h->first_pass = false;
   h->st.steps++;
@@ -1110,7 +1054,6 @@ int32_t upload_ensemble(mfixdem_handle* h) {
       ST[q] = 1;
     }
   }
-  invalidate_graphs(h);
   h->cur = h->pcur = h->tw = h->lt = 0;
   CHECKRC(reset_deposit(h));
   HIPOK(hipMemcpy(h->pos[0], h->st_pos.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
@@ -1386,8 +1329,6 @@ int32_t mfixdem_create(const mfixdem_params* p, mfixdem_handle** out) {
 int32_t mfixdem_destroy(mfixdem_handle* h) {
   if (!h) return MFIXDEM_ERR_ARG;
   if (h->stream) (void)sync_stream(h);
-  invalidate_graphs(h);
-  reap_graphs(h);
   for_each_buffer(h, [](auto*& p) { dfree(p); });
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
@@ -1448,7 +1389,6 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
     }
   }
   HIPOK(sync_stream(h));  // steps already queued still use the buffers
-  invalidate_graphs(h);
   h->cur = h->pcur = h->tw = h->lt = 0;
   CHECKRC(reset_deposit(h));
   HIPOK(hipMemcpy(h->pos[0], P3.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
@@ -1518,7 +1458,6 @@ int32_t mfixdem_set_facets(mfixdem_handle* h, int32_t nf, const double* vertex,
   setup_facets(h->S, nf, vertex, normal, default_walls != 0);
   small_facets(h->S, h->P);
   CHECKRC(upload_facets(h, h->S));
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 
@@ -1531,8 +1470,7 @@ int32_t mfixdem_set_wall_motion(mfixdem_handle* h, int32_t first, int32_t count,
     return MFIXDEM_ERR_ARG;
   HIPOK(sync_stream(h));
   set_wall_motion(h->S, first, count, vel, omega, rot_center);
-  small_facets(h->S, h->P);  // facets in the kernel arguments: graphs recorded again
-  invalidate_graphs(h);
+  small_facets(h->S, h->P);  // facets in the kernel arguments
   std::vector<FacetDev> fac;
   facets_dev(h->S, fac);
   if (!fac.empty())
@@ -1565,7 +1503,6 @@ int32_t mfixdem_set_dem_bcs(mfixdem_handle* h, int32_t n, const mfixdem_dem_bc* 
   dfree(h->d_seeds);
   h->dbc = DemBoundaries{};
   h->P.nbc = 0;
-  invalidate_graphs(h);
   if (n == 0) return MFIXDEM_OK;
   const int64_t N = h->n;
   CHECKRC(dalloc(&h->d_bcs, n));
@@ -1626,7 +1563,6 @@ int32_t mfixdem_set_gas(mfixdem_handle* h, const double* u_g, const double* v_g,
   HIPOK(hipGetLastError());
   HIPOK(sync_stream(h));  // the caller's arrays are free again on return
   h->gas_set = true;
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 
@@ -1642,7 +1578,6 @@ int32_t mfixdem_set_gas_pressure(mfixdem_handle* h, const double* p_g) {
                      h->fluid, h->gas_stage, h->p_force);
   HIPOK(hipGetLastError());
   HIPOK(sync_stream(h));
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 
@@ -1725,7 +1660,6 @@ int32_t mfixdem_synchronize(mfixdem_handle* h) {
 
 int32_t mfixdem_calc_force_dem(mfixdem_handle* h) {
   if (!h || !h->inited) return h ? MFIXDEM_ERR_NOT_READY : MFIXDEM_ERR_ARG;
-  invalidate_graphs(h);
   CHECKRC(launch_step<kModeForce>(h));
   h->pcur = 1 - h->pcur;
   return MFIXDEM_OK;
@@ -1922,9 +1856,8 @@ int32_t mfixdem_drag_gs_gas_noalloc(mfixdem_handle* h, double* f_gds, double* dr
 
 int32_t mfixdem_set_debug(mfixdem_handle* h, int32_t flags) {
   if (!h) return MFIXDEM_ERR_ARG;
-  HIPOK(sync_stream(h));  // queued graph launches finish under the old flags
+  HIPOK(sync_stream(h));  // queued steps finish under the old flags
   h->debug = flags;
-  invalidate_graphs(h);
   return MFIXDEM_OK;
 }
 

@@ -90,9 +90,6 @@ class SweepServer:
                 req.params, req.parts = req.make()
             s = DemSystem(req.params)
             try:
-                # several handles are driven from different threads: no
-                # stream capture (a pure-DEM step is one kernel anyway)
-                s.set_debug(abi.DEBUG_NO_GRAPH)
                 s.set_particles(req.parts)
                 s.init()
                 nn, left = 1, req.nsteps

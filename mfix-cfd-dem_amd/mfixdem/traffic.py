@@ -1,7 +1,7 @@
 """HBM traffic of the fused step kernel from rocprofv3 counters.
 
-  run        build the 1M-sphere fluidised bed, step it eagerly (no graph, so
-             every launch is a dispatch the counters see), then launch a
+  run        build the 1M-sphere fluidised bed, step it (every
+             launch is a dispatch the counters see), then launch a
              plain device-to-device copy of known size for calibration.
   summarize  read two counter_collection.csv files (one FETCH_SIZE pass,
              one WRITE_SIZE pass), scale each counter by what it reads for
@@ -47,7 +47,6 @@ def run(steps=12):
     s = DemSystem(p)
     s.set_particles(parts)
     s.set_gas(gas)
-    s.set_debug(abi.DEBUG_NO_GRAPH)
     s.init()
     s.run(1, 30)          # past the first rebuild and warm-up
     s.run(31, steps)
