@@ -81,7 +81,8 @@ struct StepPtrs {
   uint8_t* wmask;
   int* wfid;
   double* wpft;
-  const int *nbr_start, *nbr_split, *nbr, *nbr_pid;
+  const int *nbr_start, *nbr, *nbr_pid;
+  const uint8_t* nbr_row;       // per entry: slot of its row mod 64, kRowOwn set for own entries
   const double* pft_in;         // tangential history [3*pair + d], valid where pfl is 1
   double* pft_out;
   const uint8_t* pfl_in;        // 1: the pair's history is set; 0: it is zero (pft unread)
@@ -504,39 +505,57 @@ __device__ __forceinline__ void keep_history(const StepPtrs& a, int pid) {
     for (int c = 0; c < 3; c++) a.pft_out[3 * pid + c] = a.pft_in[3 * pid + c];
 }
 
-// One pair entry of a row (calc_force_dem.f:210-412): particle ip (position
-// xp, radius rp) is L of the pair (owner, own row) or I (incoming row);
-// partner j, pair id pid.
-// Writes the pair's new history when ip owns it and returns 1 with the
-// increments of ip's force and torque in d[0..5] when the pair is in
-// contact; returns 0 when it adds nothing.
-template <bool MIXED, bool BATCH>
-__device__ __forceinline__ int pair_entry(const DevParams& P0, const StepPtrs& a,
-                                          const BatchDev& B, int ip, const double xp[3],
-                                          double rp, int j, int pid, bool owner, double d[6]) {
-  const int S = P0.stride;
-  const DevParams& P = sys_params<BATCH>(P0, B, ip);
+// Bit of StepPtrs::nbr_row: the entry belongs to the own part of its row
+// (the row's particle is L of the pair), below it the row's slot mod 64.
+constexpr unsigned kRowOwn = 64u;
+
+// The contact test of one pair entry (calc_force_dem.f:210-262): particle
+// (xp, rp) is L of the pair (owner, own row) or I (incoming row); partner j,
+// pair id pid.  Returns whether the pair is in contact; the histories of the
+// pairs that are not are written here.
+__device__ __forceinline__ bool pair_touches(const StepPtrs& a, int S, const double xp[3],
+                                             double rp, int j, int pid, bool owner) {
   const uint8_t stj = a.state[j];
   double xj[3];
   load3(a.pos, S, j, xj);
   const double rj = a.radius[j];
   if (stj == 0) {  // IF(IS_NONEXISTENT(I)) CYCLE: history kept
     if (owner) keep_history(a, pid);
-    return 0;
+    return false;
   }
-  // contact test in the reference's orientation: |x_I - x_L|^2, r_L + r_I
-  const double r_lm = owner ? rp + rj : rj + rp;
-  const double d0 = owner ? xj[0] - xp[0] : xp[0] - xj[0];
-  const double d1 = owner ? xj[1] - xp[1] : xp[1] - xj[1];
-  const double d2 = owner ? xj[2] - xp[2] : xp[2] - xj[2];
+  // in the reference's orientation |x_I - x_L|^2 and r_L + r_I; the square
+  // and the sum are the same the other way round
+  const double r_lm = rp + rj;
+  const double d0 = xj[0] - xp[0], d1 = xj[1] - xp[1], d2 = xj[2] - xp[2];
   const double dm = d0 * d0 + d1 * d1 + d2 * d2;
   const double rs = r_lm - kSmall;
   if (dm > rs * rs) {  // PFT_NEIGHBOR(:,CC) = 0: the flag says so, no 24-byte write
     if (owner) a.pfl_out[pid] = 0;
-    return 0;
+    return false;
   }
+  if (dm == 0.0) {  // counted once per pair, on the owner's row
+    if (owner) {
+      atomicAdd(&a.flags[kFlagZeroDist], 1);
+      keep_history(a, pid);
+    }
+    return false;
+  }
+  return true;
+}
+
+// The contact law of a pair that touches (calc_force_dem.f:263-412), for the
+// row's particle ip at xp, rp: the increments of its force and torque in
+// d[0..5]; the owner's row writes the pair's new history.
+template <bool MIXED, bool BATCH>
+__device__ __forceinline__ void pair_contact(const DevParams& P0, const StepPtrs& a,
+                                             const BatchDev& B, int ip, const double xp[3],
+                                             double rp, int j, int pid, bool owner, double d[6]) {
+  const int S = P0.stride;
+  const DevParams& P = sys_params<BATCH>(P0, B, ip);
   PairIn in;
-  double vj[3], wj[3], vp[3], wp[3];
+  double xj[3], vj[3], wj[3], vp[3], wp[3];
+  load3(a.pos, S, j, xj);
+  const double rj = a.radius[j];
   load3(a.vel, S, j, vj);
   load3(a.omega, S, j, wj);
   load3(a.vel, S, ip, vp);
@@ -561,98 +580,126 @@ __device__ __forceinline__ int pair_entry(const DevParams& P0, const StepPtrs& a
   if (a.pfl_in[pid])
     for (int c = 0; c < 3; c++) hin[c] = a.pft_in[3 * pid + c];
   PairOut o;
-  const int r = MIXED ? pair_force_mixed(P, in, hin, o) : pair_force_fp64(P, in, hin, o);
-  if (r == 2) {  // counted once per pair, on the owner's row
-    if (owner) {
-      atomicAdd(&a.flags[kFlagZeroDist], 1);
-      keep_history(a, pid);
-    }
-    return 0;
-  }
+  if (MIXED) pair_force_mixed(P, in, hin, o);
+  else pair_force_fp64(P, in, hin, o);
   if (owner) {
     for (int c = 0; c < 3; c++) a.pft_out[3 * pid + c] = o.pft[c];
     a.pfl_out[pid] = 1;
     if (P0.store_forces) atomicAdd(&a.flags[kFlagContacts], 1);
-    for (int c = 0; c < 3; c++) d[c] = o.fct[c];
-    for (int c = 0; c < 3; c++) d[3 + c] = o.tl[c];
-  } else {  // FC(I) = FC(I) - FC_pair: adding the negation rounds the same
-    for (int c = 0; c < 3; c++) d[c] = -o.fct[c];
-    for (int c = 0; c < 3; c++) d[3 + c] = o.ti[c];
   }
-  return 1;
+  // FC(I) = FC(I) - FC_pair: adding the negation rounds the same
+  for (int c = 0; c < 3; c++) d[c] = owner ? o.fct[c] : -o.fct[c];
+  for (int c = 0; c < 3; c++) d[3 + c] = owner ? o.tl[c] : o.ti[c];
 }
 
-// The pair part of CALC_FORCE_DEM for the 64 particles of a wavefront.
-// Their rows ([incoming | own], consecutive particles) are one contiguous
-// run of entries; the lanes take the entries 64 at a time (one pair entry
-// per lane, so a long row does not hold the other lanes back), put each
-// entry's force and torque increment in LDS, and then every lane adds the
-// increments of its own row in row order -- the reference's summation
-// order, so the sums are bit-identical to a per-particle loop.  Rows of a
-// nonexistent particle only carry their history over.  Every lane of the
-// wavefront must call this (lanes past n with live = false).  The lane's
-// row is [r0, r1) with its own entries from sp on; xr is the lane's own
-// position and radius, which the lanes working on its row read from LDS.
-template <bool MIXED, bool BATCH>
-__device__ __forceinline__ void wave_pairs(const DevParams& P0, const StepPtrs& a,
-                                           const BatchDev& B, int i, int st, int r0, int sp,
-                                           int r1, const double xr[4], double fc[3],
-                                           double tow[3]) {
-  __shared__ double s_xr[kBS / 64][4][64];
-  __shared__ int s_row[kBS / 64][65];
-  __shared__ int s_split[kBS / 64][64];
-  __shared__ int s_st[kBS / 64][64];
-  __shared__ int s_hit[kBS / 64][64];
-  __shared__ double s_d[kBS / 64][6][64];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  s_row[w][lane] = r0;
-  s_split[w][lane] = sp;
-  s_st[w][lane] = st;
-  for (int c = 0; c < 4; c++) s_xr[w][c][lane] = xr[c];
-  if (lane == 63) s_row[w][64] = r1;
+// Orders the LDS accesses of a wavefront's lanes: no barrier is needed
+// between them, only that the compiler keeps them apart.
+__device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int e_first = s_row[w][0], e_last = s_row[w][64];
-  const int my1 = s_row[w][lane + 1];
-  const int wbase = i - lane;
-  for (int base = e_first; base < e_last; base += 64) {
-    const int f = base + lane;
-    int hit = 0;
-    double d[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (f < e_last) {
-      // the lane whose row holds entry f: the last p with s_row[p] <= f
-      int p = 0;
-#pragma unroll
-      for (int step = 32; step > 0; step >>= 1)
-        if (s_row[w][p + step] <= f) p += step;
-      const bool owner = f >= s_split[w][p];
-      const int pid = a.nbr_pid[f];
-      if (s_st[w][p] == 0) {
-        if (owner) keep_history(a, pid);  // rows of a removed particle keep their history
-      } else {
-        const double xp[3] = {s_xr[w][0][p], s_xr[w][1][p], s_xr[w][2][p]};
-        hit = pair_entry<MIXED, BATCH>(P0, a, B, wbase + p, xp, s_xr[w][3][p], a.nbr[f], pid,
-                                       owner, d);
+}
+
+// The pair part of CALC_FORCE_DEM for the particles of a wavefront (2^lgw of
+// them, slots wbase on, one per lane of the first 2^lgw lanes).  Their rows
+// ([incoming | own], consecutive particles) are one contiguous run of
+// entries [e0, e1).  The lanes take the entries 64 at a time, one per lane,
+// and test them for contact; the entries that touch wait in an LDS queue in
+// their order and go through the contact law 64 at a time, so that the law
+// (some 800 FP64 instructions) runs with full lanes and once per 64 contacts
+// instead of in every window that holds one.  Each batch leaves its force
+// and torque increments in LDS and every lane adds those of its own row in
+// row order -- the reference's summation order, so the sums are
+// bit-identical to a per-particle loop.  Rows of a nonexistent particle
+// (xr[3] < 0) only carry their history over.  Every lane of the wavefront
+// must call this; xr is the lane's own position and radius, which the lanes
+// working on its row read from LDS.
+template <bool MIXED, bool BATCH>
+__device__ __forceinline__ void wave_pairs(const DevParams& P0, const StepPtrs& a,
+                                           const BatchDev& B, int lgw, int wbase, int e0, int e1,
+                                           const double xr[4], double fc[3], double tow[3]) {
+  constexpr int kQueue = 128;
+  __shared__ double s_xr[kBS / 64][4][64];
+  __shared__ double s_d[kBS / 64][6][64];
+  __shared__ int q_j[kBS / 64][kQueue], q_pid[kBS / 64][kQueue];
+  __shared__ uint8_t q_row[kBS / 64][kQueue];
+  __shared__ uint8_t s_beg[kBS / 64][64], s_end[kBS / 64][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const unsigned rmask = (1u << lgw) - 1u;
+  for (int c = 0; c < 4; c++) s_xr[w][c][lane] = xr[c];
+  int j = 0, pid = 0;
+  unsigned rb = 0;
+  if (e0 + lane < e1) {
+    j = a.nbr[e0 + lane];
+    pid = a.nbr_pid[e0 + lane];
+    rb = a.nbr_row[e0 + lane];
+  }
+  wave_lds_fence();
+  int base = e0, qh = 0, qn = 0;  // next window; queue head and length
+  for (;;) {
+    if (base < e1 && qn < 64) {
+      const int jc = j, pc = pid;
+      const unsigned rc = rb;
+      const bool in = base + lane < e1;
+      const int f = base + 64 + lane;
+      if (f < e1) {  // the next window's entries, ahead of this one's tests
+        j = a.nbr[f];
+        pid = a.nbr_pid[f];
+        rb = a.nbr_row[f];
       }
-    }
-    s_hit[w][lane] = hit;
-#pragma unroll
-    for (int k = 0; k < 6; k++) s_d[w][k][lane] = d[k];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int lo = r0 > base ? r0 : base, hi = my1 < base + 64 ? my1 : base + 64;
-    for (int g = lo; g < hi; g++) {
-      const int t = g - base;
-      if (s_hit[w][t]) {
-        for (int c = 0; c < 3; c++) fc[c] = fc[c] + s_d[w][c][t];
-        for (int c = 0; c < 3; c++) tow[c] = tow[c] + s_d[w][3 + c][t];
+      bool hit = false;
+      if (in) {
+        const int p = (int)(rc & rmask);
+        const bool owner = (rc & kRowOwn) != 0u;
+        const double rp = s_xr[w][3][p];
+        if (rp < 0.0) {
+          if (owner) keep_history(a, pc);  // rows of a removed particle keep their history
+        } else {
+          const double xp[3] = {s_xr[w][0][p], s_xr[w][1][p], s_xr[w][2][p]};
+          hit = pair_touches(a, P0.stride, xp, rp, jc, pc, owner);
+        }
       }
+      const unsigned long long m = __ballot(hit);
+      if (hit) {
+        const int q = (qh + qn + __builtin_popcountll(m & ((1ull << lane) - 1ull))) & (kQueue - 1);
+        q_j[w][q] = jc;
+        q_pid[w][q] = pc;
+        q_row[w][q] = (uint8_t)rc;
+      }
+      qn += __builtin_popcountll(m);
+      base += 64;
+      if (base < e1 && qn < 64) continue;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int nb = qn < 64 ? qn : 64;
+    if (nb == 0) break;
+    s_beg[w][lane] = 0;
+    s_end[w][lane] = 0;
+    wave_lds_fence();
+    int p = -1;
+    if (lane < nb) {
+      const int q = (qh + lane) & (kQueue - 1);
+      const unsigned rc = q_row[w][q];
+      p = (int)(rc & rmask);
+      const double xp[3] = {s_xr[w][0][p], s_xr[w][1][p], s_xr[w][2][p]};
+      double d[6];
+      pair_contact<MIXED, BATCH>(P0, a, B, wbase + p, xp, s_xr[w][3][p], q_j[w][q], q_pid[w][q],
+                                 (rc & kRowOwn) != 0u, d);
+#pragma unroll
+      for (int k = 0; k < 6; k++) s_d[w][k][lane] = d[k];
+    }
+    // a row's contacts are consecutive in the batch: its first and last
+    const int before = __shfl_up(p, 1, 64), after = __shfl_down(p, 1, 64);
+    if (lane < nb && (lane == 0 || before != p)) s_beg[w][p] = (uint8_t)lane;
+    if (lane < nb && (lane == nb - 1 || after != p)) s_end[w][p] = (uint8_t)(lane + 1);
+    wave_lds_fence();
+    const int t1 = s_end[w][lane];
+    for (int t = s_beg[w][lane]; t < t1; t++) {
+      for (int c = 0; c < 3; c++) fc[c] = fc[c] + s_d[w][c][t];
+      for (int c = 0; c < 3; c++) tow[c] = tow[c] + s_d[w][3 + c][t];
+    }
+    wave_lds_fence();
+    qh = (qh + nb) & (kQueue - 1);
+    qn -= nb;
   }
 }
 
@@ -929,12 +976,15 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const DevParams& 
 // P0.fuse_dep it also deposits the particles' new positions
 // (COMP_MEAN_FIELDS0 node sums) before it ends.
 template <bool MIXED, int MODE, bool FILTER, bool BATCH = false, bool STL = false>
-__global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev B) {
+__global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev B, int lgw) {
   constexpr bool kPairs = MODE == kModeFused || MODE == kModeForce;
   constexpr bool kEarlyDrag = MODE == kModeFused && !FILTER && !BATCH;
   __shared__ double s_drag[kEarlyDrag ? 6 : 1][kBS];
-  const int i = xcd_tile(blockIdx.x, gridDim.x) * kBS + threadIdx.x;
-  const bool live = i < P0.n;
+  // a wavefront holds 2^lgw consecutive particles, one per lane of its first
+  // 2^lgw lanes (lgw = 6 in the modes without pairs)
+  const int wbase = (xcd_tile(blockIdx.x, gridDim.x) * (kBS / 64) + (int)(threadIdx.x >> 6)) << lgw;
+  const int i = wbase + (int)(threadIdx.x & 63);
+  const bool live = (int)(threadIdx.x & 63) < (1 << lgw) && i < P0.n;
   if (!kPairs && !live) return;  // the pair modes keep every lane for the wave passes
   const int S = P0.stride;
   const DevParams& P = sys_params<BATCH>(P0, B, live ? i : 0);
@@ -943,12 +993,11 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
   bool drag = false;
 
   if (kPairs) {
-    // the row bounds go out with the particle's own loads
-    const int n = P0.n;
-    const int r0 = a.nbr_start[live ? i : n];
-    const int sp = live ? a.nbr_split[i] : r0;
-    const int r1 = a.nbr_start[live ? i + 1 : n];
-    double xr[4] = {0.0, 0.0, 0.0, 0.0};
+    // the bounds of the wavefront's entries go out with the particles' loads
+    const int w0 = __builtin_amdgcn_readfirstlane(wbase);
+    const int e0 = a.nbr_start[w0 < P0.n ? w0 : P0.n];
+    const int e1 = a.nbr_start[w0 + (1 << lgw) < P0.n ? w0 + (1 << lgw) : P0.n];
+    double xr[4] = {0.0, 0.0, 0.0, -1.0};
     if (live && st != 0) {
       double pos[3], vel[3], om[3];
       load3(a.pos, S, i, pos);
@@ -1041,7 +1090,7 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
       if (wm != wm0) a.wmask[i] = wm;
     }
     // ---- pairs (calc_force_dem.f:180-412), summed after the walls
-    wave_pairs<MIXED, BATCH>(P0, a, B, i, st, r0, sp, r1, xr, fc, tow);
+    wave_pairs<MIXED, BATCH>(P0, a, B, lgw, w0, e0, e1, xr, fc, tow);
   }
   DepIn dep;
   if (live)
@@ -2388,13 +2437,15 @@ __global__ __launch_bounds__(kBS) void k_place(int n, const int* own_cnt, int* o
                                                uint64_t* own_key, const int* pair_base,
                                                const int* nbr_start, const int* in_cnt,
                                                int* nbr_split, int* in_cur, int* nbr,
-                                               int* nbr_pid, uint8_t* pfl_new,
+                                               int* nbr_pid, uint8_t* nbr_row, uint8_t* pfl_new,
                                                PlaceGuard pg) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n || !place_ok(pg)) return;
   const int split = nbr_start[i] + in_cnt[i];
   nbr_split[i] = split;
   const int cnt = own_cnt[i];
+  for (int e = nbr_start[i]; e < split + cnt; e++)
+    nbr_row[e] = (uint8_t)((i & 63) | (e < split ? 0u : kRowOwn));
   if (cnt == 0) return;
   if (own_key && cnt > 1) sort_own_row(own_tmp + i, own_key + i, (size_t)n, cnt);
   const int pb = pair_base[i];

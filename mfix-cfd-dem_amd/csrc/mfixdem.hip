@@ -103,6 +103,7 @@ struct mfixdem_handle {
   int row_kernel = MFIXDEM_ROWS_THREAD;
   int *nbr_start[2]{}, *nbr_split[2]{}, *pair_base[2]{};
   int *nbr[2]{}, *nbr_pid[2]{};
+  uint8_t* nbr_row[2]{};        // row of each entry within its 64 slots, own / incoming
   int64_t nbr_cap[2]{0, 0};
   double* pft[2]{};
   uint8_t* pfl[2]{};            // per pair: 1 when pft holds the history, 0 when it is zero
@@ -256,8 +257,8 @@ StepPtrs step_ptrs(mfixdem_handle* h) {
   a.cell_fmask = h->cell_fmask;
   a.fac = h->fac; a.dg_foff = h->dg_foff; a.dg_fids = h->dg_fids;
   a.wmask = h->wmask[t]; a.wfid = h->wfid[t]; a.wpft = h->wpft[t];
-  a.nbr_start = h->nbr_start[l]; a.nbr_split = h->nbr_split[l];
-  a.nbr = h->nbr[l]; a.nbr_pid = h->nbr_pid[l];
+  a.nbr_start = h->nbr_start[l];
+  a.nbr = h->nbr[l]; a.nbr_pid = h->nbr_pid[l]; a.nbr_row = h->nbr_row[l];
   a.pft_in = h->pft[p]; a.pft_out = h->pft[1 - p];
   a.pfl_in = h->pfl[p]; a.pfl_out = h->pfl[1 - p];
   a.fc = h->fc; a.tow = h->tow; a.fc_id = h->fc_id; a.tow_id = h->tow_id;
@@ -346,6 +347,25 @@ void t_end(mfixdem_handle* h, int slot) {
   h->ev_open = -1;
 }
 
+// Particles per wavefront of the step kernel, 2^lgw.  With 64 the lanes are
+// full in the per-particle part and a wavefront walks r entries per particle
+// (r = 2 pairs / particle) in r windows of 64, one after another.  Fewer
+// particles shorten that walk and spread it over more wavefronts, at the
+// price of idle lanes in the per-particle part, which pays while the chip
+// (1,024 SIMDs) has room: always up to one wavefront per SIMD, and beyond
+// that the more the longer the rows are.  Measured per step (64 / 32 / 16 / 8
+// particles): 2,003 settled spheres, r = 11.5, 44 / 34 / 28 / 24 us; 20,000,
+// r = 12.6, 43 / 32 / 28 / 28; 301,057, r = 13, 129 / 121 / 133 / 172;
+// 120,000 mixed, r = 8, 33 / 32 / 36 / 45; 150,000 coupled, r = 5, 75 / 81 /
+// 96 / 128 (with the transfers of its fluid step).
+int step_lgw(const mfixdem_handle* h) {
+  const double r = 0.5 * (double)h->n_pairs / std::max(h->n, 1);  // r / 4
+  const double room = 1024.0 * std::max(1.0, r * r);
+  int lgw = 6;
+  while (lgw > 3 && (double)(h->n >> (lgw - 1)) <= room) lgw--;
+  return lgw;
+}
+
 template <int MODE>
 int32_t launch_step(mfixdem_handle* h) {
   DevParams P = h->P;
@@ -353,28 +373,30 @@ int32_t launch_step(mfixdem_handle* h) {
   P.store_forces = (h->debug & MFIXDEM_DEBUG_STORE_FORCES) ? 1 : 0;
   P.fuse_dep = (MODE == kModeFused && fused_dep(h)) ? 1 : 0;
   StepPtrs a = step_ptrs(h);
-  const dim3 grid(nblk(h->n)), blk(kBS);
+  const int lgw = (MODE == kModeFused || MODE == kModeForce) ? step_lgw(h) : 6;
+  const int per = (kBS / 64) << lgw;
+  const dim3 grid((h->n + per - 1) / per), blk(kBS);
   const bool mixed = h->S.p.precision == MFIXDEM_MIXED;
   const BatchDev B = h->B;
   if (h->nsys > 1) {  // ensembles: pure DEM, per-system parameter tables
-    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, false, true>), grid, blk, 0, h->stream, P, a, B);
-    else hipLaunchKernelGGL((k_step<false, MODE, false, true>), grid, blk, 0, h->stream, P, a, B);
+    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+    else hipLaunchKernelGGL((k_step<false, MODE, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
   } else if (P.nfs == 0) {  // more facets than wall slots: facet table and slot search
     const bool filt = h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012;
     if (filt && mixed)
-      hipLaunchKernelGGL((k_step<true, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B);
+      hipLaunchKernelGGL((k_step<true, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else if (filt)
-      hipLaunchKernelGGL((k_step<false, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B);
+      hipLaunchKernelGGL((k_step<false, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else if (mixed)
-      hipLaunchKernelGGL((k_step<true, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B);
+      hipLaunchKernelGGL((k_step<true, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else
-      hipLaunchKernelGGL((k_step<false, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B);
+      hipLaunchKernelGGL((k_step<false, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
   } else if (h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012) {
-    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, true>), grid, blk, 0, h->stream, P, a, B);
-    else hipLaunchKernelGGL((k_step<false, MODE, true>), grid, blk, 0, h->stream, P, a, B);
+    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+    else hipLaunchKernelGGL((k_step<false, MODE, true>), grid, blk, 0, h->stream, P, a, B, lgw);
   } else {
-    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, false>), grid, blk, 0, h->stream, P, a, B);
-    else hipLaunchKernelGGL((k_step<false, MODE, false>), grid, blk, 0, h->stream, P, a, B);
+    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, false>), grid, blk, 0, h->stream, P, a, B, lgw);
+    else hipLaunchKernelGGL((k_step<false, MODE, false>), grid, blk, 0, h->stream, P, a, B, lgw);
   }
   HIPOK(hipGetLastError());
   return MFIXDEM_OK;
@@ -385,8 +407,10 @@ int32_t ensure_list_capacity(mfixdem_handle* h, int nl, int64_t entries) {
   const int64_t cap = std::max<int64_t>(entries + entries / 4, 1024);
   dfree(h->nbr[nl]);
   dfree(h->nbr_pid[nl]);
+  dfree(h->nbr_row[nl]);
   CHECKRC(dalloc(&h->nbr[nl], cap));
   CHECKRC(dalloc(&h->nbr_pid[nl], cap));
+  CHECKRC(dalloc(&h->nbr_row[nl], cap));
   h->nbr_cap[nl] = cap;
   return MFIXDEM_OK;
 }
@@ -582,7 +606,7 @@ int32_t do_neighbour(mfixdem_handle* h) {
     hipLaunchKernelGGL(k_place, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->own_cnt,
                        h->own_tmp, nsq || wave_rows ? nullptr : h->own_key, h->pair_base[nl],
                        h->nbr_start[nl], h->in_cnt, h->nbr_split[nl], h->in_cur, h->nbr[nl],
-                       h->nbr_pid[nl], cp.pfl_new, pg);
+                       h->nbr_pid[nl], h->nbr_row[nl], cp.pfl_new, pg);
     hipLaunchKernelGGL(k_carry, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->bin_inv, cp,
                        h->pair_base[nl], h->nbr_split[nl], h->nbr_start[nl], h->nbr[nl], pg);
     hipLaunchKernelGGL(k_sort_in, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->gid[t],
@@ -1094,7 +1118,7 @@ void for_each_buffer(mfixdem_handle* h, F f) {
     f(h->racc[b]); f(h->gid[b]); f(h->fcell[b]); f(h->dgc[b]);
     f(h->state[b]); f(h->phase[b]); f(h->wmask[b]); f(h->wfid[b]); f(h->wpft[b]);
     f(h->keys[b]); f(h->vals[b]); f(h->nbr_start[b]); f(h->nbr_split[b]);
-    f(h->pair_base[b]); f(h->nbr[b]); f(h->nbr_pid[b]); f(h->pft[b]); f(h->pfl[b]);
+    f(h->pair_base[b]); f(h->nbr[b]); f(h->nbr_pid[b]); f(h->nbr_row[b]); f(h->pft[b]); f(h->pfl[b]);
     f(h->rops_fix[b]);
   }
   f(h->fc); f(h->tow); f(h->fc_id); f(h->tow_id); f(h->sort_tmp); f(h->rm_cnt); f(h->rm_list); f(h->f_gp); f(h->drag_fc);
