@@ -1414,7 +1414,24 @@ __device__ __forceinline__ T block_excl_scan(T v, T* total, T* lds) {
 constexpr int kScanPer = 4;
 constexpr int kScanTile = kBS * kScanPer;
 
-// exclusive scan of in[0..n) into out[0..n], out[n] = total (3 launches)
+// The sum of a[0..m) in every thread of the workgroup.
+template <typename T>
+__device__ __forceinline__ T block_sum(const T* a, int m, T* lds) {
+  T s = 0;
+  for (int q = threadIdx.x; q < m; q += kBS) s += a[q];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = 0;
+  for (int w = 0; w < kBS / 64; w++) s += lds[w];
+  return s;
+}
+
+// Exclusive scan of in[0..n) into out[0..n], out[n] = total, in two launches
+// of one workgroup per tile: each tile scanned by itself, then every
+// workgroup sums the totals of the tiles before its own (a launch of its own
+// for those took 4.5 us a rebuild, this sum nothing that shows).
 __global__ __launch_bounds__(kBS) void k_scan_tiles(const int* in, int* out, int n, int* bsum) {
   __shared__ int lds[kBS / 64 + 1];
   const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
@@ -1432,28 +1449,14 @@ __global__ __launch_bounds__(kBS) void k_scan_tiles(const int* in, int* out, int
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(kBS) void k_scan_sums(int* bsum, int nb) {
-  __shared__ int lds[kBS / 64 + 1];
-  const int per = (nb + kBS - 1) / kBS;
-  const int b0 = threadIdx.x * per;
-  int s = 0;
-  for (int q = 0; q < per; q++)
-    if (b0 + q < nb) s += bsum[b0 + q];
-  int tot;
-  int pre = block_excl_scan(s, &tot, lds);
-  for (int q = 0; q < per; q++)
-    if (b0 + q < nb) {
-      const int t = bsum[b0 + q];
-      bsum[b0 + q] = pre;
-      pre += t;
-    }
-  if (threadIdx.x == 0) bsum[nb] = tot;
-}
-
-__global__ __launch_bounds__(kBS) void k_scan_add(int* out, int n, const int* bsum, int nb) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i < n) out[i] += bsum[i / kScanTile];
-  if (i == 0) out[n] = bsum[nb];
+__global__ __launch_bounds__(kBS) void k_scan_add(int* out, int n, const int* bsum) {
+  __shared__ int lds[kBS / 64];
+  const int pre = block_sum(bsum, blockIdx.x, lds);
+  for (int q = 0; q < kScanPer; q++) {
+    const int i = blockIdx.x * kScanTile + q * kBS + threadIdx.x;
+    if (i < n) out[i] += pre;
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = pre + bsum[blockIdx.x];
 }
 
 // The offsets of the neighbour rows in one scan: each particle's own and
@@ -1482,38 +1485,34 @@ __global__ __launch_bounds__(kBS) void k_scan_rows_tiles(const int* own, const i
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(kBS) void k_scan_sums64(long long* bsum, int nb) {
-  __shared__ long long lds[kBS / 64 + 1];
-  const int per = (nb + kBS - 1) / kBS;
-  const int b0 = threadIdx.x * per;
-  long long s = 0;
-  for (int q = 0; q < per; q++)
-    if (b0 + q < nb) s += bsum[b0 + q];
-  long long tot;
-  long long pre = block_excl_scan(s, &tot, lds);
-  for (int q = 0; q < per; q++)
-    if (b0 + q < nb) {
-      const long long t = bsum[b0 + q];
-      bsum[b0 + q] = pre;
-      pre += t;
-    }
-  if (threadIdx.x == 0) bsum[nb] = tot;
-}
+// The flags as the host reads them: in pinned host memory, the sequence
+// number of the build written last, so that the host can go on while the
+// rest of the build runs.
+struct HostFlags {
+  int fl[kFlagCount];
+  int seq;
+};
 
 __global__ __launch_bounds__(kBS) void k_scan_rows_add(int* pair_base, int* row_start, int n,
-                                                       const long long* bsum, int nb,
-                                                       int* flags) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i < n) {
-    const long long o = bsum[i / kScanTile];
-    pair_base[i] += (int)(o >> 32);
-    row_start[i] += (int)(o >> 32) + (int)(o & 0xffffffffll);
+                                                       const long long* bsum, int* flags,
+                                                       HostFlags* host, int seq) {
+  __shared__ long long lds[kBS / 64];
+  const long long pre = block_sum(bsum, blockIdx.x, lds);
+  const int ph = (int)(pre >> 32), pl = (int)(pre & 0xffffffffll);
+  for (int q = 0; q < kScanPer; q++) {
+    const int i = blockIdx.x * kScanTile + q * kBS + threadIdx.x;
+    if (i < n) {
+      pair_base[i] += ph;
+      row_start[i] += ph + pl;
+    }
   }
-  if (i == 0) {
-    const long long t = bsum[nb];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    const long long t = pre + bsum[blockIdx.x];
     pair_base[n] = (int)(t >> 32);
     row_start[n] = (int)(t >> 32) + (int)(t & 0xffffffffll);
     flags[kFlagPairs] = (int)(t >> 32);  // read back with the other flags
+    for (int k = 0; k < kFlagCount; k++) host->fl[k] = flags[k];
+    __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -1869,7 +1868,7 @@ struct BuildPtrs {
 // as often as its busiest lane has hits rather than in almost every step
 // of the walk.
 constexpr int kHalfCells = 14;
-constexpr int kHitCap = 8;
+constexpr int kHits = 4;   // candidates that wait per lane
 
 // The owner and stencil checks of a pair within the cut-off (h, t) and the
 // append to the owner's row.  Only normal particles have rows; a row takes
@@ -1926,20 +1925,14 @@ __device__ __forceinline__ void own_row_exact(const GridDev& G, const BuildPtrs&
   own_row_hit<BATCH>(G, b, S, g_r, h, gh, b.idx ? b.idx[t] : t);
 }
 
-// kRowLanes lanes share one particle's half stencil (lane p takes the cells
-// p, p + kRowLanes, ...): shorter candidate walks per lane, and the range
-// table each lane keeps in LDS shrinks with them, so more wavefronts fit on a
-// CU to hide the walk's dependent loads.
-#ifndef MFIXDEM_ROW_LANES
-#define MFIXDEM_ROW_LANES 2
-#endif
-constexpr int kRowLanes = MFIXDEM_ROW_LANES;
-
-template <bool BATCH = false>
+// kRowLanes (2, 7 or 14) lanes share one particle's half stencil (lane p
+// takes the cells p, p + kRowLanes, ...): shorter candidate walks per lane,
+// and the range table each lane keeps in LDS shrinks with them, so more
+// wavefronts fit on a CU to hide the walk's dependent loads.
+template <bool BATCH, int kRowLanes>
 __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, BuildPtrs b,
                                                   BatchDev B) {
   constexpr int kCells = (kHalfCells + kRowLanes - 1) / kRowLanes;
-  constexpr int kHits = kRowLanes == 1 ? kHitCap : kHitCap / 2;
   __shared__ int s_lo[kCells][kBS], s_hi[kCells][kBS];
   __shared__ int s_hit[kHits][kBS];
   // XCD-aware order: the cells a row walks in the next planes of search
@@ -2091,52 +2084,6 @@ __global__ __launch_bounds__(kBS) void k_pack_xr(int n, int S, GridDev G, const 
   const int i = idx ? idx[k] : k;
   const double p[3] = {pos[i], pos[S + i], pos[2 * S + i]};
   pack_candidate(G, p, radius[i], state[i] != 0, xr, xf, k);
-}
-
-// A row of k_own_rows put in the reference's order (keys are distinct: the
-// partner id is part of the key), in place.  Rows are short: up to kRegRow
-// entries are sorted in registers, longer ones by insertion in place.
-constexpr int kRegRow = 8;
-__device__ __forceinline__ void sort_own_row(int* row, uint64_t* key, size_t ld, int cnt) {
-  if (cnt <= kRegRow) {
-    uint64_t k[kRegRow];
-    int v[kRegRow];
-#pragma unroll
-    for (int a = 0; a < kRegRow; a++)
-      if (a < cnt) {
-        k[a] = key[a * ld];
-        v[a] = row[a * ld];
-      }
-    // insertion sort, unrolled: entry a sinks past larger keys before it
-#pragma unroll
-    for (int a = 1; a < kRegRow; a++)
-#pragma unroll
-      for (int q = a; q > 0; q--)
-        if (a < cnt && k[q - 1] > k[q]) {
-          const uint64_t tk = k[q - 1];
-          k[q - 1] = k[q];
-          k[q] = tk;
-          const int tv = v[q - 1];
-          v[q - 1] = v[q];
-          v[q] = tv;
-        }
-#pragma unroll
-    for (int a = 0; a < kRegRow; a++)
-      if (a < cnt) row[a * ld] = v[a];
-    return;
-  }
-  for (int a = 1; a < cnt; a++) {
-    const uint64_t k = key[a * ld];
-    const int v = row[a * ld];
-    int q = a;
-    while (q > 0 && key[(q - 1) * ld] > k) {
-      key[q * ld] = key[(q - 1) * ld];
-      row[q * ld] = row[(q - 1) * ld];
-      q--;
-    }
-    key[q * ld] = k;
-    row[q * ld] = v;
-  }
 }
 
 // Own rows, one wavefront per search-grid cell.  The candidates of the 27
@@ -2428,154 +2375,113 @@ __device__ __forceinline__ bool place_ok(const PlaceGuard& g) {
          pairs <= g.cap_pairs;
 }
 
-// Places the own entries of each row (put in the reference's order first
-// when they were appended through atomic slots: own_key given) and
-// scatters the transposed (incoming) entries through atomic slots.  Every
-// new pair starts with no history; k_carry then brings over the histories
-// there are.
-__global__ __launch_bounds__(kBS) void k_place(int n, const int* own_cnt, int* own_tmp,
-                                               uint64_t* own_key, const int* pair_base,
-                                               const int* nbr_start, const int* in_cnt,
-                                               int* nbr_split, int* in_cur, int* nbr,
-                                               int* nbr_pid, uint8_t* nbr_row, uint8_t* pfl_new,
-                                               PlaceGuard pg) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n || !place_ok(pg)) return;
-  const int split = nbr_start[i] + in_cnt[i];
-  nbr_split[i] = split;
-  const int cnt = own_cnt[i];
-  for (int e = nbr_start[i]; e < split + cnt; e++)
-    nbr_row[e] = (uint8_t)((i & 63) | (e < split ? 0u : kRowOwn));
-  if (cnt == 0) return;
-  if (own_key && cnt > 1) sort_own_row(own_tmp + i, own_key + i, (size_t)n, cnt);
-  const int pb = pair_base[i];
-  if (cnt <= kRegRow) {
-    // a short row: every load, atomic and store of the row issued side by
-    // side rather than one entry after another
-    int jv[kRegRow], nj[kRegRow], sl[kRegRow];
-#pragma unroll
-    for (int k = 0; k < kRegRow; k++)
-      if (k < cnt) jv[k] = own_tmp[(size_t)k * n + i];
-#pragma unroll
-    for (int k = 0; k < kRegRow; k++)
-      if (k < cnt) {
-        nj[k] = nbr_start[jv[k]];
-        sl[k] = atomicAdd(&in_cur[jv[k]], 1);
-      }
-#pragma unroll
-    for (int k = 0; k < kRegRow; k++)
-      if (k < cnt) {
-        nbr[split + k] = jv[k];
-        nbr_pid[split + k] = pb + k;
-        nbr[nj[k] + sl[k]] = i;
-        nbr_pid[nj[k] + sl[k]] = pb + k;
-        pfl_new[pb + k] = 0;
-      }
-    return;
-  }
-  for (int k = 0; k < cnt; k++) {
-    const int j = own_tmp[(size_t)k * n + i];
-    nbr[split + k] = j;
-    nbr_pid[split + k] = pb + k;
-    const int slot = atomicAdd(&in_cur[j], 1);
-    nbr[nbr_start[j] + slot] = i;
-    nbr_pid[nbr_start[j] + slot] = pb + k;
-    pfl_new[pb + k] = 0;
-  }
-}
+// An incoming entry between k_place and k_sort_in: its owner's global id
+// (the sort key) and slot, and the pair id.
+struct InEntry {
+  int gid, slot, pid, pad;
+};
 
-// NEIGHBOUR's history carry-over (neighbour.f:67-126): a new pair takes the
-// history of the same pair (same owner, same partner) in the owner's old
-// row, or starts at zero.  Only old pairs that hold a history (flag set:
-// the pairs in contact, a small share of the list) have anything to give,
-// so the carry starts from them: the thread of each old row finds each of
-// its flagged pairs in the owner's new row and copies the history there.
-// Slots map through inv (old slot -> new slot; null: the slots stayed).
+// Places the own entries of each row, kG lanes to a row and one entry to a
+// lane, in the reference's order: an entry's place is the number of smaller
+// keys in its row (keys are distinct: the partner id is part of the key;
+// own_key null: the rows are built in order).  Each entry goes to its
+// partner's incoming entries as well, through an atomic slot.
+// NEIGHBOUR's history carry-over (neighbour.f:67-126) is part of it: a new
+// pair takes the history of the same pair (same owner, same partner) in the
+// owner's old row, or starts at zero.  Only old pairs that hold a history
+// (flag set) have anything to give, so the lanes look for those of the old
+// row and compare each with the row's new partners.  perm (new slot -> old
+// slot) and inv (old slot -> new slot) map the slots, null where they stayed.
 // A pair whose owner changed is not in the owner's new row and, as in the
 // reference, starts at zero.
-__global__ __launch_bounds__(kBS) void k_carry(int n, const int* inv, CarryPtrs c,
-                                               const int* pair_base, const int* nbr_split,
-                                               const int* nbr_start, const int* nbr,
-                                               PlaceGuard pg) {
-  const int o = blockIdx.x * kBS + threadIdx.x;  // the owner's old slot
+// One lane per row ran 8 entries side by side and longer rows one after the
+// other in global memory (52 us of latency at 20,000 settled spheres, with
+// 31 us for the carry in a kernel of its own).
+template <int kG>
+__global__ __launch_bounds__(kBS) void k_place(int n, const int* own_cnt, const int* own_tmp,
+                                               const uint64_t* own_key, const int* pair_base,
+                                               const int* nbr_start, const int* in_cnt,
+                                               const int* gid, int* nbr_split, int* in_cur,
+                                               int* nbr, int* nbr_pid, uint8_t* nbr_row,
+                                               InEntry* in_tmp, const int* perm, const int* inv,
+                                               CarryPtrs c, PlaceGuard pg) {
+  const int id = blockIdx.x * kBS + threadIdx.x, i = id / kG, q = id % kG;
   if (!place_ok(pg)) return;
-  if (o == 0) {  // the host has read this build's flags: the next build's start values
+  if (id == 0) {  // the host has this build's flags: the next build's start values
     c.flags[kFlagRogueGid] = INT_MAX;
     c.flags[kFlagRogueCount] = 0;
     c.flags[kFlagOwnOverflow] = 0;
   }
-  if (o >= n) return;
-  const int os = c.old_split[o], oe = c.old_start[o + 1];
-  if (os == oe) return;
-  const int opb = c.old_pair_base[o];
-  int i = -1, s0 = 0, s1 = 0, pb = 0;
-  for (int r = os; r < oe; r++) {
-    const int op = opb + (r - os);
-    if (!c.pfl_old[op]) continue;
-    if (i < 0) {
-      i = inv ? inv[o] : o;
-      s0 = nbr_split[i];
-      s1 = nbr_start[i + 1];
-      pb = pair_base[i];
+  if (i >= n) return;
+  const int split = nbr_start[i] + in_cnt[i];
+  if (q == 0) nbr_split[i] = split;
+  const int cnt = own_cnt[i];
+  if (cnt == 0) return;
+  const int o = perm ? perm[i] : i;
+  const int pb = pair_base[i], gi = gid[i];
+  const int os = c.old_split[o], oe = c.old_start[o + 1], opb = c.old_pair_base[o];
+  const unsigned g0 = __lane_id() & ~(unsigned)(kG - 1);  // the group's first lane
+  for (int kb = 0; kb < cnt; kb += kG) {
+    const int k = kb + q;
+    const bool has = k < cnt;
+    int j = -1, r = k;
+    if (has) j = own_tmp[(size_t)k * n + i];
+    if (has && own_key) {
+      const uint64_t key = own_key[(size_t)k * n + i];
+      r = 0;
+#pragma unroll 4
+      for (int m = 0; m < cnt; m++) r += own_key[(size_t)m * n + i] < key ? 1 : 0;
     }
-    const int jo = c.old_nbr[r];
-    const int j = inv ? inv[jo] : jo;
-    for (int q = s0; q < s1; q++)
-      if (nbr[q] == j) {
-        const int p = pb + (q - s0);
-        c.pfl_new[p] = 1;
-        for (int d = 0; d < 3; d++) c.pft_new[3 * p + d] = c.pft_old[3 * op + d];
-        break;
+    int from = -1;  // the old pair whose history this pair takes
+    for (int ob = os; ob < oe; ob += kG) {
+      const int e = ob + q;
+      const bool held = e < oe && c.pfl_old[opb + (e - os)];
+      int jn = -1;
+      if (held) {
+        const int jo = c.old_nbr[e];
+        jn = inv ? inv[jo] : jo;
       }
+      unsigned long long m = (__ballot(held) >> g0) & ((1ull << kG) - 1ull);
+      while (m) {
+        const int t = __builtin_ctzll(m);
+        m &= m - 1ull;
+        if (__shfl(jn, (int)g0 + t, 64) == j && has) from = opb + (ob + t - os);
+      }
+    }
+    if (!has) continue;
+    const int p = pb + r, dst = split + r;
+    const int slot = atomicAdd(&in_cur[j], 1);
+    nbr[dst] = j;
+    nbr_pid[dst] = p;
+    nbr_row[dst] = (uint8_t)((i & 63) | kRowOwn);
+    in_tmp[nbr_start[j] - pair_base[j] + slot] = InEntry{gi, i, p, 0};
+    c.pfl_new[p] = from >= 0 ? 1 : 0;
+    if (from >= 0)
+      for (int d = 0; d < 3; d++) c.pft_new[3 * (size_t)p + d] = c.pft_old[3 * (size_t)from + d];
   }
 }
 
-// incoming entries in ascending owner id (short rows in registers)
-__global__ __launch_bounds__(kBS) void k_sort_in(int n, const int* gid, const int* nbr_start,
-                                                 const int* nbr_split, int* nbr, int* nbr_pid,
-                                                 PlaceGuard pg) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
+// The incoming entries of each row in ascending owner id, kG lanes to a row:
+// an entry's place is the number of smaller ids in its row.
+template <int kG>
+__global__ __launch_bounds__(kBS) void k_sort_in(int n, const int* pair_base,
+                                                 const int* nbr_start, const int* in_cnt,
+                                                 const InEntry* in_tmp, int* nbr, int* nbr_pid,
+                                                 uint8_t* nbr_row, PlaceGuard pg) {
+  const int id = blockIdx.x * kBS + threadIdx.x, i = id / kG, q = id % kG;
   if (i >= n || !place_ok(pg)) return;
-  const int s = nbr_start[i], e = nbr_split[i], cnt = e - s;
-  if (cnt < 2) return;
-  if (cnt <= kRegRow) {
-    int g[kRegRow], v[kRegRow], pv[kRegRow];
-#pragma unroll
-    for (int a = 0; a < kRegRow; a++)
-      if (a < cnt) {
-        v[a] = nbr[s + a];
-        pv[a] = nbr_pid[s + a];
-      }
-#pragma unroll
-    for (int a = 0; a < kRegRow; a++)
-      if (a < cnt) g[a] = gid[v[a]];
-#pragma unroll
-    for (int a = 1; a < kRegRow; a++)
-#pragma unroll
-      for (int q = a; q > 0; q--)
-        if (a < cnt && g[q - 1] > g[q]) {
-          int t = g[q - 1]; g[q - 1] = g[q]; g[q] = t;
-          t = v[q - 1]; v[q - 1] = v[q]; v[q] = t;
-          t = pv[q - 1]; pv[q - 1] = pv[q]; pv[q] = t;
-        }
-#pragma unroll
-    for (int a = 0; a < kRegRow; a++)
-      if (a < cnt) {
-        nbr[s + a] = v[a];
-        nbr_pid[s + a] = pv[a];
-      }
-    return;
-  }
-  for (int a = s + 1; a < e; a++) {
-    const int j = nbr[a], pj = nbr_pid[a], gj = gid[j];
-    int q = a;
-    while (q > s && gid[nbr[q - 1]] > gj) {
-      nbr[q] = nbr[q - 1];
-      nbr_pid[q] = nbr_pid[q - 1];
-      q--;
-    }
-    nbr[q] = j;
-    nbr_pid[q] = pj;
+  const int cnt = in_cnt[i];
+  if (q >= cnt) return;
+  const int s = nbr_start[i];
+  const InEntry* row = in_tmp + (s - pair_base[i]);
+  for (int k = q; k < cnt; k += kG) {
+    const InEntry t = row[k];
+    int r = 0;
+#pragma unroll 4
+    for (int m = 0; m < cnt; m++) r += row[m].gid < t.gid ? 1 : 0;
+    nbr[s + r] = t.slot;
+    nbr_pid[s + r] = t.pid;
+    nbr_row[s + r] = (uint8_t)(i & 63);
   }
 }
 

@@ -19,6 +19,7 @@
 #include <cstring>
 #include <array>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/mfixdem.h"
@@ -108,12 +109,14 @@ struct mfixdem_handle {
   double* pft[2]{};
   uint8_t* pfl[2]{};            // per pair: 1 when pft holds the history, 0 when it is zero
   int64_t pft_cap[2]{0, 0};
+  InEntry* in_tmp = nullptr;    // incoming entries while a list is built
+  int64_t in_cap = 0;
   int64_t n_pairs = 0;
   int* scan_bsum = nullptr;
   long long* scan_bsum64 = nullptr;
   bool counts_zeroed = false;  // own_cnt, in_cnt, in_cur cleared by the last binning
   bool xr_packed = false;      // the row walk's candidate data written by the last binning
-  bool flags_set = false;      // the rebuild flags hold their start values (k_carry sets them)
+  bool flags_set = false;      // the rebuild flags hold their start values (k_place sets them)
   // A binning of one system with the thread-row search moves the particle
   // data into the search-cell order only every kPermuteEvery-th time (and
   // the first time); otherwise the slots stay and bin_idx lists them in that
@@ -124,6 +127,8 @@ struct mfixdem_handle {
   int bins_since_permute = 0;
   bool order_set = false;
   int* flags = nullptr;
+  HostFlags* host_flags = nullptr;  // pinned host memory (wait_flags)
+  int flags_seq = 0;
   // gas
   double* ugc = nullptr;  // cell-centre gas velocity (filter schemes)
   double* gas_stage = nullptr;  // 3*ncell: staged U_G/V_G/W_G, P_G or P_FORCE uploads
@@ -222,28 +227,46 @@ int32_t fill_i32(hipStream_t s, int* a, int64_t n, int v) {
 
 // exclusive scan of in[0..n) -> out[0..n]; out[n] = total
 int32_t scan_i32(mfixdem_handle* h, const int* in, int* out, int64_t n) {
-  const int nb = (int)((n + kScanTile - 1) / kScanTile);
-  hipLaunchKernelGGL(k_scan_tiles, dim3(std::max(nb, 1)), dim3(kBS), 0, h->stream, in, out,
-                     (int)n, h->scan_bsum);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kBS), 0, h->stream, h->scan_bsum, std::max(nb, 1));
-  hipLaunchKernelGGL(k_scan_add, dim3(nblk(n + 1)), dim3(kBS), 0, h->stream, out, (int)n,
-                     h->scan_bsum, std::max(nb, 1));
+  const int nb = std::max((int)((n + kScanTile - 1) / kScanTile), 1);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(nb), dim3(kBS), 0, h->stream, in, out, (int)n,
+                     h->scan_bsum);
+  hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kBS), 0, h->stream, out, (int)n, h->scan_bsum);
   HIPOK(hipGetLastError());
   return MFIXDEM_OK;
 }
 
 // Pair ids and row starts of the neighbour lists in one scan of the own and
-// incoming counts (k_scan_rows_tiles).
+// incoming counts (k_scan_rows_tiles); the flags go to the host with it.
 int32_t scan_rows(mfixdem_handle* h, const int* own, const int* in, int* pair_base,
                   int* row_start, int64_t n) {
-  const int nb = (int)((n + kScanTile - 1) / kScanTile);
-  hipLaunchKernelGGL(k_scan_rows_tiles, dim3(std::max(nb, 1)), dim3(kBS), 0, h->stream, own, in,
-                     pair_base, row_start, (int)n, h->scan_bsum64);
-  hipLaunchKernelGGL(k_scan_sums64, dim3(1), dim3(kBS), 0, h->stream, h->scan_bsum64,
-                     std::max(nb, 1));
-  hipLaunchKernelGGL(k_scan_rows_add, dim3(nblk(n + 1)), dim3(kBS), 0, h->stream, pair_base,
-                     row_start, (int)n, h->scan_bsum64, std::max(nb, 1), h->flags);
+  const int nb = std::max((int)((n + kScanTile - 1) / kScanTile), 1);
+  hipLaunchKernelGGL(k_scan_rows_tiles, dim3(nb), dim3(kBS), 0, h->stream, own, in, pair_base,
+                     row_start, (int)n, h->scan_bsum64);
+  hipLaunchKernelGGL(k_scan_rows_add, dim3(nb), dim3(kBS), 0, h->stream, pair_base, row_start,
+                     (int)n, h->scan_bsum64, h->flags, h->host_flags, ++h->flags_seq);
   HIPOK(hipGetLastError());
+  return MFIXDEM_OK;
+}
+
+// Waits until the last scan_rows has written its flags to the host, without
+// waiting for what is queued behind it (a copy and a wait for the stream cost
+// 23 us and left the stream empty).  Ends with an error if the stream ends
+// first, which a failed launch or a device error makes it do.
+int32_t wait_flags(mfixdem_handle* h, int fl[kFlagCount]) {
+  auto seen = [&] {
+    return __atomic_load_n(&h->host_flags->seq, __ATOMIC_ACQUIRE) == h->flags_seq;
+  };
+  for (int spin = 0; !seen(); spin++) {
+    if ((spin & 1023) != 1023) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    const hipError_t e = hipStreamQuery(h->stream);
+    if (e == hipErrorNotReady) continue;
+    HIPOK(e);
+    if (!seen()) return MFIXDEM_ERR_HIP;
+  }
+  std::memcpy(fl, h->host_flags->fl, sizeof(int) * kFlagCount);
   return MFIXDEM_OK;
 }
 
@@ -427,6 +450,15 @@ int32_t ensure_pft_capacity(mfixdem_handle* h, int b, int64_t pairs) {
   return MFIXDEM_OK;
 }
 
+int32_t ensure_in_capacity(mfixdem_handle* h, int64_t pairs) {
+  if (h->in_cap >= pairs && h->in_tmp) return MFIXDEM_OK;
+  const int64_t cap = std::max<int64_t>(pairs + pairs / 4, 1024);
+  dfree(h->in_tmp);
+  CHECKRC(dalloc(&h->in_tmp, cap));
+  h->in_cap = cap;
+  return MFIXDEM_OK;
+}
+
 // The particle data moves into the search-cell order every kPermuteEvery-th
 // binning: particles move little between binnings (at most a fraction of a
 // search cell in NEIGHBOR_SEARCH_N steps), so the slots stay close to that
@@ -603,14 +635,25 @@ int32_t do_neighbour(mfixdem_handle* h) {
     cp.pft_new = h->pft[1 - h->pcur];
     cp.pfl_old = h->pfl[h->pcur];
     cp.pfl_new = h->pfl[1 - h->pcur];
-    hipLaunchKernelGGL(k_place, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->own_cnt,
-                       h->own_tmp, nsq || wave_rows ? nullptr : h->own_key, h->pair_base[nl],
-                       h->nbr_start[nl], h->in_cnt, h->nbr_split[nl], h->in_cur, h->nbr[nl],
-                       h->nbr_pid[nl], h->nbr_row[nl], cp.pfl_new, pg);
-    hipLaunchKernelGGL(k_carry, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->bin_inv, cp,
-                       h->pair_base[nl], h->nbr_split[nl], h->nbr_start[nl], h->nbr[nl], pg);
-    hipLaunchKernelGGL(k_sort_in, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->gid[t],
-                       h->nbr_start[nl], h->nbr_split[nl], h->nbr[nl], h->nbr_pid[nl], pg);
+    const uint64_t* key = nsq || wave_rows ? nullptr : h->own_key;
+    const int* perm = h->bin_inv ? h->vals[1] : nullptr;
+    auto go = [&](auto lanes) {
+      constexpr int kG = decltype(lanes)::value;
+      const dim3 grid(nblk((int64_t)n * kG)), blk(kBS);
+      hipLaunchKernelGGL(k_place<kG>, grid, blk, 0, h->stream, n, h->own_cnt, h->own_tmp, key,
+                         h->pair_base[nl], h->nbr_start[nl], h->in_cnt, h->gid[t],
+                         h->nbr_split[nl], h->in_cur, h->nbr[nl], h->nbr_pid[nl], h->nbr_row[nl],
+                         h->in_tmp, perm, h->bin_inv, cp, pg);
+      hipLaunchKernelGGL(k_sort_in<kG>, grid, blk, 0, h->stream, n, h->pair_base[nl],
+                         h->nbr_start[nl], h->in_cnt, h->in_tmp, h->nbr[nl], h->nbr_pid[nl],
+                         h->nbr_row[nl], pg);
+    };
+    // 8 lanes to a row where rows are long or the chip has room, else 4.
+    // Measured (k_place + k_sort_in, 8 / 4 / 2 lanes): 2,003 settled spheres,
+    // 5.7 pairs each, 15 / 25 / 46 us; 301,057, 6.5 pairs, 149 / 181 / 268;
+    // 120,000, 4 pairs, 20 / 20 / 27; 1M, 1.6 pairs, 119 / 89 / 90.
+    if (h->n_pairs >= 4 * (int64_t)n || n <= 32768) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 4>{});
     HIPOK(hipGetLastError());
     return MFIXDEM_OK;
   };
@@ -642,11 +685,23 @@ int32_t do_neighbour(mfixdem_handle* h) {
         hipLaunchKernelGGL(k_pack_xr, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
                            b.idx, b.pos, b.radius, b.state, h->xr_pack,
                            reinterpret_cast<float4*>(h->stage));
-      const dim3 rg(nblk((int64_t)n * kRowLanes));  // kRowLanes threads per particle
-      if (h->nsys > 1)
-        hipLaunchKernelGGL((k_own_rows<true>), rg, dim3(kBS), 0, h->stream, n, S, h->G, b, h->B);
-      else
-        hipLaunchKernelGGL((k_own_rows<false>), rg, dim3(kBS), 0, h->stream, n, S, h->G, b, h->B);
+      auto rows = [&](auto lanes) {
+        constexpr int kL = decltype(lanes)::value;
+        const dim3 rg(nblk((int64_t)n * kL)), blk(kBS);
+        if (h->nsys > 1)
+          hipLaunchKernelGGL((k_own_rows<true, kL>), rg, blk, 0, h->stream, n, S, h->G, b, h->B);
+        else
+          hipLaunchKernelGGL((k_own_rows<false, kL>), rg, blk, 0, h->stream, n, S, h->G, b, h->B);
+      };
+      // Lanes per particle: all 14 cells of the half stencil side by side
+      // while that leaves the chip room, 7 where rows are long (2 lanes then
+      // have more hits than their LDS lists hold), else 2.  Measured (2 / 7 /
+      // 14 lanes): 2,003 settled spheres 39 / 14 / 11 us; 301,057 211 / 170 /
+      // 192; 120,000 at 4 pairs each 30 / 31 / 40; 1M at 1.6, 126 / 181 / 262.
+      if (n <= 20480) rows(std::integral_constant<int, 14>{});
+      else if (n <= 65536 || (h->n_pairs >= 5 * (int64_t)n && n < (1 << 24)))
+        rows(std::integral_constant<int, 7>{});
+      else rows(std::integral_constant<int, 2>{});
     }
     HIPOK(hipGetLastError());
     zeroed = false;
@@ -657,19 +712,21 @@ int32_t do_neighbour(mfixdem_handle* h) {
       CHECKRC(scan_i32(h, h->own_cnt, h->pair_base[nl], n));
       HIPOK(hipMemcpyAsync(h->flags + kFlagPairs, h->pair_base[nl] + n, sizeof(int),
                            hipMemcpyDeviceToDevice, h->stream));
+      HIPOK(hipMemcpyAsync(fl, h->flags, sizeof(fl), hipMemcpyDeviceToHost, h->stream));
     } else {
       CHECKRC(scan_rows(h, h->own_cnt, h->in_cnt, h->pair_base[nl], h->nbr_start[nl], n));
     }
-    HIPOK(hipMemcpyAsync(fl, h->flags, sizeof(fl), hipMemcpyDeviceToHost, h->stream));
     // thread rows have their row starts already: place them ahead of the
     // wait, guarded, while the host waits for the flags
     placed = false;
-    if (!nsq && !wave_rows && cur_zeroed && h->nbr[nl] && h->pft[1 - h->pcur]) {
-      spec = PlaceGuard{h->flags, h->maxrow, h->nbr_cap[nl], h->pft_cap[1 - h->pcur]};
+    if (!nsq && !wave_rows && cur_zeroed && h->nbr[nl] && h->pft[1 - h->pcur] && h->in_tmp) {
+      spec = PlaceGuard{h->flags, h->maxrow, h->nbr_cap[nl],
+                        std::min(h->pft_cap[1 - h->pcur], h->in_cap)};
       CHECKRC(place(spec));
       placed = true;
     }
-    HIPOK(sync_stream(h));
+    if (nsq || wave_rows) HIPOK(sync_stream(h));
+    else CHECKRC(wait_flags(h, fl));
     npairs = fl[kFlagPairs];
     if (fl[kFlagOwnOverflow] <= h->maxrow) break;
     int z = 0;
@@ -694,6 +751,7 @@ int32_t do_neighbour(mfixdem_handle* h) {
   if (!fits) {
     CHECKRC(ensure_list_capacity(h, nl, 2 * (int64_t)npairs));
     CHECKRC(ensure_pft_capacity(h, 1 - h->pcur, npairs));
+    CHECKRC(ensure_in_capacity(h, npairs));
     if (nsq || wave_rows) {  // rows built sorted: count the incoming entries here
       CHECKRC(fill_i32(h->stream, h->in_cnt, n, 0));
       hipLaunchKernelGGL(k_count_in, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->own_cnt,
@@ -1122,7 +1180,7 @@ void for_each_buffer(mfixdem_handle* h, F f) {
     f(h->rops_fix[b]);
   }
   f(h->fc); f(h->tow); f(h->fc_id); f(h->tow_id); f(h->sort_tmp); f(h->rm_cnt); f(h->rm_list); f(h->f_gp); f(h->drag_fc);
-  f(h->xr_pack);
+  f(h->xr_pack); f(h->in_tmp);
   f(h->fstart); f(h->fend); f(h->fine_rank); f(h->fine_cnt); f(h->fine_off);
   f(h->own_cnt); f(h->own_tmp); f(h->own_key); f(h->in_cnt); f(h->in_cur);
   f(h->tot_cnt); f(h->scan_bsum); f(h->scan_bsum64); f(h->flags); f(h->csz); f(h->xe); f(h->yn);
@@ -1240,6 +1298,9 @@ int32_t alloc_buffers(mfixdem_handle* h) {
     return fail(MFIXDEM_ERR_OOM);
   if ((rc = upload_setup(h)) || (rc = setup_fine_cells(h))) return fail(rc);
   if (hipMemset(h->flags, 0, sizeof(int) * kFlagCount) != hipSuccess) return fail(MFIXDEM_ERR_HIP);
+  if (hipHostMalloc((void**)&h->host_flags, sizeof(HostFlags), hipHostMallocDefault) != hipSuccess)
+    return fail(MFIXDEM_ERR_OOM);
+  *h->host_flags = HostFlags{};
   return MFIXDEM_OK;
 }
 
@@ -1354,6 +1415,7 @@ int32_t mfixdem_destroy(mfixdem_handle* h) {
   if (!h) return MFIXDEM_ERR_ARG;
   if (h->stream) (void)sync_stream(h);
   for_each_buffer(h, [](auto*& p) { dfree(p); });
+  if (h->host_flags) (void)hipHostFree(h->host_flags);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
   if (h->stream) (void)hipStreamDestroy(h->stream);
