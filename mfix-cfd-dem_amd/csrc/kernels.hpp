@@ -3302,17 +3302,31 @@ __global__ __launch_bounds__(kBS) void k_delete_outside(int n, int S, const int*
 }
 
 // ------------------------------------------------------------- exports
-__global__ void k_scatter_gid_d3(int n, int S, int ld, const int* gid, const uint8_t* state,
-                                 const double* src, double* dst) {
+// The particles of n slots in global-id order for the host, one launch for
+// all of them: the given arrays' component planes (null: not wanted) and
+// PARTICLE_STATE, packed one after another into out, so that one stream of
+// copies takes them to the host.  A thread reads its slot coalesced and
+// writes 8 bytes to each plane at its id.
+__global__ __launch_bounds__(kBS) void k_export(int n, int S, const int* gid,
+                                                const uint8_t* state, const double* pos,
+                                                const double* vel, const double* omega,
+                                                bool want_state, double* out) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
   const int g = gid[i];
-  for (int c = 0; c < 3; c++) dst[(size_t)c * ld + g] = src[c * S + i];
-}
-__global__ void k_scatter_gid_i(int n, const int* gid, const int* src, int add, int* dst) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n) return;
-  dst[gid[i]] = src[i] + add;
+  const double* src[3] = {pos, vel, omega};
+  double* o = out + g;
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+    if (src[a])
+      for (int c = 0; c < 3; c++) {
+        *o = src[a][(size_t)c * S + i];
+        o += n;
+      }
+  if (want_state) {
+    const uint8_t v = state[i];  // a seeded particle is ENTERING
+    reinterpret_cast<uint8_t*>(o - g)[g] = v == kSeeded ? kEntering : v;
+  }
 }
 // Holes at set-up: slots q < n whose PARTICLE_STATE st[q] is 0 become
 // nonexistent with zero radius and state (slot order = global-id order

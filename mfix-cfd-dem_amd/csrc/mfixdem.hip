@@ -128,6 +128,8 @@ struct mfixdem_handle {
   bool order_set = false;
   int* flags = nullptr;
   HostFlags* host_flags = nullptr;  // pinned host memory (wait_flags)
+  char* ring = nullptr;             // pinned chunks of read_back, on first use
+  hipEvent_t ring_ev[4]{};
   int flags_seq = 0;
   // gas
   double* ugc = nullptr;  // cell-centre gas velocity (filter schemes)
@@ -156,7 +158,9 @@ struct mfixdem_handle {
   FacetDev* fac = nullptr;
   int *dg_foff = nullptr, *dg_fids = nullptr;
   uint8_t* cell_fmask = nullptr;
-  double* stage = nullptr;  // export staging, 3*n doubles
+  // export staging (73 bytes a particle of the largest system); the row
+  // walk's candidates during a rebuild
+  double* stage = nullptr;
   // DEM mass inlets / outlets (mfixdem_set_dem_bcs): host schedule and
   // layout, the device table, this step's seeds, the slot of each global id
   // (rewritten at every binning) and the particles deleted in a step
@@ -610,7 +614,7 @@ int32_t do_neighbour(mfixdem_handle* h) {
   b.pos = h->pos[c]; b.radius = h->radius[t]; b.gid = h->gid[t]; b.dgc = h->dgc[t];
   b.xr = h->xr_pack;
   // the single-precision copy for the walk's prefilter lives in the export
-  // stage (3 doubles per slot), which no call uses during a rebuild
+  // stage (at least 3 doubles per slot), which no call uses during a rebuild
   b.xf = reinterpret_cast<float4*>(h->stage);
   b.state = h->state[t]; b.fstart = h->fstart; b.fend = h->fend;
   b.idx = h->bin_idx;
@@ -917,14 +921,12 @@ bool rebin_each_step(const mfixdem_handle* h) {
 
 // The free global ids, from the particle states (at init, and after rogue
 // particles have been removed).
+int32_t export_particles(mfixdem_handle* h, int first, int n, double* pos, double* vel,
+                         double* omega, int8_t* state, int64_t ld);
 int32_t refresh_free_gids(mfixdem_handle* h) {
   const int n = h->n;
-  hipLaunchKernelGGL(k_scatter_gid_u8, dim3(nblk(n)), dim3(kBS), 0, h->stream, n,
-                     h->gid[h->tw], h->state[h->tw], (int8_t*)h->stage);
-  HIPOK(hipGetLastError());
   std::vector<int8_t> st(n);
-  HIPOK(hipMemcpyAsync(st.data(), h->stage, n, hipMemcpyDeviceToHost, h->stream));
-  HIPOK(sync_stream(h));
+  CHECKRC(export_particles(h, 0, n, nullptr, nullptr, nullptr, st.data(), n));
   h->dbc.free_gids.clear();
   for (int g = 0; g < n; g++)
     if (st[g] == kNonexistent) h->dbc.free_gids.insert(g);
@@ -1024,17 +1026,102 @@ int32_t one_step(mfixdem_handle* h, int32_t nn) {
   return MFIXDEM_OK;
 }
 
-int32_t scatter_d3(mfixdem_handle* h, const double* src, double* host, int64_t ld) {
-  const int n = h->n;
-  hipLaunchKernelGGL(k_scatter_gid_d3, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->stride, n,
-                     h->gid[h->tw], h->state[h->tw], src, h->stage);
+// A piece of a result: device memory to the caller's host memory.
+struct OutPiece {
+  const void* dev;
+  void* host;
+  size_t bytes;
+};
+constexpr size_t kRingChunk = 512 << 10;
+constexpr int kRingChunks = 4;
+
+// Brings the pieces to the host in their order, through a ring of pinned
+// chunks: the copy engine fills one while the host empties another, and
+// pieces that follow each other in device memory share a copy.  Copies into
+// the caller's pageable memory were taken through the runtime's own staging
+// at 17 GB/s with 15-20 us for each of them (10 for the particles); the ring
+// moves 28 GB/s, and a small result takes one copy and 15 us.
+int32_t read_back(mfixdem_handle* h, const std::vector<OutPiece>& pieces) {
+  if (!h->ring) {
+    if (hipHostMalloc((void**)&h->ring, kRingChunk * kRingChunks, hipHostMallocDefault) !=
+        hipSuccess)
+      return MFIXDEM_ERR_OOM;
+    for (auto& e : h->ring_ev) HIPOK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  struct Part {
+    void* host;
+    size_t at, bytes;
+  };
+  std::vector<Part> parts[kRingChunks];
+  int head = 0, tail = 0;  // chunks [tail, head) are on their way
+  auto empty = [&]() -> int32_t {
+    const int c = tail++ % kRingChunks;
+    HIPOK(hipEventSynchronize(h->ring_ev[c]));
+    for (const Part& p : parts[c])
+      std::memcpy(p.host, h->ring + c * kRingChunk + p.at, p.bytes);
+    parts[c].clear();
+    return MFIXDEM_OK;
+  };
+  // queued copies must not outlive the call: the ring is the next call's
+  auto fill = [&]() -> int32_t {
+    size_t at = 0, from = 0;         // of the open chunk: filled, start of the open copy
+    const char* src = nullptr;       // device address of the open copy
+    auto flush = [&]() -> int32_t {
+      if (at > from)
+        HIPOK(hipMemcpyAsync(h->ring + (head % kRingChunks) * kRingChunk + from, src, at - from,
+                             hipMemcpyDeviceToHost, h->stream));
+      from = at;
+      return MFIXDEM_OK;
+    };
+    auto close = [&]() -> int32_t {
+      CHECKRC(flush());
+      HIPOK(hipEventRecord(h->ring_ev[head % kRingChunks], h->stream));
+      head++;
+      at = from = 0;
+      if (head - tail == kRingChunks) CHECKRC(empty());
+      return MFIXDEM_OK;
+    };
+    for (const OutPiece& p : pieces)
+      for (size_t done = 0; done < p.bytes;) {
+        const char* d = (const char*)p.dev + done;
+        if (at == from || d != src + (at - from)) {
+          CHECKRC(flush());
+          src = d;
+        }
+        const size_t m = std::min(p.bytes - done, kRingChunk - at);
+        parts[head % kRingChunks].push_back({(char*)p.host + done, at, m});
+        at += m;
+        done += m;
+        if (at == kRingChunk) CHECKRC(close());
+      }
+    if (at > 0) CHECKRC(close());
+    while (tail < head) CHECKRC(empty());
+    return MFIXDEM_OK;
+  };
+  const int32_t rc = fill();
+  if (rc != MFIXDEM_OK) (void)sync_stream(h);
+  return rc;
+}
+
+// The particles of n slots from slot first on (one system, or a member of an
+// ensemble), in global-id order with leading dimension ld.
+int32_t export_particles(mfixdem_handle* h, int first, int n, double* pos, double* vel,
+                         double* omega, int8_t* state, int64_t ld) {
+  const int c = h->cur, t = h->tw;
+  if (n <= 0 || !(pos || vel || omega || state)) return MFIXDEM_OK;
+  h->xr_packed = false;  // the stage held them
+  hipLaunchKernelGGL(k_export, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->stride,
+                     h->gid[t] + first, h->state[t] + first, pos ? h->pos[c] + first : nullptr,
+                     vel ? h->vel[c] + first : nullptr, omega ? h->omega[c] + first : nullptr,
+                     state != nullptr, h->stage);
   HIPOK(hipGetLastError());
-  std::vector<double> tmp((size_t)3 * n);
-  HIPOK(hipMemcpyAsync(tmp.data(), h->stage, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
-                       h->stream));
-  HIPOK(sync_stream(h));
-  for (int c = 0; c < 3; c++) std::memcpy(host + c * ld, tmp.data() + (size_t)c * n, sizeof(double) * n);
-  return MFIXDEM_OK;
+  std::vector<OutPiece> out;
+  const double* d = h->stage;
+  for (double* a : {pos, vel, omega})
+    if (a)
+      for (int k = 0; k < 3; k++, d += n) out.push_back({d, a + k * ld, sizeof(double) * n});
+  if (state) out.push_back({d, state, (size_t)n});
+  return read_back(h, out);
 }
 
 template <typename T>
@@ -1235,6 +1322,9 @@ int32_t setup_fine_cells(mfixdem_handle* h) {
 // destroys the handle.
 int32_t alloc_buffers(mfixdem_handle* h) {
   const int64_t n = h->n, S = h->stride, nc = h->S.ncell;
+  int64_t max_cap = h->nsys > 1 ? 0 : n;  // the most particles of one system
+  for (int s = 0; s < h->nsys && h->nsys > 1; s++)
+    max_cap = std::max<int64_t>(max_cap, h->sys_off[s + 1] - h->sys_off[s]);
   int32_t rc = MFIXDEM_OK;
   auto fail = [&](int32_t r) { return r; };
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
@@ -1276,7 +1366,7 @@ int32_t alloc_buffers(mfixdem_handle* h) {
       (rc = dalloc(&h->fluid, nc)) || (rc = dalloc(&h->pic_cnt, nc)) ||
       (rc = dalloc(&h->pic_off, nc + 1)) || (rc = dalloc(&h->pic_cur, nc)) ||
       (rc = dalloc(&h->pic, n)) ||
-      (rc = dalloc(&h->stage, 3 * n)) ||
+      (rc = dalloc(&h->stage, std::max<int64_t>(3 * n, (73 * max_cap + 7) / 8))) ||
       (rc = dalloc(&h->rops_fix[0], nc * h->S.p.nphases)) ||
       (rc = dalloc(&h->rops_fix[1], nc * h->S.p.nphases)) || (rc = dalloc(&h->rm_cnt, 2)) ||
       (rc = dalloc(&h->rm_list, n)))
@@ -1416,6 +1506,9 @@ int32_t mfixdem_destroy(mfixdem_handle* h) {
   if (h->stream) (void)sync_stream(h);
   for_each_buffer(h, [](auto*& p) { dfree(p); });
   if (h->host_flags) (void)hipHostFree(h->host_flags);
+  if (h->ring) (void)hipHostFree(h->ring);
+  for (auto& e : h->ring_ev)
+    if (e) (void)hipEventDestroy(e);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1607,17 +1700,7 @@ int32_t mfixdem_get_particles(mfixdem_handle* h, double* pos, double* vel, doubl
                               int8_t* state, int64_t ld) {
   if (h && h->nsys > 1) return MFIXDEM_ERR_ARG;  // single-system call
   if (!h || ld < h->n) return MFIXDEM_ERR_ARG;
-  if (pos) CHECKRC(scatter_d3(h, h->pos[h->cur], pos, ld));
-  if (vel) CHECKRC(scatter_d3(h, h->vel[h->cur], vel, ld));
-  if (omega) CHECKRC(scatter_d3(h, h->omega[h->cur], omega, ld));
-  if (state) {
-    hipLaunchKernelGGL(k_scatter_gid_u8, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, h->n,
-                       h->gid[h->tw], h->state[h->tw], (int8_t*)h->stage);
-    HIPOK(hipGetLastError());
-    HIPOK(hipMemcpyAsync(state, h->stage, h->n, hipMemcpyDeviceToHost, h->stream));
-    HIPOK(sync_stream(h));
-  }
-  return MFIXDEM_OK;
+  return export_particles(h, 0, h->n, pos, vel, omega, state, ld);
 }
 
 int32_t mfixdem_set_gas(mfixdem_handle* h, const double* u_g, const double* v_g,
@@ -1677,13 +1760,11 @@ int32_t mfixdem_get_p_force(mfixdem_handle* h, double* p_force) {
 
 int32_t mfixdem_get_gas(mfixdem_handle* h, double* ep_g, double* rop_s) {
   if (!h) return MFIXDEM_ERR_ARG;
-  const int nc = h->S.ncell;
-  if (ep_g) HIPOK(hipMemcpyAsync(ep_g, h->ep_g, sizeof(double) * nc, hipMemcpyDeviceToHost, h->stream));
-  if (rop_s)
-    HIPOK(hipMemcpyAsync(rop_s, h->rop_s, sizeof(double) * nc * h->S.p.nphases,
-                         hipMemcpyDeviceToHost, h->stream));
-  HIPOK(sync_stream(h));
-  return MFIXDEM_OK;
+  const size_t nc = (size_t)h->S.ncell;
+  std::vector<OutPiece> out;
+  if (ep_g) out.push_back({h->ep_g, ep_g, sizeof(double) * nc});
+  if (rop_s) out.push_back({h->rop_s, rop_s, sizeof(double) * nc * h->S.p.nphases});
+  return read_back(h, out);
 }
 
 int32_t mfixdem_init(mfixdem_handle* h) {
@@ -1886,17 +1967,11 @@ int32_t mfixdem_get_gas_drag(mfixdem_handle* h, double* f_gds, double* drag_am,
   if (!h) return MFIXDEM_ERR_ARG;
   if (!h->gas_drag_ready) return MFIXDEM_ERR_NOT_READY;
   const size_t nc = (size_t)h->S.ncell;
-  if (f_gds)
-    HIPOK(hipMemcpyAsync(f_gds, h->gd_fgds, sizeof(double) * nc, hipMemcpyDeviceToHost,
-                         h->stream));
-  if (drag_am)
-    HIPOK(hipMemcpyAsync(drag_am, h->gd_am, sizeof(double) * nc, hipMemcpyDeviceToHost,
-                         h->stream));
-  if (drag_bm)
-    HIPOK(hipMemcpyAsync(drag_bm, h->gd_bm, sizeof(double) * 3 * nc, hipMemcpyDeviceToHost,
-                         h->stream));
-  HIPOK(sync_stream(h));
-  return MFIXDEM_OK;
+  std::vector<OutPiece> out;
+  if (f_gds) out.push_back({h->gd_fgds, f_gds, sizeof(double) * nc});
+  if (drag_am) out.push_back({h->gd_am, drag_am, sizeof(double) * nc});
+  if (drag_bm) out.push_back({h->gd_bm, drag_bm, sizeof(double) * 3 * nc});
+  return read_back(h, out);
 }
 
 // mfixdem_drag_gs_gas without allocation or host-device copies: results go
@@ -2265,27 +2340,7 @@ int32_t mfixdem_ensemble_get_particles(mfixdem_handle* h, int32_t s, double* pos
   if (!h || h->nsys < 2 || s < 0 || s >= h->nsys) return MFIXDEM_ERR_ARG;
   const int off = h->sys_off[s], cap = h->sys_off[s + 1] - off;
   if (ld < cap) return MFIXDEM_ERR_ARG;
-  const int64_t S = h->stride;
-  std::vector<int> g(cap);
-  std::vector<int8_t> st(cap);
-  std::vector<double> tmp(cap);
-  HIPOK(hipMemcpyAsync(g.data(), h->gid[h->tw] + off, sizeof(int) * cap, hipMemcpyDeviceToHost,
-                       h->stream));
-  HIPOK(hipMemcpyAsync(st.data(), h->state[h->tw] + off, cap, hipMemcpyDeviceToHost, h->stream));
-  HIPOK(sync_stream(h));
-  const double* src[3] = {h->pos[h->cur], h->vel[h->cur], h->omega[h->cur]};
-  double* dst[3] = {pos, vel, omega};
-  for (int a = 0; a < 3; a++) {
-    if (!dst[a]) continue;
-    for (int c = 0; c < 3; c++) {
-      HIPOK(hipMemcpy(tmp.data(), src[a] + c * S + off, sizeof(double) * cap,
-                      hipMemcpyDeviceToHost));
-      for (int q = 0; q < cap; q++) dst[a][c * ld + g[q]] = tmp[q];
-    }
-  }
-  if (state)
-    for (int q = 0; q < cap; q++) state[g[q]] = st[q];
-  return MFIXDEM_OK;
+  return export_particles(h, off, cap, pos, vel, omega, state, ld);
 }
 
 int32_t mfixdem_set_tuning(mfixdem_handle* h, double cell_scale, int32_t row_kernel) {
