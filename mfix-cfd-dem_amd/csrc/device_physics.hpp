@@ -30,7 +30,9 @@ struct FacetDev {
   int ignore_edges;  // bit e set: contacts on edge e are ignored
 };
 
-// Everything a step kernel needs besides array pointers; passed by value.
+// Everything a step kernel needs besides array pointers; passed by value, or
+// read from a table by the ensemble kernels (the functions below take it as
+// PT, whichever address space it is in).
 struct DevParams {
   int n;            // particle slots
   int stride;       // leading dimension of SoA arrays
@@ -95,7 +97,8 @@ struct PairOut {
 
 // CALC_FORCE_DEM pair body (calc_force_dem.f:210-412) with CFRELVEL
 // (cfrelvel.f:54-77).  Returns 0 no contact, 1 contact, 2 zero distance.
-__device__ __forceinline__ int pair_force_fp64(const DevParams& P, const PairIn& a,
+template <class PT>
+__device__ __forceinline__ int pair_force_fp64(const PT& P, const PairIn& a,
                                                const double pft_in[3], PairOut& o) {
   const double r_lm = a.rL + a.rI;
   double dist[3] = {a.xI[0] - a.xL[0], a.xI[1] - a.xL[1], a.xI[2] - a.xL[2]};
@@ -164,7 +167,8 @@ __device__ __forceinline__ int pair_force_fp64(const DevParams& P, const PairIn&
 
 // Mixed precision: contact geometry test in FP64 (same contact set as the
 // FP64 path), everything after it in FP32 except the history update.
-__device__ __forceinline__ int pair_force_mixed(const DevParams& P, const PairIn& a,
+template <class PT>
+__device__ __forceinline__ int pair_force_mixed(const PT& P, const PairIn& a,
                                                 const double pft_in[3], PairOut& o) {
   const double r_lm = a.rL + a.rI;
   const double dist[3] = {a.xI[0] - a.xL[0], a.xI[1] - a.xL[1], a.xI[2] - a.xL[2]};
@@ -243,7 +247,8 @@ __device__ __forceinline__ int pair_force_mixed(const DevParams& P, const PairIn
 }
 
 // ClosestPtPointTriangle, stl_functions_des_mod.f:25-160.
-__device__ __forceinline__ void closest_pt_tri(const FacetDev& F, const double pp[3],
+template <class FT>
+__device__ __forceinline__ void closest_pt_tri(const FT& F, const double pp[3],
                                                double cp[3], int* pe, int* edge) {
   double ab[3], ac[3], ap[3];
   *pe = 0;
@@ -311,8 +316,8 @@ __device__ __forceinline__ void closest_pt_tri(const FacetDev& F, const double p
 // (calc_collision_wall_mod.f:300-606).  hist/hist_set: the facet's stored
 // tangential history.  Returns: 0 = removed (history cleared), 1 = contact
 // (fc/tow updated, hist written), 2 = skipped (edge contact ignored).
-template <bool MIXED>
-__device__ __forceinline__ int wall_contact(const DevParams& P, const FacetDev& F,
+template <bool MIXED, class PT, class FT>
+__device__ __forceinline__ int wall_contact(const PT& P, const FT& F,
                                             const double pos[3], const double vel[3],
                                             const double om[3], double r, double pmass,
                                             int ph, double hist[3], bool hist_set,
@@ -323,7 +328,8 @@ __device__ __forceinline__ int wall_contact(const DevParams& P, const FacetDev& 
   if (F.fmin > pmax) return 0;
   if (F.fmax < pmin) return 0;
   const double vv[3] = {F.v[0][0] - pos[0], F.v[0][1] - pos[1], F.v[0][2] - pos[2]};
-  const double line_t = dot3(vv, F.n);
+  const double fnrm[3] = {F.n[0], F.n[1], F.n[2]};
+  const double line_t = dot3(vv, fnrm);
   if (line_t <= -1.0001 * r) return 0;
   double cp[3];
   int pe, edge;

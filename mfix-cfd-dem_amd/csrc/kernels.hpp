@@ -128,10 +128,15 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 }
 
 // Ensembles: many independent systems in one set of particle arrays.  The
-// slots of system s are a fixed range; each slot carries its system id, and
+// slots of system s are a fixed range that starts at a multiple of 64 (the
+// slots between a system's capacity and that multiple stay NONEXISTENT), so
+// that the particles of a wavefront belong to one system and its parameters
+// are read through the scalar cache (read per lane, the step of 3M spheres in
+// 64 systems took 419 us, so 301).  Each slot carries its system id, and
 // parameters, grids, search-grid cell offsets, DES-cell offsets and rogue
-// flags are per-system tables.  The BATCH kernel variants read them; with
-// BATCH = false the kernels take the single system's blocks by value.
+// flags are per-system tables, none of which a kernel writes except the
+// flags.  The BATCH kernel variants read them; with BATCH = false the kernels
+// take the single system's blocks by value.
 struct GridDev;
 struct BatchDev {
   const uint16_t* sys;      // system of each slot
@@ -141,13 +146,30 @@ struct BatchDev {
   const int* dg_off;        // first DES cell of system s in the facet lists
   int* rogue;               // [2s]: smallest rogue id, [2s+1]: rogue count
   int nsys;
-  int sys_shift;            // bit position of the system id in the sort key
 };
+#define MFIXDEM_CONST __attribute__((address_space(4)))
+// the system of the wavefront whose particles begin at the (uniform) slot i
 template <bool BATCH>
-__device__ __forceinline__ const DevParams& sys_params(const DevParams& P0, const BatchDev& B,
-                                                       int i) {
-  if constexpr (BATCH) return B.ptab[B.sys[i]];
-  else return P0;
+__device__ __forceinline__ int wave_system(const BatchDev& B, int i) {
+  if constexpr (BATCH) return __builtin_amdgcn_readfirstlane((int)B.sys[i]);
+  else return 0;
+}
+template <bool BATCH>
+__device__ __forceinline__ decltype(auto) sys_params(const DevParams& P0, const BatchDev& B,
+                                                     int s) {
+  if constexpr (BATCH) return (((const MFIXDEM_CONST DevParams*)B.ptab)[s]);
+  else return (P0);
+}
+// a table entry that is the same in every lane, through the scalar cache
+template <class T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "");
+  const MFIXDEM_CONST uint32_t* u = (const MFIXDEM_CONST uint32_t*)p;
+  T t;
+  uint32_t* o = reinterpret_cast<uint32_t*>(&t);
+#pragma unroll
+  for (int k = 0; k < (int)(sizeof(T) / 4); k++) o[k] = u[k];
+  return t;
 }
 
 __device__ __forceinline__ void load3(const double* a, int S, int i, double v[3]) {
@@ -175,16 +197,6 @@ __device__ __forceinline__ void unpack_ijk(int c, int& I, int& J, int& K) {
 // linear IJK (FUNIJK, J fastest), 0-based
 __device__ __forceinline__ int lin_ijk(int I, int J, int K, int ni, int nj) {
   return (J - 1) + (I - 1) * nj + (K - 1) * nj * ni;
-}
-
-// 10-bit value spread to every third bit (Morton codes)
-__device__ __forceinline__ uint32_t spread10(uint32_t v) {
-  v &= 0x3ff;
-  v = (v | (v << 16)) & 0x030000FF;
-  v = (v | (v << 8)) & 0x0300F00F;
-  v = (v | (v << 4)) & 0x030C30C3;
-  v = (v | (v << 2)) & 0x09249249;
-  return v;
 }
 
 // ---------------------------------------------------- filter schemes (DES1)
@@ -546,12 +558,11 @@ __device__ __forceinline__ bool pair_touches(const StepPtrs& a, int S, const dou
 // The contact law of a pair that touches (calc_force_dem.f:263-412), for the
 // row's particle ip at xp, rp: the increments of its force and torque in
 // d[0..5]; the owner's row writes the pair's new history.
-template <bool MIXED, bool BATCH>
-__device__ __forceinline__ void pair_contact(const DevParams& P0, const StepPtrs& a,
-                                             const BatchDev& B, int ip, const double xp[3],
-                                             double rp, int j, int pid, bool owner, double d[6]) {
+template <bool MIXED, class PT>
+__device__ __forceinline__ void pair_contact(const DevParams& P0, const PT& P, const StepPtrs& a,
+                                             int ip, const double xp[3], double rp, int j,
+                                             int pid, bool owner, double d[6]) {
   const int S = P0.stride;
-  const DevParams& P = sys_params<BATCH>(P0, B, ip);
   PairIn in;
   double xj[3], vj[3], wj[3], vp[3], wp[3];
   load3(a.pos, S, j, xj);
@@ -614,9 +625,9 @@ __device__ __forceinline__ void wave_lds_fence() {
 // (xr[3] < 0) only carry their history over.  Every lane of the wavefront
 // must call this; xr is the lane's own position and radius, which the lanes
 // working on its row read from LDS.
-template <bool MIXED, bool BATCH>
-__device__ __forceinline__ void wave_pairs(const DevParams& P0, const StepPtrs& a,
-                                           const BatchDev& B, int lgw, int wbase, int e0, int e1,
+template <bool MIXED, class PT>
+__device__ __forceinline__ void wave_pairs(const DevParams& P0, const PT& P, const StepPtrs& a,
+                                           int lgw, int wbase, int e0, int e1,
                                            const double xr[4], double fc[3], double tow[3]) {
   constexpr int kQueue = 128;
   __shared__ double s_xr[kBS / 64][4][64];
@@ -682,8 +693,8 @@ __device__ __forceinline__ void wave_pairs(const DevParams& P0, const StepPtrs& 
       p = (int)(rc & rmask);
       const double xp[3] = {s_xr[w][0][p], s_xr[w][1][p], s_xr[w][2][p]};
       double d[6];
-      pair_contact<MIXED, BATCH>(P0, a, B, wbase + p, xp, s_xr[w][3][p], q_j[w][q], q_pid[w][q],
-                                 (rc & kRowOwn) != 0u, d);
+      pair_contact<MIXED>(P0, P, a, wbase + p, xp, s_xr[w][3][p], q_j[w][q], q_pid[w][q],
+                          (rc & kRowOwn) != 0u, d);
 #pragma unroll
       for (int k = 0; k < 6; k++) s_d[w][k][lane] = d[k];
     }
@@ -829,7 +840,8 @@ __device__ __forceinline__ void fused_deposit(const DevParams& P, const StepPtrs
 // particle in the cells of an outlet other than MASS_OUTFLOW takes this
 // step's acceleration and keeps only the component normal to the outlet,
 // once per such outlet.
-__device__ __forceinline__ void exit_velocity(const DevParams& P, const BcDev* bcs, int dc,
+template <class PT>
+__device__ __forceinline__ void exit_velocity(const PT& P, const BcDev* bcs, int dc,
                                            const double fc[3], double mi, double vel[3]) {
   for (int k = 0; k < P.nbc; k++) {
     const BcDev& b = bcs[k];
@@ -841,8 +853,8 @@ __device__ __forceinline__ void exit_velocity(const DevParams& P, const BcDev* b
   }
 }
 
-template <bool MIXED, int MODE, bool FILTER, bool BATCH, bool kEarlyDrag>
-__device__ __forceinline__ void step_tail(const DevParams& P0, const DevParams& P,
+template <bool MIXED, int MODE, bool FILTER, bool BATCH, bool kEarlyDrag, class PT>
+__device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
                                           const StepPtrs& a, int i, int st, double fc[3],
                                           double tow[3], bool drag, const double* s_drag,
                                           DepIn& dep) {
@@ -869,7 +881,8 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const DevParams& 
   const double mi = a.pmass[i];
   if (MODE == kModeDrag) {
     load3(a.fc, S, i, fc);
-    if (P.coupled) add_drag<MIXED, FILTER>(P, a, i, pos, vel, fc);
+    if constexpr (!BATCH)  // ensembles are uncoupled
+      if (P.coupled) add_drag<MIXED, FILTER>(P, a, i, pos, vel, fc);
     store3(a.fc, S, i, fc);
     return;
   }
@@ -878,8 +891,8 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const DevParams& 
       for (int d = 0; d < 3; d++) fc[d] = fc[d] + s_drag[d * kBS + threadIdx.x];
       for (int d = 0; d < 3; d++) fc[d] = fc[d] + s_drag[(3 + d) * kBS + threadIdx.x];
     }
-  } else if (MODE == kModeFused && P.coupled) {
-    add_drag<MIXED, FILTER>(P, a, i, pos, vel, fc);
+  } else if constexpr (MODE == kModeFused && !BATCH) {
+    if (P.coupled) add_drag<MIXED, FILTER>(P, a, i, pos, vel, fc);
   }
   if (MODE == kModeIntegrate) {
     load3(a.fc, S, i, fc);
@@ -987,14 +1000,15 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
   const bool live = (int)(threadIdx.x & 63) < (1 << lgw) && i < P0.n;
   if (!kPairs && !live) return;  // the pair modes keep every lane for the wave passes
   const int S = P0.stride;
-  const DevParams& P = sys_params<BATCH>(P0, B, live ? i : 0);
+  const int w0 = __builtin_amdgcn_readfirstlane(wbase);
+  const int sys = wave_system<BATCH>(B, w0 < P0.n ? w0 : 0);
+  decltype(auto) P = sys_params<BATCH>(P0, B, sys);
   const int st = live ? a.state[i] : 0;
   double fc[3] = {0.0, 0.0, 0.0}, tow[3] = {0.0, 0.0, 0.0};
   bool drag = false;
 
   if (kPairs) {
     // the bounds of the wavefront's entries go out with the particles' loads
-    const int w0 = __builtin_amdgcn_readfirstlane(wbase);
     const int e0 = a.nbr_start[w0 < P0.n ? w0 : P0.n];
     const int e1 = a.nbr_start[w0 + (1 << lgw) < P0.n ? w0 + (1 << lgw) : P0.n];
     double xr[4] = {0.0, 0.0, 0.0, -1.0};
@@ -1018,12 +1032,12 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
       // only normal particles meet the walls (calc_collision_wall_mod.f:
       // 105); entering and exiting ones keep their wall slots as they are
       const bool walls = st == kNormal;
-      const int dc = (BATCH ? B.dg_off[B.sys[i]] : 0) + a.dgc[i];
+      const int dc = (BATCH ? B.dg_off[sys] : 0) + a.dgc[i];
       const int fm = STL || !walls ? 0 : a.cell_fmask[dc];
       const int fl0 = STL && walls ? a.dg_foff[dc] : 0;
       const int fl1 = STL && walls ? a.dg_foff[dc + 1] : 0;
       uint8_t wm = a.wmask[i];
-      if (kEarlyDrag && P.coupled) {
+      if constexpr (kEarlyDrag) if (P.coupled) {
         double t[3], q[3];
         drag = garg_drag_terms<MIXED>(P, a, pc, pos, vel, pv, 2.0 * ri, t, q);
         if (drag)
@@ -1090,7 +1104,7 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
       if (wm != wm0) a.wmask[i] = wm;
     }
     // ---- pairs (calc_force_dem.f:180-412), summed after the walls
-    wave_pairs<MIXED, BATCH>(P0, a, B, lgw, w0, e0, e1, xr, fc, tow);
+    wave_pairs<MIXED>(P0, P, a, lgw, w0, e0, e1, xr, fc, tow);
   }
   DepIn dep;
   if (live)
@@ -1535,7 +1549,6 @@ struct GridDev {
   // neighbour-search grid
   int fn[3];
   double f_lo[3], f_inv;
-  int mbits;  // bits of the Morton code in the sort key
   // single-precision prefilter of the row walk: coordinates relative to
   // pf_c; |x - pf_c| <= pf_xmax on every axis for particles it covers;
   // pf_slack bounds the rounding of a distance so computed
@@ -1587,50 +1600,6 @@ __device__ __forceinline__ int cell_system(const BatchDev& B, int c) {
   return lo;
 }
 
-// DESGRID_PIC locate (desgrid_mod.f:900-915) + sort key on the search grid.
-// Ensembles put the system id above the Morton code, so every system keeps
-// its slot range (its empty slots sort to the end of that range).
-template <bool BATCH = false>
-__global__ __launch_bounds__(kBS) void k_bin(int n, int S, GridDev G0, const double* pos,
-                                             const uint8_t* state, const int* gid, int* dgc,
-                                             uint64_t* keys, int* vals, int* flags, BatchDev B) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n) return;
-  vals[i] = i;
-  const int s = BATCH ? B.sys[i] : 0;
-  const uint64_t sys_key = BATCH ? (uint64_t)s << B.sys_shift : 0ull;
-  if (state[i] == 0) {
-    keys[i] = BATCH ? sys_key | ((1ull << B.sys_shift) - 1) : ~0ull;
-    dgc[i] = 0;
-    return;
-  }
-  const GridDev& G = sys_grid<BATCH>(G0, B, s);
-  const double x[3] = {pos[i], pos[S + i], pos[2 * S + i]};
-  const int nn[3] = {G.dg_ni, G.dg_nj, G.dg_nk};
-  int c3[3], f3[3];
-  for (int d = 0; d < 3; d++) {
-    int v = floor_sat_d((x[d] - G.dg_lo[d]) * G.dg_inv[d]) + 2;
-    c3[d] = v < 1 ? 1 : (v > nn[d] ? nn[d] : v);
-    int f = floor_sat_d((x[d] - G.f_lo[d]) * G.f_inv);
-    f3[d] = f < 0 ? 0 : (f >= G.fn[d] ? G.fn[d] - 1 : f);
-  }
-  dgc[i] = (c3[1] - 1) + (c3[0] - 1) * G.dg_nj + (c3[2] - 1) * G.dg_nj * G.dg_ni;
-  // rogue: a normal particle in the ghost layer (only normal particles have
-  // rows, desgrid_mod.f:1096-1104); entering ones start outside the box
-  if (state[i] == kNormal && dg_ghost(G, c3[0], c3[1], c3[2])) {
-    if (BATCH) {
-      atomicMin(&B.rogue[2 * s], gid[i]);
-      atomicAdd(&B.rogue[2 * s + 1], 1);
-    }
-    atomicMin(&flags[kFlagRogueGid], gid[i]);
-    atomicAdd(&flags[kFlagRogueCount], 1);
-  }
-  // the sort is stable, so particles keep their previous relative order
-  // within a search cell (no result depends on that order)
-  const uint64_t m = (uint64_t)(spread10(f3[0]) | (spread10(f3[1]) << 1) | (spread10(f3[2]) << 2));
-  keys[i] = sys_key | m;
-}
-
 // The single-precision copy is relative to G.pf_c; a particle beyond
 // pf_xmax on some axis gets radius -1 there (every test with it is then
 // made in double precision), a nonexistent one a position no cut-off
@@ -1657,26 +1626,40 @@ __device__ __forceinline__ void pack_candidate(const GridDev& G, const double p[
   xf[k] = make_float4(f[0], f[1], f[2], in ? (float)r : -1.0f);
 }
 
-// DESGRID_PIC locate as k_bin, for one system, with a counting sort in
-// place of the key sort: each particle counts itself into its search cell
-// (cells numbered in Morton order by cell_rank; nonexistent particles into
-// a last cell after them) and keeps the place it drew.  A cell's particles
-// end up in no particular order among themselves (no result depends on it).
-__global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G, const double* pos,
+// DESGRID_PIC locate (desgrid_mod.f:900-915) and the counting of a counting
+// sort over the search cells: each particle counts itself into its search
+// cell (cells numbered in Morton order by cell_rank; nonexistent particles
+// into a last cell after them) and keeps the place it drew.  A cell's
+// particles end up in no particular order among themselves (no result
+// depends on it).  Ensembles number the systems' cells one system after
+// another, each with its own last cell, so that every system keeps its slot
+// range; there the key sort this replaces took 275 us of kernels at 3M
+// spheres and moved all particle data at every binning.
+template <bool BATCH>
+__device__ __forceinline__ int absent_cell(const BatchDev& B, int s, int nfine) {
+  return BATCH ? B.cell_off[s + 1] + s : nfine;
+}
+template <bool BATCH>
+__global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G0, const double* pos,
                                                    uint8_t* state, const int* gid,
                                                    int* dgc, const int* cell_rank,
                                                    int* cell_cnt, int nfine, uint64_t* place,
-                                                   int* flags) {
+                                                   int* flags, BatchDev B) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
-  int r = nfine;
+  const int s = wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(i));
+  int r = absent_cell<BATCH>(B, s, nfine);
   if (state[i] == kNonexistent) {
     dgc[i] = 0;
   } else {
+    GridDev Gs;
+    if constexpr (BATCH) Gs = load_uniform(B.gtab + s);
+    const GridDev& G = BATCH ? Gs : G0;
     if (state[i] == kSeeded) state[i] = kEntering;  // binned now: in a DES cell list
     const double x[3] = {pos[i], pos[S + i], pos[2 * S + i]};
     const int nn[3] = {G.dg_ni, G.dg_nj, G.dg_nk};
     int c3[3], f3[3];
+#pragma unroll
     for (int d = 0; d < 3; d++) {
       const int v = floor_sat_d((x[d] - G.dg_lo[d]) * G.dg_inv[d]) + 2;
       c3[d] = v < 1 ? 1 : (v > nn[d] ? nn[d] : v);
@@ -1684,11 +1667,17 @@ __global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G, cons
       f3[d] = f < 0 ? 0 : (f >= G.fn[d] ? G.fn[d] - 1 : f);
     }
     dgc[i] = (c3[1] - 1) + (c3[0] - 1) * G.dg_nj + (c3[2] - 1) * G.dg_nj * G.dg_ni;
-    if (state[i] == kNormal && dg_ghost(G, c3[0], c3[1], c3[2])) {  // rogue, as in k_bin
+    // rogue: a normal particle in the ghost layer (only normal particles have
+    // rows, desgrid_mod.f:1096-1104); entering ones start outside the box
+    if (state[i] == kNormal && dg_ghost(G, c3[0], c3[1], c3[2])) {
+      if (BATCH) {
+        atomicMin(&B.rogue[2 * s], gid[i]);
+        atomicAdd(&B.rogue[2 * s + 1], 1);
+      }
       atomicMin(&flags[kFlagRogueGid], gid[i]);
       atomicAdd(&flags[kFlagRogueCount], 1);
     }
-    r = cell_rank[f3[0] + G.fn[0] * (f3[1] + G.fn[1] * f3[2])];
+    r = cell_rank[(BATCH ? B.cell_off[s] : 0) + f3[0] + G.fn[0] * (f3[1] + G.fn[1] * f3[2])];
   }
   // The particles are still in the last binning's order, so neighbouring
   // lanes mostly share a cell: each run of equal cells takes its places
@@ -1721,11 +1710,14 @@ struct BinPack {               // k_bin_place's packing of the row walk's candid
   double* xr;
   float4* xf;
 };
-__global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, const uint64_t* place,
+template <bool BATCH>
+__global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, int nsys,
+                                                   const uint64_t* place,
                                                    const int* cell_rank, const int* cell_off,
                                                    int* cell_cnt, int* perm, int* inv,
                                                    int* cstart, int* cend, int* zero0,
-                                                   int* zero1, int* zero2, BinPack bp) {
+                                                   int* zero1, int* zero2, BinPack bp,
+                                                   BatchDev B) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i < n) {
     const uint64_t p = place[i];
@@ -1733,8 +1725,11 @@ __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, const uint6
     perm[np] = i;
     inv[i] = np;
     // the candidate data of the row walk, at the particle's new place
+    GridDev Gs;
+    if constexpr (BATCH)
+      Gs = load_uniform(B.gtab + wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(i)));
     const double x[3] = {bp.pos[i], bp.pos[bp.S + i], bp.pos[2 * bp.S + i]};
-    pack_candidate(bp.G, x, bp.radius[i], bp.state[i] != 0, bp.xr, bp.xf, np);
+    pack_candidate(BATCH ? Gs : bp.G, x, bp.radius[i], bp.state[i] != 0, bp.xr, bp.xf, np);
     zero0[i] = 0;  // the row counters of the neighbour build that follows
     zero1[i] = 0;
     zero2[i] = 0;
@@ -1745,7 +1740,7 @@ __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, const uint6
     cend[i] = cell_off[r + 1];
     cell_cnt[r] = 0;
   }
-  if (i == 0) cell_cnt[nfine] = 0;
+  if (i < nsys) cell_cnt[absent_cell<BATCH>(B, i, nfine)] = 0;
 }
 
 struct PermPtrs {
@@ -1796,35 +1791,6 @@ __global__ __launch_bounds__(kBS) void k_permute(int n, int S, PermPtrs p) {
       p.acc_o[c * S + i] = p.acc[c * S + o];
       p.racc_o[c * S + i] = p.racc[c * S + o];
     }
-}
-
-__device__ __forceinline__ uint32_t compact10(uint64_t v) {
-  v &= 0x09249249;
-  v = (v | (v >> 2)) & 0x030C30C3;
-  v = (v | (v >> 4)) & 0x0300F00F;
-  v = (v | (v >> 8)) & 0x030000FF;
-  v = (v | (v >> 16)) & 0x3ff;
-  return (uint32_t)v;
-}
-
-// search-grid cell ranges of the sorted particles (from the Morton part of
-// the sort key)
-template <bool BATCH = false>
-__global__ __launch_bounds__(kBS) void k_cell_ranges(int n, GridDev G0, const uint64_t* keys,
-                                                     const uint8_t* state, int* cstart,
-                                                     int* cend, BatchDev B) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n || state[i] == 0) return;
-  const int s = BATCH ? B.sys[i] : 0;
-  const GridDev& G = sys_grid<BATCH>(G0, B, s);
-  const uint64_t k = keys[i];  // system id (ensembles) and Morton code
-  const bool first = (i == 0) || keys[i - 1] != k;
-  const bool last = (i + 1 == n) || keys[i + 1] != k;
-  const uint64_t m = k & ((1ull << G.mbits) - 1);
-  const int c = (BATCH ? B.cell_off[s] : 0) + (int)compact10(m) +
-                G.fn[0] * ((int)compact10(m >> 1) + G.fn[1] * (int)compact10(m >> 2));
-  if (first) cstart[c] = i;
-  if (last) cend[c] = i + 1;
 }
 
 struct BuildPtrs {
@@ -1942,8 +1908,15 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
   if (hp >= n) return;
   const int h = b.idx ? b.idx[hp] : hp;                   // and slot
   if (b.state[h] == 0) return;
-  const int s = BATCH ? B.sys[h] : 0;
-  const GridDev& G = sys_grid<BATCH>(G0, B, s);
+  // a system's positions are its slot range: with two lanes per particle a
+  // wavefront's 32 positions are of one system
+  constexpr bool kUniform = BATCH && kRowLanes == 2;
+  const int s = kUniform ? wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(hp))
+                         : (BATCH ? B.sys[hp] : 0);
+  GridDev Gs;
+  if constexpr (kUniform) Gs = load_uniform(B.gtab + s);
+  else if constexpr (BATCH) Gs = B.gtab[s];
+  const GridDev& G = BATCH ? Gs : G0;
   const int cbase = BATCH ? B.cell_off[s] : 0;
   const int g_r = BATCH ? B.rogue[2 * s] : b.flags[kFlagRogueGid];
   const double x[3] = {b.pos[h], b.pos[S + h], b.pos[2 * S + h]};
@@ -1994,7 +1967,7 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
     }
     const int tn = k < m ? t : tc;  // in range either way
     u = b.xf[tn];
-    const float lim = frlm * (xh.w + uc.w) + G0.pf_slack;  // the grid k_pack_xr used
+    const float lim = frlm * (xh.w + uc.w) + G.pf_slack;
     const float e0 = xh.x - uc.x, e1 = xh.y - uc.y, e2 = xh.z - uc.z;
     if (coarse && uc.w >= 0.0f && e0 * e0 + e1 * e1 + e2 * e2 > lim * lim) continue;
     if (nh < kHits) s_hit[nh++][threadIdx.x] = tc;
@@ -2076,14 +2049,16 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
 // five), after a binning that did not pack them (k_bin_place does).  A
 // nonexistent particle gets a position no cut-off reaches, so the walk
 // needs no state load; the hit path checks the state itself.
-__global__ __launch_bounds__(kBS) void k_pack_xr(int n, int S, GridDev G, const int* idx,
+template <bool BATCH>
+__global__ __launch_bounds__(kBS) void k_pack_xr(int n, int S, GridDev G0, const int* idx,
                                                  const double* pos, const double* radius,
-                                                 const uint8_t* state, double* xr, float4* xf) {
+                                                 const uint8_t* state, double* xr, float4* xf,
+                                                 BatchDev B) {
   const int k = blockIdx.x * kBS + threadIdx.x;  // position in the search-cell order
   if (k >= n) return;
   const int i = idx ? idx[k] : k;
   const double p[3] = {pos[i], pos[S + i], pos[2 * S + i]};
-  pack_candidate(G, p, radius[i], state[i] != 0, xr, xf, k);
+  pack_candidate(BATCH ? B.gtab[B.sys[i]] : G0, p, radius[i], state[i] != 0, xr, xf, k);
 }
 
 // Own rows, one wavefront per search-grid cell.  The candidates of the 27
@@ -2617,13 +2592,6 @@ __global__ __launch_bounds__(kBS) void k_seed(int ns, const SeedDev* sd, SeedPtr
   p.phase[i] = (uint8_t)d.phase;
   p.wmask[i] = 0;
   p.state[i] = kSeeded;
-}
-
-// the inverse of a binning's order (ensembles, whose key sort gives the
-// order only)
-__global__ __launch_bounds__(kBS) void k_invert(int n, const int* perm, int* inv) {
-  const int k = blockIdx.x * kBS + threadIdx.x;
-  if (k < n) inv[perm[k]] = k;
 }
 
 // slot of each global id, after a binning has reordered the slots
@@ -3302,18 +3270,19 @@ __global__ __launch_bounds__(kBS) void k_delete_outside(int n, int S, const int*
 }
 
 // ------------------------------------------------------------- exports
-// The particles of n slots in global-id order for the host, one launch for
+// The n particles of nslots slots in global-id order for the host, one launch for
 // all of them: the given arrays' component planes (null: not wanted) and
 // PARTICLE_STATE, packed one after another into out, so that one stream of
 // copies takes them to the host.  A thread reads its slot coalesced and
 // writes 8 bytes to each plane at its id.
-__global__ __launch_bounds__(kBS) void k_export(int n, int S, const int* gid,
+__global__ __launch_bounds__(kBS) void k_export(int nslots, int n, int S, const int* gid,
                                                 const uint8_t* state, const double* pos,
                                                 const double* vel, const double* omega,
                                                 bool want_state, double* out) {
   const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n) return;
+  if (i >= nslots) return;
   const int g = gid[i];
+  if (g >= n) return;  // a slot that fills an ensemble member's range up to a multiple of 64
   const double* src[3] = {pos, vel, omega};
   double* o = out + g;
 #pragma unroll

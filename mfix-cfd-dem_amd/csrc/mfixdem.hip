@@ -11,7 +11,6 @@
 // the coupled 1M-sphere bed: 227 -> 216).
 #include <hip/hip_runtime.h>
 #include <cstring>
-#include <rocprim/device/device_radix_sort.hpp>
 
 #include <algorithm>
 #include <climits>
@@ -57,10 +56,10 @@ struct mfixdem_handle {
   // ensembles (nsys > 1): per-system set-ups and device tables
   int nsys = 1;
   BatchDev B{};
-  int key_bits = 0;                       // significant bits of the rebuild sort key
   std::vector<Setup> sys_setup;           // per system (ensembles)
   std::vector<GridDev> sys_grid;          // per-system grids (host copy of d_gtab)
-  std::vector<int> sys_off;               // first slot of each system (+ total)
+  std::vector<int> sys_off;               // first slot of each system (+ total), multiples of 64
+  std::vector<int> sys_cap;               // capacity of each system
   std::vector<int> sys_n;                 // particles set per system
   std::vector<int> rogue_init;            // {INT_MAX, 0} per system
   uint16_t* d_sys = nullptr;
@@ -86,14 +85,12 @@ struct mfixdem_handle {
   double* wpft[2]{};    // and history per slot
   double *fc = nullptr, *tow = nullptr, *fc_id = nullptr, *tow_id = nullptr;
   // rebuild
-  uint64_t* keys[2]{};
+  uint64_t* place = nullptr;
   int* vals[2]{};
-  void* sort_tmp = nullptr;
-  size_t sort_tmp_bytes = 0;
   int *fstart = nullptr, *fend = nullptr;
   int n_fine = 0;
-  // one system: counting sort over the search cells (Morton rank of each
-  // cell, counts with one more cell for nonexistent particles, their scan)
+  // counting sort over the search cells (Morton rank of each cell, counts
+  // with one more cell per system for its nonexistent particles, their scan)
   int *fine_rank = nullptr, *fine_cnt = nullptr, *fine_off = nullptr;
   int *own_cnt = nullptr, *own_tmp = nullptr, *in_cnt = nullptr, *in_cur = nullptr,
       *tot_cnt = nullptr;
@@ -195,18 +192,6 @@ namespace {
 inline int nblk(int64_t n) { return (int)((n + kBS - 1) / kBS); }
 inline int field_blocks(int64_t ncell) {
   return (int)((ncell + kFieldCells - 1) / kFieldCells);
-}
-
-// Stable LSD radix sort of (key, slot) pairs on key bits [0, bits).  The
-// library default switches to a merge sort up to 2^20 items; for the few
-// key bits used here the onesweep radix passes are several times faster,
-// so the merge-sort limit is set to 0.
-using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
-                                              rocprim::default_config, 0>;
-hipError_t sort_pairs(void* tmp, size_t& bytes, const uint64_t* kin, uint64_t* kout,
-                      const int* vin, int* vout, int n, int bits, hipStream_t s) {
-  return rocprim::radix_sort_pairs<SortConfig>(tmp, bytes, kin, kout, vin, vout, (size_t)n, 0u,
-                                               (unsigned)bits, s);
 }
 
 template <typename T>
@@ -480,8 +465,8 @@ int32_t do_bin(mfixdem_handle* h) {
   // only the rebuild flags are reset here
   const bool thread_rows = h->S.p.des_neighbor_search != MFIXDEM_NSEARCH_NSQUARE &&
                            (h->row_kernel == MFIXDEM_ROWS_THREAD || h->P.nbc);
-  const bool permute = h->nsys > 1 || !thread_rows || !h->order_set ||
-                       h->bins_since_permute + 1 >= kPermuteEvery;
+  const bool permute =
+      !thread_rows || !h->order_set || h->bins_since_permute + 1 >= kPermuteEvery;
   if (!h->flags_set) {
     HIPOK(hipMemcpyAsync(h->flags + kFlagRogueGid, init, 2 * sizeof(int),
                          hipMemcpyHostToDevice, h->stream));
@@ -494,39 +479,32 @@ int32_t do_bin(mfixdem_handle* h) {
     HIPOK(hipMemcpyAsync(h->d_rogue, h->rogue_init.data(), sizeof(int) * 2 * h->nsys,
                          hipMemcpyHostToDevice, h->stream));
   const int t = h->tw, c = h->cur;
-  if (batch) {  // ensembles: key sort (system id above the Morton code)
-    hipLaunchKernelGGL((k_bin<true>), dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
-                       h->pos[c], h->state[t], h->gid[t], h->dgc[t], h->keys[0], h->vals[0],
-                       h->flags, h->B);
-    HIPOK(hipGetLastError());
-    size_t tb = h->sort_tmp_bytes;
-    HIPOK(sort_pairs(h->sort_tmp, tb, h->keys[0], h->keys[1], h->vals[0], h->vals[1], n,
-                     h->key_bits, h->stream));
-    hipLaunchKernelGGL(k_invert, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->vals[1],
-                       h->vals[0]);
-    HIPOK(hipGetLastError());
-  } else {  // one system: counting sort over the search cells
-    const int nf = h->n_fine;
-    hipLaunchKernelGGL(k_bin_count, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
+  const int nf = h->n_fine;
+  BinPack bp{};
+  bp.G = h->G;
+  bp.S = S;
+  bp.pos = h->pos[c];
+  bp.radius = h->radius[t];
+  bp.state = h->state[t];
+  bp.xr = h->xr_pack;
+  bp.xf = reinterpret_cast<float4*>(h->stage);
+  auto bin = [&](auto many) -> int32_t {
+    constexpr bool kB = decltype(many)::value;
+    hipLaunchKernelGGL(k_bin_count<kB>, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
                        h->pos[c], h->state[t], h->gid[t], h->dgc[t], h->fine_rank, h->fine_cnt,
-                       nf, h->keys[0], h->flags);
+                       nf, h->place, h->flags, h->B);
     HIPOK(hipGetLastError());
-    CHECKRC(scan_i32(h, h->fine_cnt, h->fine_off, (int64_t)nf + 1));
-    BinPack bp{};
-    bp.G = h->G;
-    bp.S = S;
-    bp.pos = h->pos[c];
-    bp.radius = h->radius[t];
-    bp.state = h->state[t];
-    bp.xr = h->xr_pack;
-    bp.xf = reinterpret_cast<float4*>(h->stage);
-    hipLaunchKernelGGL(k_bin_place, dim3(nblk(std::max(n, nf))), dim3(kBS), 0, h->stream, n, nf,
-                       h->keys[0], h->fine_rank, h->fine_off, h->fine_cnt, h->vals[1],
-                       h->vals[0], h->fstart, h->fend, h->own_cnt, h->in_cnt, h->in_cur, bp);
+    CHECKRC(scan_i32(h, h->fine_cnt, h->fine_off, (int64_t)nf + h->nsys));
+    hipLaunchKernelGGL(k_bin_place<kB>, dim3(nblk(std::max(std::max(n, nf), h->nsys))), dim3(kBS),
+                       0, h->stream, n, nf, h->nsys, h->place, h->fine_rank, h->fine_off,
+                       h->fine_cnt, h->vals[1], h->vals[0], h->fstart, h->fend, h->own_cnt,
+                       h->in_cnt, h->in_cur, bp, h->B);
     HIPOK(hipGetLastError());
-    h->counts_zeroed = true;
-    h->xr_packed = true;
-  }
+    return MFIXDEM_OK;
+  };
+  CHECKRC(batch ? bin(std::true_type{}) : bin(std::false_type{}));
+  h->counts_zeroed = true;
+  h->xr_packed = true;
   PermPtrs p{};
   p.perm = h->vals[1];
   p.pos = h->pos[c]; p.vel = h->vel[c]; p.omega = h->omega[c];
@@ -555,13 +533,6 @@ int32_t do_bin(mfixdem_handle* h) {
     h->bin_idx = h->vals[1];
     h->bin_inv = nullptr;
     h->bins_since_permute++;
-  }
-  if (batch) {
-    CHECKRC(fill_i32(h->stream, h->fstart, h->n_fine, 0));
-    CHECKRC(fill_i32(h->stream, h->fend, h->n_fine, 0));
-    hipLaunchKernelGGL((k_cell_ranges<true>), dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->G,
-                       h->keys[1], h->state[h->tw], h->fstart, h->fend, h->B);
-    HIPOK(hipGetLastError());
   }
   if (h->slot_of_gid) {  // inlets place their seeds by global id
     hipLaunchKernelGGL(k_slot_of_gid, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->gid[h->tw],
@@ -685,10 +656,12 @@ int32_t do_neighbour(mfixdem_handle* h) {
         CHECKRC(fill_i32(h->stream, h->own_cnt, n, 0));
         CHECKRC(fill_i32(h->stream, h->in_cnt, n, 0));
       }
-      if (!packed)
-        hipLaunchKernelGGL(k_pack_xr, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
-                           b.idx, b.pos, b.radius, b.state, h->xr_pack,
-                           reinterpret_cast<float4*>(h->stage));
+      if (!packed) {
+        auto pack = h->nsys > 1 ? k_pack_xr<true> : k_pack_xr<false>;
+        hipLaunchKernelGGL(pack, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G, b.idx,
+                           b.pos, b.radius, b.state, h->xr_pack,
+                           reinterpret_cast<float4*>(h->stage), h->B);
+      }
       auto rows = [&](auto lanes) {
         constexpr int kL = decltype(lanes)::value;
         const dim3 rg(nblk((int64_t)n * kL)), blk(kBS);
@@ -702,8 +675,10 @@ int32_t do_neighbour(mfixdem_handle* h) {
       // have more hits than their LDS lists hold), else 2.  Measured (2 / 7 /
       // 14 lanes): 2,003 settled spheres 39 / 14 / 11 us; 301,057 211 / 170 /
       // 192; 120,000 at 4 pairs each 30 / 31 / 40; 1M at 1.6, 126 / 181 / 262.
+      // (Ensembles of any size but a small one keep 2, whose wavefronts read one
+      // system's grid.)
       if (n <= 20480) rows(std::integral_constant<int, 14>{});
-      else if (n <= 65536 || (h->n_pairs >= 5 * (int64_t)n && n < (1 << 24)))
+      else if (h->nsys == 1 && (n <= 65536 || (h->n_pairs >= 5 * (int64_t)n && n < (1 << 24))))
         rows(std::integral_constant<int, 7>{});
       else rows(std::integral_constant<int, 2>{});
     }
@@ -921,12 +896,12 @@ bool rebin_each_step(const mfixdem_handle* h) {
 
 // The free global ids, from the particle states (at init, and after rogue
 // particles have been removed).
-int32_t export_particles(mfixdem_handle* h, int first, int n, double* pos, double* vel,
-                         double* omega, int8_t* state, int64_t ld);
+int32_t export_particles(mfixdem_handle* h, int first, int nslots, int n, double* pos,
+                         double* vel, double* omega, int8_t* state, int64_t ld);
 int32_t refresh_free_gids(mfixdem_handle* h) {
   const int n = h->n;
   std::vector<int8_t> st(n);
-  CHECKRC(export_particles(h, 0, n, nullptr, nullptr, nullptr, st.data(), n));
+  CHECKRC(export_particles(h, 0, n, n, nullptr, nullptr, nullptr, st.data(), n));
   h->dbc.free_gids.clear();
   for (int g = 0; g < n; g++)
     if (st[g] == kNonexistent) h->dbc.free_gids.insert(g);
@@ -1103,14 +1078,14 @@ int32_t read_back(mfixdem_handle* h, const std::vector<OutPiece>& pieces) {
   return rc;
 }
 
-// The particles of n slots from slot first on (one system, or a member of an
-// ensemble), in global-id order with leading dimension ld.
-int32_t export_particles(mfixdem_handle* h, int first, int n, double* pos, double* vel,
-                         double* omega, int8_t* state, int64_t ld) {
+// The n particles of the nslots slots from slot first on (one system, or a
+// member of an ensemble), in global-id order with leading dimension ld.
+int32_t export_particles(mfixdem_handle* h, int first, int nslots, int n, double* pos,
+                         double* vel, double* omega, int8_t* state, int64_t ld) {
   const int c = h->cur, t = h->tw;
   if (n <= 0 || !(pos || vel || omega || state)) return MFIXDEM_OK;
   h->xr_packed = false;  // the stage held them
-  hipLaunchKernelGGL(k_export, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->stride,
+  hipLaunchKernelGGL(k_export, dim3(nblk(nslots)), dim3(kBS), 0, h->stream, nslots, n, h->stride,
                      h->gid[t] + first, h->state[t] + first, pos ? h->pos[c] + first : nullptr,
                      vel ? h->vel[c] + first : nullptr, omega ? h->omega[c] + first : nullptr,
                      state != nullptr, h->stage);
@@ -1250,6 +1225,10 @@ int32_t upload_ensemble(mfixdem_handle* h) {
   h->n_pairs = 0;
   h->first_pass = true;
   h->binned = false;
+  h->order_set = false;  // the first binning puts the new particles in order
+  h->xr_packed = h->counts_zeroed = false;
+  h->bin_idx = h->bin_inv = nullptr;
+  h->bins_since_permute = 0;
   return MFIXDEM_OK;
 }
 
@@ -1262,12 +1241,12 @@ void for_each_buffer(mfixdem_handle* h, F f) {
     f(h->pmass[b]); f(h->omoi[b]); f(h->pvol[b]); f(h->acc[b]);
     f(h->racc[b]); f(h->gid[b]); f(h->fcell[b]); f(h->dgc[b]);
     f(h->state[b]); f(h->phase[b]); f(h->wmask[b]); f(h->wfid[b]); f(h->wpft[b]);
-    f(h->keys[b]); f(h->vals[b]); f(h->nbr_start[b]); f(h->nbr_split[b]);
+    f(h->vals[b]); f(h->nbr_start[b]); f(h->nbr_split[b]);
     f(h->pair_base[b]); f(h->nbr[b]); f(h->nbr_pid[b]); f(h->nbr_row[b]); f(h->pft[b]); f(h->pfl[b]);
     f(h->rops_fix[b]);
   }
-  f(h->fc); f(h->tow); f(h->fc_id); f(h->tow_id); f(h->sort_tmp); f(h->rm_cnt); f(h->rm_list); f(h->f_gp); f(h->drag_fc);
-  f(h->xr_pack); f(h->in_tmp);
+  f(h->fc); f(h->tow); f(h->fc_id); f(h->tow_id); f(h->rm_cnt); f(h->rm_list); f(h->f_gp); f(h->drag_fc);
+  f(h->xr_pack); f(h->in_tmp); f(h->place);
   f(h->fstart); f(h->fend); f(h->fine_rank); f(h->fine_cnt); f(h->fine_off);
   f(h->own_cnt); f(h->own_tmp); f(h->own_key); f(h->in_cnt); f(h->in_cur);
   f(h->tot_cnt); f(h->scan_bsum); f(h->scan_bsum64); f(h->flags); f(h->csz); f(h->xe); f(h->yn);
@@ -1285,46 +1264,57 @@ void fill_devparams(mfixdem_handle* h) {
   h->P.nbc = (int)h->dbc.b.size();
 }
 
-// Search cells of one system for the counting sort: the rank of each cell
-// (x fastest) in the Morton order of its (fx, fy, fz), so that the binned
-// particles lie in Morton order; zeroed counts.
+// Walks the cells of a grid in Morton order (octants of a cube that covers
+// the grid, those outside it skipped): rank[cell] = next place.
+void morton_ranks(const int fn[3], int x, int y, int z, int size, int* rank, int& next) {
+  if (x >= fn[0] || y >= fn[1] || z >= fn[2]) return;
+  if (size == 1) {
+    rank[x + fn[0] * (y + fn[1] * z)] = next++;
+    return;
+  }
+  const int s = size / 2;
+  for (int o = 0; o < 8; o++)
+    morton_ranks(fn, x + (o & 1) * s, y + ((o >> 1) & 1) * s, z + (o >> 2) * s, s, rank, next);
+}
+
+// Search cells for the counting sort: the rank of each cell (x fastest) in
+// the Morton order of its (fx, fy, fz), so that the binned particles lie in
+// Morton order, system after system, each followed by the place of its
+// nonexistent particles; zeroed counts.
 int32_t setup_fine_cells(mfixdem_handle* h) {
   dfree(h->fine_rank);
   dfree(h->fine_cnt);
   dfree(h->fine_off);
-  if (h->nsys > 1) return MFIXDEM_OK;
-  const GridDev& G = h->G;
-  const int nf = h->n_fine;
-  if ((int64_t)G.fn[0] * G.fn[1] * G.fn[2] != nf) return MFIXDEM_ERR_ARG;
-  auto spread = [](uint64_t v) {
-    uint64_t r = 0;
-    for (int b = 0; b < 10; b++) r |= ((v >> b) & 1ull) << (3 * b);
-    return r;
-  };
-  std::vector<std::pair<uint64_t, int>> code((size_t)nf);
-  for (int z = 0, c = 0; z < G.fn[2]; z++)
-    for (int y = 0; y < G.fn[1]; y++)
-      for (int x = 0; x < G.fn[0]; x++, c++)
-        code[c] = {spread(x) | (spread(y) << 1) | (spread(z) << 2), c};
-  std::sort(code.begin(), code.end());
+  const int nf = h->n_fine, ns = h->nsys;
   std::vector<int> rank((size_t)nf);
-  for (int k = 0; k < nf; k++) rank[code[k].second] = k;
+  int64_t cell = 0;
+  int next = 0;
+  for (int s = 0; s < ns; s++, next++) {
+    const int* fn = ns > 1 ? h->sys_grid[s].fn : h->G.fn;
+    int size = 1;
+    while (size < std::max(fn[0], std::max(fn[1], fn[2]))) size *= 2;
+    const int64_t cells = (int64_t)fn[0] * fn[1] * fn[2];
+    if (cell + cells > nf) return MFIXDEM_ERR_ARG;
+    morton_ranks(fn, 0, 0, 0, size, rank.data() + cell, next);
+    cell += cells;
+  }
+  if (cell != nf) return MFIXDEM_ERR_ARG;
   CHECKRC(dalloc(&h->fine_rank, nf));
-  CHECKRC(dalloc(&h->fine_cnt, (int64_t)nf + 1));
-  CHECKRC(dalloc(&h->fine_off, (int64_t)nf + 2));
+  CHECKRC(dalloc(&h->fine_cnt, (int64_t)nf + ns));
+  CHECKRC(dalloc(&h->fine_off, (int64_t)nf + ns + 1));
   HIPOK(hipMemcpy(h->fine_rank, rank.data(), sizeof(int) * nf, hipMemcpyHostToDevice));
-  HIPOK(hipMemset(h->fine_cnt, 0, sizeof(int) * ((size_t)nf + 1)));
+  HIPOK(hipMemset(h->fine_cnt, 0, sizeof(int) * ((size_t)nf + ns)));
   return MFIXDEM_OK;
 }
 
 // Device buffers, stream and events of a handle whose set-up (S, P, G,
-// n, stride, n_fine, key_bits) is filled in.  On failure the caller
+// n, stride, n_fine) is filled in.  On failure the caller
 // destroys the handle.
 int32_t alloc_buffers(mfixdem_handle* h) {
   const int64_t n = h->n, S = h->stride, nc = h->S.ncell;
   int64_t max_cap = h->nsys > 1 ? 0 : n;  // the most particles of one system
   for (int s = 0; s < h->nsys && h->nsys > 1; s++)
-    max_cap = std::max<int64_t>(max_cap, h->sys_off[s + 1] - h->sys_off[s]);
+    max_cap = std::max<int64_t>(max_cap, h->sys_cap[s]);
   int32_t rc = MFIXDEM_OK;
   auto fail = [&](int32_t r) { return r; };
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
@@ -1339,13 +1329,13 @@ int32_t alloc_buffers(mfixdem_handle* h) {
         (rc = dalloc(&h->state[b], S)) || (rc = dalloc(&h->phase[b], S)) ||
         (rc = dalloc(&h->wmask[b], S)) || (rc = dalloc(&h->wfid[b], kWallSlots * S)) ||
         (rc = dalloc(&h->wpft[b], 3 * kWallSlots * S)) ||
-        (rc = dalloc(&h->keys[b], n)) || (rc = dalloc(&h->vals[b], n)) ||
+        (rc = dalloc(&h->vals[b], n)) ||
         (rc = dalloc(&h->nbr_start[b], n + 1)) || (rc = dalloc(&h->nbr_split[b], n)) ||
         (rc = dalloc(&h->pair_base[b], n + 1)))
       return fail(rc);
   }
   if ((rc = dalloc(&h->fc, 3 * S)) || (rc = dalloc(&h->tow, 3 * S)) ||
-      (rc = dalloc(&h->xr_pack, 4 * S)) ||
+      (rc = dalloc(&h->xr_pack, 4 * S)) || (rc = dalloc(&h->place, n)) ||
       (rc = dalloc(&h->fc_id, 3 * S)) || (rc = dalloc(&h->tow_id, 3 * S)) ||
       (rc = dalloc(&h->fstart, h->n_fine)) || (rc = dalloc(&h->fend, h->n_fine)) ||
       (rc = dalloc(&h->own_cnt, n)) || (rc = dalloc(&h->own_tmp, n * h->maxrow)) ||
@@ -1353,7 +1343,7 @@ int32_t alloc_buffers(mfixdem_handle* h) {
       (rc = dalloc(&h->in_cur, n)) || (rc = dalloc(&h->tot_cnt, n)) ||
       (rc = dalloc(&h->scan_bsum64, n / kScanTile + 2)) ||
       (rc = dalloc(&h->scan_bsum,
-                   std::max<int64_t>(std::max<int64_t>(n, nc), (int64_t)h->n_fine + 1) /
+                   std::max<int64_t>(std::max<int64_t>(n, nc), (int64_t)h->n_fine + h->nsys) /
                            kScanTile + 2)) ||
       (rc = dalloc(&h->flags, kFlagCount)) || (rc = dalloc(&h->xe, h->S.ni + 1)) ||
       (rc = dalloc(&h->csz, h->S.ni + h->S.nj + h->S.nk)) ||
@@ -1381,11 +1371,6 @@ int32_t alloc_buffers(mfixdem_handle* h) {
         hipMemset(h->drag_fc, 0, sizeof(double) * 3 * n) != hipSuccess)
       return fail(MFIXDEM_ERR_HIP);
   }
-  if (sort_pairs(nullptr, h->sort_tmp_bytes, h->keys[0], h->keys[1], h->vals[0], h->vals[1],
-                 (int)n, h->key_bits, h->stream) != hipSuccess)
-    return fail(MFIXDEM_ERR_HIP);
-  if (hipMalloc(&h->sort_tmp, std::max<size_t>(h->sort_tmp_bytes, 16)) != hipSuccess)
-    return fail(MFIXDEM_ERR_OOM);
   if ((rc = upload_setup(h)) || (rc = setup_fine_cells(h))) return fail(rc);
   if (hipMemset(h->flags, 0, sizeof(int) * kFlagCount) != hipSuccess) return fail(MFIXDEM_ERR_HIP);
   if (hipHostMalloc((void**)&h->host_flags, sizeof(HostFlags), hipHostMallocDefault) != hipSuccess)
@@ -1492,7 +1477,6 @@ int32_t mfixdem_create(const mfixdem_params* p, mfixdem_handle** out) {
     delete h;
     return MFIXDEM_ERR_UNSUPPORTED;
   }
-  h->key_bits = h->G.mbits;
   if ((rc = alloc_buffers(h)) || (rc = bind_scratch(h))) {
     mfixdem_destroy(h);
     return rc;
@@ -1700,7 +1684,7 @@ int32_t mfixdem_get_particles(mfixdem_handle* h, double* pos, double* vel, doubl
                               int8_t* state, int64_t ld) {
   if (h && h->nsys > 1) return MFIXDEM_ERR_ARG;  // single-system call
   if (!h || ld < h->n) return MFIXDEM_ERR_ARG;
-  return export_particles(h, 0, h->n, pos, vel, omega, state, ld);
+  return export_particles(h, 0, h->n, h->n, pos, vel, omega, state, ld);
 }
 
 int32_t mfixdem_set_gas(mfixdem_handle* h, const double* u_g, const double* v_g,
@@ -2207,6 +2191,7 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
   h->sys_setup.resize(nsys);
   h->sys_off.assign(nsys + 1, 0);
   h->sys_n.assign(nsys, 0);
+  h->sys_cap.assign(nsys, 0);
   for (int s = 0; s < nsys; s++) {
     const mfixdem_params& q = p[s];
     int32_t rc = build_setup(q, h->sys_setup[s]);
@@ -2219,11 +2204,13 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
       delete h;
       return rc;
     }
-    h->sys_off[s + 1] = h->sys_off[s] + q.max_pip;
-  }
-  if ((int64_t)h->sys_off[nsys] > INT_MAX / 4) {
-    delete h;
-    return MFIXDEM_ERR_ARG;
+    const int64_t end = (int64_t)h->sys_off[s] + q.max_pip;
+    if (end > INT_MAX / 4) {
+      delete h;
+      return MFIXDEM_ERR_ARG;
+    }
+    h->sys_off[s + 1] = (int)(nsys > 1 ? (end + 63) / 64 * 64 : end);
+    h->sys_cap[s] = q.max_pip;
   }
   h->S = h->sys_setup[0];
   h->n = h->sys_off[nsys];
@@ -2232,7 +2219,6 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
   std::vector<DevParams> ptab(nsys);
   std::vector<GridDev> gtab(nsys);
   std::vector<int> cell_off(nsys + 1, 0), dg_off(nsys + 1, 0);
-  int mbits = 3;
   for (int s = 0; s < nsys; s++) {
     const Setup& S = h->sys_setup[s];
     fill_params(S, h->n, h->stride, ptab[s], gtab[s]);
@@ -2241,23 +2227,15 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
       delete h;
       return MFIXDEM_ERR_UNSUPPORTED;
     }
-    mbits = std::max(mbits, gtab[s].mbits);
     cell_off[s + 1] = cell_off[s] + nfine;
     dg_off[s + 1] = dg_off[s] + S.dg_ncell;
   }
-  int sys_bits = 0;
-  while ((1 << sys_bits) < nsys) sys_bits++;
-  if (mbits + sys_bits > 64) {
-    delete h;
-    return MFIXDEM_ERR_UNSUPPORTED;
-  }
-  for (auto& g : gtab) g.mbits = mbits;
   h->G = gtab[0];
   // a handle-level flag that rebuild stages apply to every slot: carry
   // Adams-Bashforth history if any member uses it
   for (int s = 0; s < nsys; s++) h->P.ab2 = std::max(h->P.ab2, ptab[s].ab2);
   h->n_fine = cell_off[nsys];
-  h->key_bits = mbits + sys_bits;
+  h->sys_grid = gtab;
   int32_t rc = alloc_buffers(h);
   std::vector<uint16_t> sys(h->stride, 0);
   for (int s = 0; s < nsys; s++)
@@ -2296,8 +2274,6 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
   h->B.dg_off = h->d_dg_off;
   h->B.rogue = h->d_rogue;
   h->B.nsys = nsys;
-  h->B.sys_shift = mbits;
-  h->sys_grid = gtab;
   const size_t S = h->stride;
   h->st_pos.assign(3 * S, 0.0);
   h->st_vel.assign(3 * S, 0.0);
@@ -2314,7 +2290,7 @@ int32_t mfixdem_ensemble_set_particles(mfixdem_handle* h, int32_t s, int64_t n, 
                                        const double* radius, const double* ro_sol,
                                        const int32_t* phase, int64_t ld) {
   if (!h || h->nsys < 2 || s < 0 || s >= h->nsys || !pos || !radius || !ro_sol) return MFIXDEM_ERR_ARG;
-  const int off = h->sys_off[s], cap = h->sys_off[s + 1] - off;
+  const int off = h->sys_off[s], cap = h->sys_cap[s];
   if (n < 0 || n > cap || ld < n) return MFIXDEM_ERR_ARG;
   const size_t S = h->stride;
   for (int64_t q = 0; q < n; q++) {
@@ -2338,9 +2314,9 @@ int32_t mfixdem_ensemble_set_particles(mfixdem_handle* h, int32_t s, int64_t n, 
 int32_t mfixdem_ensemble_get_particles(mfixdem_handle* h, int32_t s, double* pos, double* vel,
                                        double* omega, int8_t* state, int64_t ld) {
   if (!h || h->nsys < 2 || s < 0 || s >= h->nsys) return MFIXDEM_ERR_ARG;
-  const int off = h->sys_off[s], cap = h->sys_off[s + 1] - off;
+  const int off = h->sys_off[s], cap = h->sys_cap[s];
   if (ld < cap) return MFIXDEM_ERR_ARG;
-  return export_particles(h, off, cap, pos, vel, omega, state, ld);
+  return export_particles(h, off, h->sys_off[s + 1] - off, cap, pos, vel, omega, state, ld);
 }
 
 int32_t mfixdem_set_tuning(mfixdem_handle* h, double cell_scale, int32_t row_kernel) {
@@ -2353,18 +2329,15 @@ int32_t mfixdem_set_tuning(mfixdem_handle* h, double cell_scale, int32_t row_ker
     GridDev G = h->G;
     if (search_grid(h->S.p, h->n, G, n_fine, cell_scale) != MFIXDEM_OK)
       return MFIXDEM_ERR_UNSUPPORTED;
-    G.mbits = h->G.mbits;  // the key layout stays (a coarser grid needs fewer bits)
     h->G = G;
   } else {
     std::vector<GridDev> gt = h->sys_grid;
     std::vector<int> off(h->nsys + 1, 0);
     for (int s = 0; s < h->nsys; s++) {
       int nf = 0;
-      const int gb = gt[s].mbits;
       if (search_grid(h->sys_setup[s].p, h->sys_setup[s].p.max_pip, gt[s], nf, cell_scale) !=
           MFIXDEM_OK)
         return MFIXDEM_ERR_UNSUPPORTED;
-      gt[s].mbits = gb;
       off[s + 1] = off[s] + nf;
     }
     n_fine = off[h->nsys];
