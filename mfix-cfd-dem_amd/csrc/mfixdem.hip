@@ -867,7 +867,7 @@ int32_t deposit_current(mfixdem_handle* h) {
     hipLaunchKernelGGL(k_deposit_filter, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, P,
                        nullptr, h->pos[h->cur], h->pvol[h->tw], h->phase[h->tw],
                        h->state[h->tw], h->fcell[h->tw], h->xe, h->yn, h->zt, h->csz,
-                       h->fluid, h->rops_fix[h->fb], rm);
+                       h->rops_fix[h->fb], rm);
     HIPOK(hipGetLastError());
     return do_cell_fields(h, true);
   }
