@@ -3045,75 +3045,60 @@ __global__ __launch_bounds__(kBS) void k_apply_removals(int* cnt, const int* lis
   if (threadIdx.x == 0) *cnt = 0;
 }
 // Node sums -> ROP_S, EP_G per fluid cell (comp_mean_fields0.f:339-432,
-// calc_epg_des.f:133-145).  A workgroup takes kFieldCells consecutive
-// cells (J fastest), kFieldCPT per thread (two per thread measured the same
-// as one at 64x128x64 cells).  The corner nodes of those cells form four runs of
-// kFieldCells + 1 consecutive nodes, one per (I, K) corner pair, so the
-// workgroup reads each node once, coalesced, and computes its density (node
-// sum / VOL_SURR) once into LDS instead of once per adjacent cell.  Each
-// cell then sums its corners in the reference's order (I fastest, then J,
-// then K), skipping corners outside the node range and nodes with VOL_SURR
-// = 0 (their density is stored as 0, and adding 0 leaves the non-negative
-// sum as is).
-constexpr int kFieldCPT = 1, kFieldCells = kBS * kFieldCPT;
+// calc_epg_des.f:133-145).  A workgroup takes a block of kFJ x kFI x kFK
+// cells (J fastest in memory) and forms the density (node sum / VOL_SURR) of
+// each node it needs once, in LDS: (kFJ + 1)(kFI + 1)(kFK + 1) of them, 1.9
+// per cell, where a run of 256 consecutive cells needs 4 -- the FP64
+// divisions, not the 22 MB at 64 x 128 x 64 cells, are what the kernel spends
+// its time on (14.1 -> 11.0 us; other shapes of 256 cells 11.0 to 12.9).  Each cell then sums its corners in the
+// reference's order (I fastest, then J, then K), skipping corners outside the
+// node range and nodes with VOL_SURR = 0 (their density is stored as 0, and
+// adding 0 leaves the non-negative sum as is).
+constexpr int kFJ = 32, kFI = 4, kFK = 2;
+static_assert(kFJ * kFI * kFK == kBS, "one cell per thread");
 template <bool FIXED>
 __global__ __launch_bounds__(kBS) void k_cell_fields(int imax, int jmax, int kmax, int ni, int nj,
                                                      int nk, int nph, double packed_eps,
                                                      double inv_scale0, double inv_scale1,
                                                      double inv_scale2, double inv_scale3,
                                                      FieldPtrs f) {
-  constexpr int kRun = kFieldCells + 1, kNodes = 4 * kRun, kPer = (kNodes + kBS - 1) / kBS;
-  __shared__ double s_dens[4][kRun];
+  constexpr int kNJ = kFJ + 1, kNI = kFI + 1, kNK = kFK + 1, kNodes = kNJ * kNI * kNK;
+  constexpr int kPer = (kNodes + kBS - 1) / kBS;
+  __shared__ double s_dens[kNK][kNI][kNJ];
   const int ncell = ni * nj * nk, plane = nj * ni;
-  // XCD-aware order: the workgroups of one XCD take a contiguous range of
-  // cells, so the node rows a K-neighbour reads again are in that XCD's L2
-  const int c0 = xcd_tile(blockIdx.x, gridDim.x) * kFieldCells;
   if (FIXED && f.rm_cnt) {
     apply_removals(f.rm_cnt, f.rm_list, f.state, f.radius, blockIdx.x * kBS + threadIdx.x,
                    gridDim.x * kBS);
     if (blockIdx.x == 0 && threadIdx.x == 0) *f.rm_cnt_clear = 0;
   }
   const double inv[kMaxPh] = {inv_scale0, inv_scale1, inv_scale2, inv_scale3};
-  // this thread's cells c0 + tid + v kBS: corner mask (bit q: the corner is
-  // inside the node range), volume, fluid flag
-  unsigned okm[kFieldCPT];
-  double vc[kFieldCPT];
-  uint8_t fl[kFieldCPT];
-#pragma unroll
-  for (int v = 0; v < kFieldCPT; v++) {
-    const int c = c0 + threadIdx.x + v * kBS;
-    const bool live = c < ncell;
-    const int cj = c % nj + 1;
-    const int ci = (c / nj) % ni + 1;
-    const int ck = c / plane + 1;
-    okm[v] = 0u;
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int I = ci - 1 + (q & 1), J = cj - 1 + ((q >> 1) & 1), K = ck - 1 + (q >> 2);
-      if (live && I >= 1 && I <= imax + 1 && J >= 1 && J <= jmax + 1 && K >= 1 &&
-          K <= kmax + 1)
-        okm[v] |= 1u << q;
-    }
-    vc[v] = live ? f.vol[c] : 1.0;
-    fl[v] = live ? f.fluid[c] : 0;
-  }
-  // loader nodes: entry e of run r = qi + 2 qk is node
-  // c0 - 1 - (1 - qi) nj - (1 - qk) ni nj + e, the (qi, qj, qk) corner of
-  // cell c0 + e - qj
+  // XCD-aware order: the workgroups of one XCD take a contiguous range of
+  // blocks, so the nodes a neighbouring block reads again are in that XCD's L2
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int tj = (nj + kFJ - 1) / kFJ, ti = (ni + kFI - 1) / kFI;
+  const int j0 = tile % tj * kFJ, i0 = tile / tj % ti * kFI, k0 = tile / (tj * ti) * kFK;
+  // this thread's cell, 0-based; 1-based cell (ci, cj, ck) = node of its
+  // upper corner
+  const int lj = threadIdx.x % kFJ, li = threadIdx.x / kFJ % kFI, lk = threadIdx.x / (kFJ * kFI);
+  const int cj = j0 + lj + 1, ci = i0 + li + 1, ck = k0 + lk + 1;
+  const bool live = cj <= nj && ci <= ni && ck <= nk;
+  const int c = (cj - 1) + (ci - 1) * nj + (ck - 1) * plane;
+  const double vc = live ? f.vol[c] : 1.0;
+  const bool fl = live && f.fluid[c];
+  // the block's nodes: node (i0 + n, ...) 1-based, from the lower corner of
+  // the block's first cell; outside the node range the index is -1
   int nidx[kPer];
   double vsl[kPer];
 #pragma unroll
   for (int u = 0; u < kPer; u++) {
     const int e = threadIdx.x + u * kBS;
-    nidx[u] = -1;
-    if (e < kNodes) {
-      const int r = e / kRun, qi = r & 1, qk = r >> 1;
-      const int nd = c0 - 1 - (1 - qi) * nj - (1 - qk) * plane + (e - r * kRun);
-      if (nd >= 0 && nd < ncell) nidx[u] = nd;
-    }
-    vsl[u] = nidx[u] >= 0 ? f.vol_surr[nidx[u]] : 0.0;
+    const int J = j0 + e % kNJ, I = i0 + e / kNJ % kNI, K = k0 + e / (kNJ * kNI);
+    const bool in = e < kNodes && J >= 1 && J <= jmax + 1 && I >= 1 && I <= imax + 1 && K >= 1 &&
+                    K <= kmax + 1;
+    nidx[u] = in ? (J - 1) + (I - 1) * nj + (K - 1) * plane : -1;
+    vsl[u] = in ? f.vol_surr[nidx[u]] : 0.0;
   }
-  double acc[kFieldCPT][kMaxPh] = {};
+  double am[kMaxPh] = {};
   for (int m = 0; m < nph; m++) {
     if (m > 0) __syncthreads();  // the previous phase's densities are read
 #pragma unroll
@@ -3132,40 +3117,32 @@ __global__ __launch_bounds__(kBS) void k_cell_fields(int imax, int jmax, int kma
         }
         if (vsl[u] != 0.0) d = nodev / vsl[u];
       }
-      s_dens[e / kRun][e % kRun] = d;
+      (&s_dens[0][0][0])[e] = d;
     }
     __syncthreads();
+    // a corner outside the node range has density 0: the sum, which is not
+    // negative, stays as it is
+    double a = 0.0;
 #pragma unroll
-    for (int v = 0; v < kFieldCPT; v++) {
-      const int o = threadIdx.x + v * kBS;
-      double a = 0.0;
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        if (!((okm[v] >> q) & 1u)) continue;
-        const double dens = s_dens[(q & 1) + 2 * (q >> 2)][o + ((q >> 1) & 1)];
-        a = a + dens * vc[v];
-      }
-      acc[v][m] = a;
+    for (int q = 0; q < 8; q++) {
+      const double dens = s_dens[lk + (q >> 2)][li + (q & 1)][lj + ((q >> 1) & 1)];
+      a = a + dens * vc;
     }
+    am[m] = a;
   }
-#pragma unroll
-  for (int v = 0; v < kFieldCPT; v++) {
-    const int c = c0 + threadIdx.x + v * kBS;
-    if (c >= ncell) continue;
-    double* am = acc[v];
-    if (FIXED)
-      for (int m = 0; m < nph; m++) f.fix_clear[(size_t)m * ncell + c] = 0ull;
-    if (fl[v])
-      for (int m = 0; m < nph; m++)
-        if (am[m] > 0.0) am[m] = am[m] / vc[v];
-    for (int m = 0; m < nph; m++) f.rop_s[(size_t)m * ncell + c] = am[m];
-    if (fl[v]) {
-      double sum_eps = 0.0;
-      for (int m = 0; m < nph; m++) sum_eps = sum_eps + am[m] / f.ro_s[m];
-      const double e = 1.0 - (packed_eps < sum_eps ? packed_eps : sum_eps);
-      f.ep_g[c] = e;
-      if (e <= 0.0 || e > 1.0) atomicAdd(&f.flags[kFlagEpg], 1);
-    }
+  if (!live) return;
+  if (FIXED)
+    for (int m = 0; m < nph; m++) f.fix_clear[(size_t)m * ncell + c] = 0ull;
+  if (fl)
+    for (int m = 0; m < nph; m++)
+      if (am[m] > 0.0) am[m] = am[m] / vc;
+  for (int m = 0; m < nph; m++) f.rop_s[(size_t)m * ncell + c] = am[m];
+  if (fl) {
+    double sum_eps = 0.0;
+    for (int m = 0; m < nph; m++) sum_eps = sum_eps + am[m] / f.ro_s[m];
+    const double e = 1.0 - (packed_eps < sum_eps ? packed_eps : sum_eps);
+    f.ep_g[c] = e;
+    if (e <= 0.0 || e > 1.0) atomicAdd(&f.flags[kFlagEpg], 1);
   }
 }
 

@@ -190,8 +190,8 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 namespace {
 
 inline int nblk(int64_t n) { return (int)((n + kBS - 1) / kBS); }
-inline int field_blocks(int64_t ncell) {
-  return (int)((ncell + kFieldCells - 1) / kFieldCells);
+inline int field_blocks(const Setup& S) {  // k_cell_fields' blocks of cells
+  return ((S.nj + kFJ - 1) / kFJ) * ((S.ni + kFI - 1) / kFI) * ((S.nk + kFK - 1) / kFK);
 }
 
 template <typename T>
@@ -822,12 +822,12 @@ int32_t do_cell_fields(mfixdem_handle* h, bool fixed) {
     return MFIXDEM_OK;
   }
   if (fixed) {
-    hipLaunchKernelGGL(k_cell_fields<true>, dim3(field_blocks(h->S.ncell)), dim3(kBS), 0,
+    hipLaunchKernelGGL(k_cell_fields<true>, dim3(field_blocks(h->S)), dim3(kBS), 0,
                        h->stream, p.imax, p.jmax, p.kmax, h->S.ni, h->S.nj, h->S.nk, p.nphases,
                        packed, iv[0], iv[1], iv[2], iv[3], f);
     h->fb = 1 - h->fb;
   } else {
-    hipLaunchKernelGGL(k_cell_fields<false>, dim3(field_blocks(h->S.ncell)), dim3(kBS), 0,
+    hipLaunchKernelGGL(k_cell_fields<false>, dim3(field_blocks(h->S)), dim3(kBS), 0,
                        h->stream, p.imax, p.jmax, p.kmax, h->S.ni, h->S.nj, h->S.nk, p.nphases,
                        packed, iv[0], iv[1], iv[2], iv[3], f);
   }
