@@ -350,9 +350,7 @@ inline int32_t plan_seeds(const Setup& S, DemBoundaries& D) {
       for (int c = 0; c < 3; c++) sd.vel[c] = B.vel[m][c];
       const double r = d * 0.5;
       sd.radius = r;
-      sd.pvol = (4.0 / 3.0) * kPi * (r * r * r);
-      sd.pmass = sd.pvol * p.ro_s0[m];
-      sd.omoi = 2.5 / (sd.pmass * (r * r));
+      sd.pmass = (4.0 / 3.0) * kPi * (r * r * r) * p.ro_s0[m];
       sd.phase = m;
       sd.fcell = pack_ijk(ijk[0], ijk[1], ijk[2]);
       int c3[3];

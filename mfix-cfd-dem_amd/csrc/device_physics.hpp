@@ -20,6 +20,7 @@ constexpr int kWallSlots = 8;
 constexpr double kSmall = 1.0e-15;   // SMALL_NUMBER, param1_mod.f:26
 constexpr double kLarge = 1.0e32;    // LARGE_NUMBER, param1_mod.f:25
 constexpr double kUndefD = 9.87654321e31;
+constexpr double kPiD = 3.14159265358979323846;  // PI as the host set-up has it
 
 struct FacetDev {
   double v[3][3];
@@ -62,6 +63,16 @@ struct DevParams {
   // DEM mass inlets / outlets (StepPtrs::bcs): 0 when the run has none
   int nbc;
 };
+
+// PVOL and OMOI of a sphere (make_arrays_des.f:288-291), formed where they
+// are used: three multiplications and a division cost less than 16 bytes a
+// particle and step from memory.
+__device__ __forceinline__ double sphere_volume(double r) {
+  return (4.0 / 3.0) * kPiD * (r * r * r);
+}
+__device__ __forceinline__ double sphere_omoi(double mass, double r) {
+  return 2.5 / (mass * (r * r));
+}
 
 __device__ __forceinline__ double dot3(const double a[3], const double b[3]) {
   return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];

@@ -3,7 +3,7 @@
 // Layout in HBM (all per-particle arrays in the current Morton order of the
 // neighbour-search grid; component c of particle i at [c*stride + i]):
 //   pos/vel/omega      double, double-buffered (read one, write the other)
-//   radius/pmass/omoi/pvol, gid, state, phase, dgc (DES cell), fcell (fluid
+//   radius/pmass, gid, state, phase, dgc (DES cell), fcell (fluid
 //   cell), wall mask + per-facet wall history, AB2 accelerations
 //   neighbour rows     full rows: [incoming (owner has lower id) | own]
 //                      nbr_start[i] .. nbr_split[i] .. nbr_start[i+1]
@@ -56,14 +56,14 @@ __device__ __forceinline__ double bc_dist(const BcDev& b, const double x[3]) {
 // 419-642), formed on the host; slot_of_gid places it.
 struct SeedDev {
   double pos[3], vel[3];
-  double radius, pvol, pmass, omoi;
+  double radius, pmass;
   int gid, dgc, fcell, phase;
 };
 
 struct StepPtrs {
   const double *pos, *vel, *omega;
   double *pos_o, *vel_o, *omega_o;
-  const double *radius, *pmass, *omoi, *pvol;
+  const double *radius, *pmass;
   const int* gid;
   uint8_t* state;
   const uint8_t* phase;
@@ -335,7 +335,7 @@ __device__ __forceinline__ void add_drag_des1(const DevParams& P, const StepPtrs
   }
   if (lepg < 1.0e-6) lepg = a.ep_g[c0];
   if (!fluid_at(P, ci, cj, ck)) return;
-  const double pvol = a.pvol[i];
+  const double pvol = sphere_volume(a.radius[i]);
   if (!MIXED) {
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
@@ -388,7 +388,7 @@ __device__ __forceinline__ void add_drag(const DevParams& P, const StepPtrs& a, 
         const double* vn = a.vnode + 3 * (base + jj + ii * P.nj + kk * P.nj * P.ni);
         for (int d = 0; d < 3; d++) velfp[d] = velfp[d] + vn[d] * w;
       }
-  const double pvol = a.pvol[i];
+  const double pvol = sphere_volume(a.radius[i]);
   if (!MIXED) {
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
@@ -910,7 +910,7 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
 
   // ---- CFNEWVALUES (cfnewvalues.f:700-811)
   const double dt = P.dt;
-  const double omoi = a.omoi[i];
+  const double omoi = sphere_omoi(mi, a.radius[i]);
   if (!P.ab2) {
     // entering and exiting particles move at their velocity (:492, :593)
     const bool normal = st == kNormal;
@@ -1029,7 +1029,7 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
       double pv = 0.0;
       if (kEarlyDrag && P.coupled) {
         pc = a.fcell[i];
-        pv = a.pvol[i];
+        pv = sphere_volume(ri);
       }
       // ---- walls (calc_collision_wall_mod.f:184-606), the cell's facets in
       // ascending id
@@ -1316,7 +1316,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* li
 // order (list null) or list order; the workgroup's cells are summed in an LDS tile over
 // the bounding box of its targets (up to kDepCap cells), else directly.
 __global__ __launch_bounds__(kBS) void k_deposit_filter(DevParams P, const int* list,
-                                                        const double* pos, const double* pvol,
+                                                        const double* pos, const double* radius,
                                                         const uint8_t* phase, const uint8_t* state,
                                                         const int* fcell, const double* xe,
                                                         const double* yn, const double* zt,
@@ -1369,7 +1369,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_filter(DevParams P, const int* 
   __syncthreads();
   if (pc >= 0) {
     const int ph = phase[i];
-    const double vol_wt = pvol[i];
+    const double vol_wt = sphere_volume(radius[i]);
     const double sc = P.dep_scale[ph];
     unsigned long long* f = fix + (size_t)ph * P.ncell;
     auto add = [&](int I, int J, int K, double w) {
@@ -1746,8 +1746,8 @@ struct PermPtrs {
   const int* perm;
   const double *pos, *vel, *omega;
   double *pos_o, *vel_o, *omega_o;
-  const double *radius, *pmass, *omoi, *pvol, *acc, *racc;
-  double *radius_o, *pmass_o, *omoi_o, *pvol_o, *acc_o, *racc_o;
+  const double *radius, *pmass, *acc, *racc;
+  double *radius_o, *pmass_o, *acc_o, *racc_o;
   const int *gid, *fcell, *dgc;
   int *gid_o, *fcell_o, *dgc_o;
   const uint8_t *state, *phase, *wmask;
@@ -1770,8 +1770,6 @@ __global__ __launch_bounds__(kBS) void k_permute(int n, int S, PermPtrs p) {
   }
   p.radius_o[i] = p.radius[o];
   p.pmass_o[i] = p.pmass[o];
-  p.omoi_o[i] = p.omoi[o];
-  p.pvol_o[i] = p.pvol[o];
   p.gid_o[i] = p.gid[o];
   p.fcell_o[i] = p.fcell[o];
   p.dgc_o[i] = p.dgc[o];
@@ -2483,7 +2481,7 @@ __global__ __launch_bounds__(kBS) void k_delete_rogue(int n, int S, GridDev G0, 
 
 // ------------------------------------------------- DEM inlets / outlets
 struct BcPtrs {
-  double *pos, *vel, *omega, *radius, *pmass, *omoi, *pvol;
+  double *pos, *vel, *omega, *radius, *pmass;
   const int *gid, *dgc;
   uint8_t *state, *wmask;
   const uint8_t* phase;
@@ -2553,8 +2551,6 @@ __global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
     store3(b.omega, S, i, z);
     b.radius[i] = 0.0;
     b.pmass[i] = 3.4028234663852886e38;  // HUGE(0.0) as DELETE_PARTICLE sets it
-    b.pvol[i] = 3.4028234663852886e38;
-    b.omoi[i] = 0.0;
     b.wmask[i] = 0;
     b.state[i] = kNonexistent;
     b.del_list[atomicAdd(b.del_cnt, 1)] = b.gid[i];
@@ -2565,7 +2561,7 @@ __global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
 }
 
 struct SeedPtrs {
-  double *pos, *vel, *omega, *radius, *pmass, *omoi, *pvol;
+  double *pos, *vel, *omega, *radius, *pmass;
   int *dgc, *fcell;
   uint8_t *state, *phase, *wmask;
   const int* slot_of_gid;
@@ -2583,9 +2579,7 @@ __global__ __launch_bounds__(kBS) void k_seed(int ns, const SeedDev* sd, SeedPtr
   store3(p.vel, S, i, d.vel);
   store3(p.omega, S, i, z);
   p.radius[i] = d.radius;
-  p.pvol[i] = d.pvol;
   p.pmass[i] = d.pmass;
-  p.omoi[i] = d.omoi;
   p.dgc[i] = d.dgc;
   p.fcell[i] = d.fcell;
   p.phase[i] = (uint8_t)d.phase;
@@ -2760,7 +2754,7 @@ __global__ __launch_bounds__(kBS) void k_gas_fgp(DevParams P, StepPtrs a, double
       const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
       const double vrel = sqrt(dot3(vs, vs));
       const double f = drag_fgp_fp64(P.drag_type, a.ep_g[c], P.mu_g0, P.ro_g0, vrel,
-                                     2.0 * a.radius[i], a.pvol[i]);
+                                     2.0 * a.radius[i], sphere_volume(a.radius[i]));
       r[0] = zx;
       r[1] = zy;
       r[2] = zz;
@@ -2884,7 +2878,7 @@ __global__ __launch_bounds__(kBS) void k_gas_filter(DevParams P, StepPtrs a, con
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
     const double f = drag_fgp_fp64(P.drag_type, lepg, P.mu_g0, P.ro_g0, vrel, 2.0 * a.radius[i],
-                                   a.pvol[i]);
+                                   sphere_volume(a.radius[i]));
     if (a.f_gp) a.f_gp[a.gid[i]] = f;  // F_GP(NP) for explicit coupling
     const double lbm[3] = {f * vel[0], f * vel[1], f * vel[2]};
     auto add = [&](int I, int J, int K, double w) {
@@ -2949,7 +2943,7 @@ __global__ __launch_bounds__(kBS) void k_drag_fc(DevParams P, StepPtrs a) {
     for (int d = 0; d < 3; d++) velfp[d] = a.ugc[3 * c0 + d];
     for (int d = 0; d < 3; d++) lpf[d] = a.p_force[3 * c0 + d];
   }
-  const double f = a.f_gp[g], pv = a.pvol[i];
+  const double f = a.f_gp[g], pv = sphere_volume(a.radius[i]);
   double out[3];
   for (int d = 0; d < 3; d++) out[d] = f * (velfp[d] - vel[d]);
   for (int d = 0; d < 3; d++) out[d] = out[d] + lpf[d] * pv;

@@ -77,7 +77,7 @@ struct mfixdem_handle {
   // particles (cur / tw twins)
   double *pos[2]{}, *vel[2]{}, *omega[2]{};
   double* xr_pack = nullptr;  // (x, y, z, radius) per particle, written before each row build
-  double *radius[2]{}, *pmass[2]{}, *omoi[2]{}, *pvol[2]{};
+  double *radius[2]{}, *pmass[2]{};
   double *acc[2]{}, *racc[2]{};
   int *gid[2]{}, *fcell[2]{}, *dgc[2]{};
   uint8_t *state[2]{}, *phase[2]{}, *wmask[2]{};
@@ -264,7 +264,7 @@ StepPtrs step_ptrs(mfixdem_handle* h) {
   const int c = h->cur, t = h->tw, l = h->lt, p = h->pcur;
   a.pos = h->pos[c]; a.vel = h->vel[c]; a.omega = h->omega[c];
   a.pos_o = h->pos[1 - c]; a.vel_o = h->vel[1 - c]; a.omega_o = h->omega[1 - c];
-  a.radius = h->radius[t]; a.pmass = h->pmass[t]; a.omoi = h->omoi[t]; a.pvol = h->pvol[t];
+  a.radius = h->radius[t]; a.pmass = h->pmass[t];
   a.gid = h->gid[t]; a.state = h->state[t]; a.phase = h->phase[t]; a.dgc = h->dgc[t];
   a.cell_fmask = h->cell_fmask;
   a.fac = h->fac; a.dg_foff = h->dg_foff; a.dg_fids = h->dg_fids;
@@ -509,10 +509,10 @@ int32_t do_bin(mfixdem_handle* h) {
   p.perm = h->vals[1];
   p.pos = h->pos[c]; p.vel = h->vel[c]; p.omega = h->omega[c];
   p.pos_o = h->pos[1 - c]; p.vel_o = h->vel[1 - c]; p.omega_o = h->omega[1 - c];
-  p.radius = h->radius[t]; p.pmass = h->pmass[t]; p.omoi = h->omoi[t]; p.pvol = h->pvol[t];
+  p.radius = h->radius[t]; p.pmass = h->pmass[t];
   p.acc = h->acc[t]; p.racc = h->racc[t];
-  p.radius_o = h->radius[1 - t]; p.pmass_o = h->pmass[1 - t]; p.omoi_o = h->omoi[1 - t];
-  p.pvol_o = h->pvol[1 - t]; p.acc_o = h->acc[1 - t]; p.racc_o = h->racc[1 - t];
+  p.radius_o = h->radius[1 - t]; p.pmass_o = h->pmass[1 - t];
+  p.acc_o = h->acc[1 - t]; p.racc_o = h->racc[1 - t];
   p.gid = h->gid[t]; p.fcell = h->fcell[t]; p.dgc = h->dgc[t];
   p.gid_o = h->gid[1 - t]; p.fcell_o = h->fcell[1 - t]; p.dgc_o = h->dgc[1 - t];
   p.state = h->state[t]; p.phase = h->phase[t]; p.wmask = h->wmask[t];
@@ -865,7 +865,7 @@ int32_t deposit_current(mfixdem_handle* h) {
                    h->flags};
   if (h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012) {
     hipLaunchKernelGGL(k_deposit_filter, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, P,
-                       nullptr, h->pos[h->cur], h->pvol[h->tw], h->phase[h->tw],
+                       nullptr, h->pos[h->cur], h->radius[h->tw], h->phase[h->tw],
                        h->state[h->tw], h->fcell[h->tw], h->xe, h->yn, h->zt, h->csz,
                        h->rops_fix[h->fb], rm);
     HIPOK(hipGetLastError());
@@ -926,7 +926,7 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
   CHECKRC(fill_i32(h->stream, h->del_cnt, 1, 0));
   BcPtrs b{};
   b.pos = h->pos[c]; b.vel = h->vel[c]; b.omega = h->omega[c];
-  b.radius = h->radius[t]; b.pmass = h->pmass[t]; b.omoi = h->omoi[t]; b.pvol = h->pvol[t];
+  b.radius = h->radius[t]; b.pmass = h->pmass[t];
   b.gid = h->gid[t]; b.dgc = h->dgc[t]; b.state = h->state[t]; b.wmask = h->wmask[t];
   b.phase = h->phase[t];
   b.bcs = h->d_bcs; b.nbc = (int)D.b.size(); b.n = n; b.S = h->stride;
@@ -940,8 +940,8 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
                          hipMemcpyHostToDevice, h->stream));
     SeedPtrs sp{};
     sp.pos = h->pos[c]; sp.vel = h->vel[c]; sp.omega = h->omega[c];
-    sp.radius = h->radius[t]; sp.pmass = h->pmass[t]; sp.omoi = h->omoi[t];
-    sp.pvol = h->pvol[t]; sp.dgc = h->dgc[t]; sp.fcell = h->fcell[t];
+    sp.radius = h->radius[t]; sp.pmass = h->pmass[t];
+    sp.dgc = h->dgc[t]; sp.fcell = h->fcell[t];
     sp.state = h->state[t]; sp.phase = h->phase[t]; sp.wmask = h->wmask[t];
     sp.slot_of_gid = h->slot_of_gid; sp.S = h->stride;
     hipLaunchKernelGGL(k_seed, dim3(nblk(ns)), dim3(kBS), 0, h->stream, ns, h->d_seeds, sp);
@@ -1177,12 +1177,11 @@ int32_t upload_setup(mfixdem_handle* h) {
 }
 
 // Upload an ensemble's staged particles: per system, ids 0..capacity-1 in
-// slot order, PVOL/PMASS/OMOI as make_arrays_des.f:288-291, NORMAL for the
+// slot order, PMASS as make_arrays_des.f:288-291, NORMAL for the
 // particles set, NONEXISTENT for the rest of the system's slots.
 int32_t upload_ensemble(mfixdem_handle* h) {
   const int64_t N = h->n, S = h->stride;
-  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38), OI(S, 0.0),
-      PV(S, 3.4028234663852886e38);
+  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38);
   std::vector<int> G(S, 0), FC(S, -1), DG(S, 0);
   std::vector<uint8_t> ST(S, 0), PH(S, 0), WM(S, 0);
   for (int s = 0; s < h->nsys; s++) {
@@ -1191,9 +1190,7 @@ int32_t upload_ensemble(mfixdem_handle* h) {
     for (int q = off; q < off + h->sys_n[s]; q++) {
       const double r = h->st_r[q];
       R[q] = r;
-      PV[q] = (4.0 / 3.0) * kPi * (r * r * r);
-      M[q] = PV[q] * h->st_rho[q];
-      OI[q] = 2.5 / (M[q] * (r * r));
+      M[q] = (4.0 / 3.0) * kPi * (r * r * r) * h->st_rho[q];
       PH[q] = (uint8_t)(h->st_phase[q] - 1);
       ST[q] = 1;
     }
@@ -1205,8 +1202,6 @@ int32_t upload_ensemble(mfixdem_handle* h) {
   HIPOK(hipMemcpy(h->omega[0], h->st_om.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->radius[0], R.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->pmass[0], M.data(), sizeof(double) * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->omoi[0], OI.data(), sizeof(double) * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->pvol[0], PV.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->gid[0], G.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->fcell[0], FC.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->dgc[0], DG.data(), sizeof(int) * S, hipMemcpyHostToDevice));
@@ -1238,7 +1233,7 @@ template <class F>
 void for_each_buffer(mfixdem_handle* h, F f) {
   for (int b = 0; b < 2; b++) {
     f(h->pos[b]); f(h->vel[b]); f(h->omega[b]); f(h->radius[b]);
-    f(h->pmass[b]); f(h->omoi[b]); f(h->pvol[b]); f(h->acc[b]);
+    f(h->pmass[b]); f(h->acc[b]);
     f(h->racc[b]); f(h->gid[b]); f(h->fcell[b]); f(h->dgc[b]);
     f(h->state[b]); f(h->phase[b]); f(h->wmask[b]); f(h->wfid[b]); f(h->wpft[b]);
     f(h->vals[b]); f(h->nbr_start[b]); f(h->nbr_split[b]);
@@ -1322,8 +1317,7 @@ int32_t alloc_buffers(mfixdem_handle* h) {
   for (int b = 0; b < 2; b++) {
     if ((rc = dalloc(&h->pos[b], 3 * S)) || (rc = dalloc(&h->vel[b], 3 * S)) ||
         (rc = dalloc(&h->omega[b], 3 * S)) || (rc = dalloc(&h->radius[b], S)) ||
-        (rc = dalloc(&h->pmass[b], S)) || (rc = dalloc(&h->omoi[b], S)) ||
-        (rc = dalloc(&h->pvol[b], S)) || (rc = dalloc(&h->acc[b], 3 * S)) ||
+        (rc = dalloc(&h->pmass[b], S)) || (rc = dalloc(&h->acc[b], 3 * S)) ||
         (rc = dalloc(&h->racc[b], 3 * S)) || (rc = dalloc(&h->gid[b], S)) ||
         (rc = dalloc(&h->fcell[b], S)) || (rc = dalloc(&h->dgc[b], S)) ||
         (rc = dalloc(&h->state[b], S)) || (rc = dalloc(&h->phase[b], S)) ||
@@ -1513,7 +1507,7 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
   if (!h || n < 0 || n > h->n || ld < n || !pos || !radius || !ro_sol) return MFIXDEM_ERR_ARG;
   const int64_t N = h->n, S = h->stride;
   std::vector<double> P3((size_t)3 * S, 0.0), V3((size_t)3 * S, 0.0), W3((size_t)3 * S, 0.0);
-  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38), OI(S, 0.0), PV(S, 3.4028234663852886e38);
+  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38);
   std::vector<int> G(S, 0), FC(S, -1), DG(S, 0);
   std::vector<uint8_t> ST(S, 0), PH(S, 0), WM(S, 0);
   for (int64_t q = 0; q < N; q++) G[q] = (int)q;
@@ -1526,9 +1520,7 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
     const double r = radius[q];
     R[q] = r;
     // make_arrays_des.f:288-291
-    PV[q] = (4.0 / 3.0) * kPi * (r * r * r);
-    M[q] = PV[q] * ro_sol[q];
-    OI[q] = 2.5 / (M[q] * (r * r));
+    M[q] = (4.0 / 3.0) * kPi * (r * r * r) * ro_sol[q];
     const int ph = phase ? phase[q] - 1 : 0;
     if (ph < 0 || ph >= h->S.p.nphases) return MFIXDEM_ERR_ARG;
     PH[q] = (uint8_t)ph;
@@ -1559,8 +1551,6 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
   HIPOK(hipMemcpy(h->omega[0], W3.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->radius[0], R.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->pmass[0], M.data(), sizeof(double) * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->omoi[0], OI.data(), sizeof(double) * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->pvol[0], PV.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->gid[0], G.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->fcell[0], FC.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->dgc[0], DG.data(), sizeof(int) * S, hipMemcpyHostToDevice));
