@@ -50,6 +50,7 @@ struct DevParams {
   double etan_w[kMaxPh], etat_w[kMaxPh], hkwn[kMaxPh], hkwt[kMaxPh];
   // fluid grid
   int ni, nj, nk, ncell;
+  double face_lo[3], face_hi[3], face_inv[3];  // outermost faces, 1 / first cell size
   double ro_g0, mu_g0;
   double dep_scale[kMaxPh];  // fixed-point scale of the deposition sums (power of 2)
   // filter schemes (DES_INTERP_SCHEME other than GARG_2012)
@@ -504,15 +505,28 @@ __device__ __forceinline__ float drag_fgp_fp32(int drag_type, float epg, float m
   return dga * pvol;
 }
 
-// Unique cell I with faces[I-1] <= x < faces[I], 1 <= I <= nmax; 0 if none
-// (PARTICLES_IN_CELL + PIC_SEARCH, particles_in_cell.f:87-154,347-370).
-__device__ __forceinline__ int locate_cell(const double* faces, int nmax, double inv_d, double x) {
-  if (!(x >= faces[0] && x < faces[nmax])) return 0;
-  int i = (int)((x - faces[0]) * inv_d) + 1;
+// Unique cell I with faces[I-1] <= x < faces[I], 1 <= I <= nmax, and its faces
+// x0, x1; 0 if none (PARTICLES_IN_CELL + PIC_SEARCH, particles_in_cell.f:
+// 87-154,347-370).  lo and hi are the outermost faces, inv_d one over the
+// first cell's size: the first guess, which the faces then correct.
+__device__ __forceinline__ int locate_cell(const double* faces, int nmax, double lo, double hi,
+                                           double inv_d, double x, double& x0, double& x1) {
+  if (!(x >= lo && x < hi)) return 0;
+  int i = (int)((x - lo) * inv_d) + 1;
   if (i < 1) i = 1;
   if (i > nmax) i = nmax;
-  while (i > 1 && x < faces[i - 1]) i--;
-  while (i < nmax && x >= faces[i]) i++;
+  x0 = faces[i - 1];
+  x1 = faces[i];
+  while (i > 1 && x < x0) {
+    i--;
+    x1 = x0;
+    x0 = faces[i - 1];
+  }
+  while (i < nmax && x >= x1) {
+    i++;
+    x0 = x1;
+    x1 = faces[i];
+  }
   return i;
 }
 

@@ -219,7 +219,8 @@ __device__ __forceinline__ double dpvm_w(const DevParams& P, double pos1, double
 __device__ __forceinline__ bool on_grid(const DevParams& P, int I, int J, int K) {
   return I >= 1 && I <= P.ni && J >= 1 && J <= P.nj && K >= 1 && K <= P.nk;
 }
-__device__ __forceinline__ bool fluid_at(const DevParams& P, int I, int J, int K) {
+template <class PT>
+__device__ __forceinline__ bool fluid_at(const PT& P, int I, int J, int K) {
   return I >= 2 && I < P.ni && J >= 2 && J < P.nj && K >= 2 && K < P.nk;
 }
 // one axis of CALC_INTERP_WEIGHTS2 (calc_interp_weights.f:365-460) in cell
@@ -367,7 +368,7 @@ __device__ __forceinline__ void add_drag(const DevParams& P, const StepPtrs& a, 
   int ci, cj, ck;
   unpack_ijk(pc, ci, cj, ck);
   const int c = lin_ijk(ci, cj, ck, P.ni, P.nj);
-  if (!a.fluid[c]) return;
+  if (!fluid_at(P, ci, cj, ck)) return;
   const double x0 = a.xe[ci - 1], y0 = a.yn[cj - 1], z0 = a.zt[ck - 1];
   const double dxx = a.xe[ci] - x0, dyy = a.yn[cj] - y0, dzz = a.zt[ck] - z0;
   double zx = pos[0] - x0, zy = pos[1] - y0;
@@ -423,7 +424,6 @@ __device__ __forceinline__ bool garg_drag_terms(const DevParams& P, const StepPt
   if (pc >= 0) unpack_ijk(pc, ci, cj, ck);
   const int c = lin_ijk(ci, cj, ck, P.ni, P.nj);
   const int qi = ci > 2 ? ci : 2, qj = cj > 2 ? cj : 2, qk = ck > 2 ? ck : 2;
-  const uint8_t fl = a.fluid[c];
   const double epg = a.ep_g[c];
   double pf[3];
   for (int d = 0; d < 3; d++) pf[d] = a.p_force[3 * c + d];
@@ -440,7 +440,7 @@ __device__ __forceinline__ bool garg_drag_terms(const DevParams& P, const StepPt
         const double* v = a.vnode + 3 * (base + jj + ii * P.nj + kk * P.nj * P.ni);
         for (int d = 0; d < 3; d++) vn[(kk * 2 + jj) * 2 + ii][d] = v[d];
       }
-  if (pc < 0 || !fl) return false;
+  if (pc < 0 || !fluid_at(P, ci, cj, ck)) return false;
   const double dxx = x1 - x0, dyy = y1 - y0, dzz = z1 - z0;
   double zx = pos[0] - x0, zy = pos[1] - y0;
   zx = zx / dxx;
@@ -531,11 +531,12 @@ constexpr unsigned kRowOwn = 64u;
 // pairs that are not are written here.
 __device__ __forceinline__ bool pair_touches(const StepPtrs& a, int S, const double xp[3],
                                              double rp, int j, int pid, bool owner) {
-  const uint8_t stj = a.state[j];
   double xj[3];
   load3(a.pos, S, j, xj);
   const double rj = a.radius[j];
-  if (stj == 0) {  // IF(IS_NONEXISTENT(I)) CYCLE: history kept
+  // IF(IS_NONEXISTENT(I)) CYCLE: history kept.  A nonexistent particle has
+  // radius 0 (set with its state), so the state is read only then.
+  if (rj == 0.0 && a.state[j] == 0) {
     if (owner) keep_history(a, pid);
     return false;
   }
@@ -718,14 +719,14 @@ __device__ __forceinline__ void wave_pairs(const DevParams& P0, const PT& P, con
   }
 }
 
-// Inputs of the fused deposition from one particle's step: its new
-// position, mass and phase and the fluid cell it is deposited into (-1:
-// none), or a removal (the particle left the fluid grid).
+// Inputs of the fused deposition from one particle's step: its mass and
+// phase, the fluid cell it is deposited into (-1: none) and its normalised
+// place there, or a removal (the particle left the fluid grid).
 struct DepIn {
   int pc = -1;
   int ph = 0;
   bool remove = false;
-  double x[3] = {0.0, 0.0, 0.0};
+  double z[3] = {0.0, 0.0, 0.0};
   double m = 0.0;
 };
 
@@ -743,7 +744,6 @@ struct DepIn {
 __device__ __forceinline__ void fused_deposit(const DevParams& P, const StepPtrs& a, int i,
                                               const DepIn& d, unsigned long long* tile,
                                               int cap) {
-  __shared__ int box[6];
   if (d.remove) {
     const int q = atomicAdd(a.rm_cnt, 1);
     a.rm_list[q] = i;
@@ -751,45 +751,46 @@ __device__ __forceinline__ void fused_deposit(const DevParams& P, const StepPtrs
   }
   int ci = 0, cj = 0, ck = 0;
   if (d.pc >= 0) unpack_ijk(d.pc, ci, cj, ck);
-  int lo0 = d.pc >= 0 ? ci : INT_MAX, lo1 = d.pc >= 0 ? cj : INT_MAX;
-  int lo2 = d.pc >= 0 ? ck : INT_MAX;
-  int hi0 = d.pc >= 0 ? ci : INT_MIN, hi1 = d.pc >= 0 ? cj : INT_MIN;
-  int hi2 = d.pc >= 0 ? ck : INT_MIN;
+  // the bounding box of the workgroup's cells: six minima (of ci, cj, ck and
+  // of 1023 less them) in three packed values, across the lanes and then the
+  // wavefronts
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  __shared__ u16x2 s_box[kBS / 64][3];
+  u16x2 m[3] = {{0xFFFF, 0xFFFF}, {0xFFFF, 0xFFFF}, {0xFFFF, 0xFFFF}};
+  if (d.pc >= 0) {
+    m[0] = u16x2{(unsigned short)ci, (unsigned short)cj};
+    m[1] = u16x2{(unsigned short)ck, (unsigned short)(1023 - ci)};
+    m[2] = u16x2{(unsigned short)(1023 - cj), (unsigned short)(1023 - ck)};
+  }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo0 = min(lo0, __shfl_xor(lo0, o, 64));
-    lo1 = min(lo1, __shfl_xor(lo1, o, 64));
-    lo2 = min(lo2, __shfl_xor(lo2, o, 64));
-    hi0 = max(hi0, __shfl_xor(hi0, o, 64));
-    hi1 = max(hi1, __shfl_xor(hi1, o, 64));
-    hi2 = max(hi2, __shfl_xor(hi2, o, 64));
-  }
-  if (threadIdx.x < 3) box[threadIdx.x] = INT_MAX;
-  else if (threadIdx.x < 6) box[threadIdx.x] = INT_MIN;
+  for (int o = 32; o > 0; o >>= 1)
+    for (int k = 0; k < 3; k++)
+      m[k] = __builtin_elementwise_min(
+          m[k], __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(int, m[k]), o, 64)));
+  if ((threadIdx.x & 63) == 0)
+    for (int k = 0; k < 3; k++) s_box[threadIdx.x >> 6][k] = m[k];
   __syncthreads();  // also: every lane is done with the LDS that tile aliases
-  if ((threadIdx.x & 63) == 0 && lo0 != INT_MAX) {
-    atomicMin(&box[0], lo0); atomicMin(&box[1], lo1); atomicMin(&box[2], lo2);
-    atomicMax(&box[3], hi0); atomicMax(&box[4], hi1); atomicMax(&box[5], hi2);
-  }
-  __syncthreads();
-  // tile nodes I in [bi-1, box_hi]: a cell I touches nodes I-1 and I
-  const int bi = box[0], bj = box[1], bk = box[2];
-  const int ti_n = box[3] - bi + 2, tj_n = box[4] - bj + 2, tk_n = box[5] - bk + 2;
-  const bool any = bi != INT_MAX;
+  for (int k = 0; k < 3; k++) m[k] = s_box[0][k];
+#pragma unroll
+  for (int w = 1; w < kBS / 64; w++)
+    for (int k = 0; k < 3; k++) m[k] = __builtin_elementwise_min(m[k], s_box[w][k]);
+  // tile nodes I in [bi-1, box_hi]: a cell I touches nodes I-1 and I; the box
+  // is the same in every lane
+  const int bi = __builtin_amdgcn_readfirstlane((int)m[0].x);
+  const int bj = __builtin_amdgcn_readfirstlane((int)m[0].y);
+  const int bk = __builtin_amdgcn_readfirstlane((int)m[1].x);
+  const bool any = bi != 0xFFFF;
+  const int ti_n = 1023 - __builtin_amdgcn_readfirstlane((int)m[1].y) - bi + 2;
+  const int tj_n = 1023 - __builtin_amdgcn_readfirstlane((int)m[2].x) - bj + 2;
+  const int tk_n = 1023 - __builtin_amdgcn_readfirstlane((int)m[2].y) - bk + 2;
   const int vol = any ? ti_n * tj_n * tk_n : 0;
   const bool tiled = any && P.nph == 1 && vol <= cap;
   if (tiled)
     for (int q = threadIdx.x; q < vol; q += kBS) tile[q] = 0ull;
   __syncthreads();
   if (d.pc >= 0) {
-    const double x0 = a.xe[ci - 1], y0 = a.yn[cj - 1], z0 = a.zt[ck - 1];
-    const double dxx = a.xe[ci] - x0, dyy = a.yn[cj] - y0, dzz = a.zt[ck] - z0;
-    double zx = d.x[0] - x0, zy = d.x[1] - y0;
-    zx = zx / dxx;
-    zy = zy / dyy;
-    double zz = d.x[2] - z0;
-    zz = zz / dzz;
-    const double xv[2] = {1.0 - zx, zx}, yv[2] = {1.0 - zy, zy}, zv[2] = {1.0 - zz, zz};
+    const double xv[2] = {1.0 - d.z[0], d.z[0]}, yv[2] = {1.0 - d.z[1], d.z[1]},
+                 zv[2] = {1.0 - d.z[2], d.z[2]};
     const double sc = P.dep_scale[d.ph];
     if (tiled) {
       const int tb = (ci - bi) + ti_n * ((cj - bj) + tj_n * (ck - bk));
@@ -946,11 +947,12 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
   }
 
   // ---- PARTICLES_IN_CELL locate, fused (particles_in_cell.f:87-154)
-  int pc = 0;
+  int pc = 0, I = 0, J = 0, K = 0;
+  double x0[3] = {0.0, 0.0, 0.0}, x1[3] = {1.0, 1.0, 1.0};
   if (MODE == kModeFused && P.coupled && !P.explicit_cpl) {
-    const int I = locate_cell(a.xe, P.ni, 1.0 / (a.xe[1] - a.xe[0]), pos[0]);
-    const int J = locate_cell(a.yn, P.nj, 1.0 / (a.yn[1] - a.yn[0]), pos[1]);
-    const int K = locate_cell(a.zt, P.nk, 1.0 / (a.zt[1] - a.zt[0]), pos[2]);
+    I = locate_cell(a.xe, P.ni, P.face_lo[0], P.face_hi[0], P.face_inv[0], pos[0], x0[0], x1[0]);
+    J = locate_cell(a.yn, P.nj, P.face_lo[1], P.face_hi[1], P.face_inv[1], pos[1], x0[1], x1[1]);
+    K = locate_cell(a.zt, P.nk, P.face_lo[2], P.face_hi[2], P.face_inv[2], pos[2], x0[2], x1[2]);
     pc = (I && J && K) ? pack_ijk(I, J, K) : -1;
     a.fcell[i] = pc;
   }
@@ -968,14 +970,13 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
   store3(a.pos_o, S, i, pos);
   store3(a.vel_o, S, i, vel);
   store3(a.omega_o, S, i, om);
-  if (kEarlyDrag && P0.fuse_dep) {
-    int I, J, K;
-    unpack_ijk(pc, I, J, K);
-    if (a.fluid[lin_ijk(I, J, K, P.ni, P.nj)]) {
-      dep.pc = pc;
-      dep.ph = a.phase[i];
-      dep.m = mi;
-      for (int c = 0; c < 3; c++) dep.x[c] = pos[c];
+  if (kEarlyDrag && P0.fuse_dep && fluid_at(P, I, J, K)) {
+    dep.pc = pc;
+    dep.ph = a.phase[i];
+    dep.m = mi;
+    for (int d = 0; d < 3; d++) {
+      const double w = x1[d] - x0[d], z = pos[d] - x0[d];
+      dep.z[d] = z / w;
     }
   }
 }
@@ -2594,20 +2595,30 @@ __global__ __launch_bounds__(kBS) void k_slot_of_gid(int n, const int* gid, int*
 }
 
 // ---------------------------------------------------------- gas coupling
-__global__ __launch_bounds__(kBS) void k_locate(int n, int S, int ni, int nj, int nk,
-                                                const double* xe, const double* yn,
-                                                const double* zt, const double* pos,
-                                                const uint8_t* state, int* fcell) {
+// The faces of the fluid grid: cells per axis, and DevParams' face_*.
+struct FaceGrid {
+  int n[3];
+  double lo[3], hi[3], inv[3];
+};
+// PARTICLES_IN_CELL locate; with kDelete the particles outside the fluid grid
+// are deleted as well (particles_in_cell.f:175-184).
+template <bool kDelete>
+__global__ __launch_bounds__(kBS) void k_locate(int n, int S, FaceGrid f, const double* xe,
+                                                const double* yn, const double* zt, int* fcell,
+                                                Removal rm) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
-  if (state[i] == 0) {
+  if (rm.state[i] == 0) {
     fcell[i] = -1;
     return;
   }
-  const int I = locate_cell(xe, ni, 1.0 / (xe[1] - xe[0]), pos[i]);
-  const int J = locate_cell(yn, nj, 1.0 / (yn[1] - yn[0]), pos[S + i]);
-  const int K = locate_cell(zt, nk, 1.0 / (zt[1] - zt[0]), pos[2 * S + i]);
-  fcell[i] = (I && J && K) ? pack_ijk(I, J, K) : -1;
+  double x0, x1;
+  const int I = locate_cell(xe, f.n[0], f.lo[0], f.hi[0], f.inv[0], rm.pos[i], x0, x1);
+  const int J = locate_cell(yn, f.n[1], f.lo[1], f.hi[1], f.inv[1], rm.pos[S + i], x0, x1);
+  const int K = locate_cell(zt, f.n[2], f.lo[2], f.hi[2], f.inv[2], rm.pos[2 * S + i], x0, x1);
+  const bool in = I && J && K;
+  fcell[i] = in ? pack_ijk(I, J, K) : -1;
+  if (kDelete && !in) remove_outside(rm, S, i);
 }
 
 // PIC counts; deletes particles outside the fluid grid (particles_in_cell.f:175-184)
@@ -3260,25 +3271,6 @@ __global__ __launch_bounds__(kBS) void k_pg_grad(int ni, int nj, int nk, const d
   f[0] = -g0;
   f[1] = -g1;
   f[2] = -g2;
-}
-
-// PARTICLES_IN_CELL deletion of particles outside the fluid grid
-// (particles_in_cell.f:175-184), for particles the fused step flagged
-__global__ __launch_bounds__(kBS) void k_delete_outside(int n, int S, const int* fcell,
-                                                        uint8_t* state, uint8_t* wmask,
-                                                        double* pos, double* vel, double* omega,
-                                                        double* radius, int* flags) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n || state[i] == 0 || fcell[i] >= 0) return;
-  state[i] = 0;
-  wmask[i] = 0;
-  for (int d = 0; d < 3; d++) {
-    pos[d * S + i] = 0.0;
-    vel[d * S + i] = 0.0;
-    omega[d * S + i] = 0.0;
-  }
-  radius[i] = 0.0;
-  atomicAdd(&flags[kFlagOutOfDomain], 1);
 }
 
 // ------------------------------------------------------------- exports

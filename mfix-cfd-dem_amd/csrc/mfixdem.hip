@@ -835,11 +835,25 @@ int32_t do_cell_fields(mfixdem_handle* h, bool fixed) {
   return MFIXDEM_OK;
 }
 
-int32_t delete_outside(mfixdem_handle* h) {
+Removal removal(mfixdem_handle* h) {
   const int t = h->tw, c = h->cur;
-  hipLaunchKernelGGL(k_delete_outside, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, h->n, h->stride,
-                     h->fcell[t], h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c],
-                     h->radius[t], h->flags);
+  return Removal{h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->radius[t],
+                 h->flags};
+}
+
+// the fluid cell of every particle, those outside the grid deleted or not
+int32_t do_locate(mfixdem_handle* h, bool remove) {
+  FaceGrid f{};
+  const int n[3] = {h->S.ni, h->S.nj, h->S.nk};
+  for (int d = 0; d < 3; d++) {
+    f.n[d] = n[d];
+    f.lo[d] = h->P.face_lo[d];
+    f.hi[d] = h->P.face_hi[d];
+    f.inv[d] = h->P.face_inv[d];
+  }
+  auto k = remove ? k_locate<true> : k_locate<false>;
+  hipLaunchKernelGGL(k, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, h->n, h->stride, f, h->xe,
+                     h->yn, h->zt, h->fcell[h->tw], removal(h));
   HIPOK(hipGetLastError());
   return MFIXDEM_OK;
 }
@@ -860,9 +874,7 @@ int32_t ref_mean_fields(mfixdem_handle* h) {
 // deposition of the current positions into the fixed-point accumulators
 int32_t deposit_current(mfixdem_handle* h) {
   DevParams P = h->P;
-  const int t = h->tw, c = h->cur;
-  const Removal rm{h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->radius[t],
-                   h->flags};
+  const Removal rm = removal(h);
   if (h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012) {
     hipLaunchKernelGGL(k_deposit_filter, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, P,
                        nullptr, h->pos[h->cur], h->radius[h->tw], h->phase[h->tw],
@@ -1746,15 +1758,9 @@ int32_t mfixdem_init(mfixdem_handle* h) {
   if (h->S.p.coupled && !h->gas_set) return MFIXDEM_ERR_NOT_READY;
   HIPOK(sync_stream(h));
   if (h->nsys > 1) CHECKRC(upload_ensemble(h));
-  const int n = h->n;
   HIPOK(hipMemsetAsync(h->flags, 0, sizeof(int) * kFlagCount, h->stream));
   h->flags_set = false;
-  if (h->S.p.coupled) {
-    hipLaunchKernelGGL(k_locate, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->stride, h->S.ni,
-                       h->S.nj, h->S.nk, h->xe, h->yn, h->zt, h->pos[h->cur], h->state[h->tw],
-                       h->fcell[h->tw]);
-    HIPOK(hipGetLastError());
-  }
+  if (h->S.p.coupled) CHECKRC(do_locate(h, false));
   CHECKRC(do_bin(h));
   CHECKRC(do_neighbour(h));
   if (h->P.nbc) CHECKRC(refresh_free_gids(h));
@@ -1829,13 +1835,9 @@ int32_t mfixdem_neighbour(mfixdem_handle* h) {
 int32_t mfixdem_particles_in_cell(mfixdem_handle* h) {
   if (!h || !h->inited) return h ? MFIXDEM_ERR_NOT_READY : MFIXDEM_ERR_ARG;
   h->xr_packed = false;  // particles may be removed: the walk's candidates are packed again
-  const int n = h->n;
-  hipLaunchKernelGGL(k_locate, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->stride, h->S.ni,
-                     h->S.nj, h->S.nk, h->xe, h->yn, h->zt, h->pos[h->cur], h->state[h->tw],
-                     h->fcell[h->tw]);
-  HIPOK(hipGetLastError());
-  if (ref_deposition(h)) return do_pic_lists(h);
-  return delete_outside(h);
+  const bool ref = ref_deposition(h);  // deletes in do_pic_lists
+  CHECKRC(do_locate(h, !ref));
+  return ref ? do_pic_lists(h) : MFIXDEM_OK;
 }
 // CALC_INTERP_WEIGHTS (calc_interp_weights.f:22-33): the filter weights are
 // evaluated inside the drag and deposition kernels from the current

@@ -69,6 +69,12 @@ inline void fill_params(const Setup& S, int n, int stride, DevParams& P, GridDev
     P.hkwt[a] = S.d.hert_kwt[a];
   }
   P.ni = S.ni; P.nj = S.nj; P.nk = S.nk; P.ncell = S.ncell;
+  const std::vector<double>* faces[3] = {&S.xe, &S.yn, &S.zt};
+  for (int d = 0; d < 3; d++) {
+    P.face_lo[d] = faces[d]->front();
+    P.face_hi[d] = faces[d]->back();
+    P.face_inv[d] = 1.0 / ((*faces[d])[1] - (*faces[d])[0]);
+  }
   P.ro_g0 = p.ro_g0; P.mu_g0 = p.mu_g0;
   P.interp = p.interp_scheme;
   P.interp_on = p.des_interp_on;
