@@ -125,6 +125,12 @@ struct mfixdem_handle {
   bool order_set = false;
   int* flags = nullptr;
   HostFlags* host_flags = nullptr;  // pinned host memory (wait_flags)
+  struct Block {  // one allocation shared by `live` buffers
+    char* base;
+    size_t bytes;
+    int live;
+  };
+  std::vector<Block> blocks;
   char* ring = nullptr;             // pinned chunks of read_back, on first use
   hipEvent_t ring_ev[4]{};
   int flags_seq = 0;
@@ -194,16 +200,73 @@ inline int field_blocks(const Setup& S) {  // k_cell_fields' blocks of cells
   return ((S.nj + kFJ - 1) / kFJ) * ((S.ni + kFI - 1) / kFI) * ((S.nk + kFK - 1) / kFK);
 }
 
-template <typename T>
-int32_t dalloc(T** p, int64_t count) {
-  *p = nullptr;
-  if (count <= 0) count = 1;
-  if (hipMalloc((void**)p, sizeof(T) * (size_t)count) != hipSuccess) return MFIXDEM_ERR_OOM;
-  return MFIXDEM_OK;
+// Device memory of a handle.  A hipMalloc costs 17 us and a hipFree, which
+// waits for the whole device, 90 us, so a handle of 2000 particles spent 1.7 ms
+// in each of mfixdem_create and mfixdem_destroy on its ~105 buffers, and held
+// up the streams of every other handle meanwhile.  Buffers that are made
+// together therefore share one allocation, which goes when the last of them
+// goes.  Buffers of more than kSharedMax have their own: they are freed by
+// themselves when they grow, and mapping their pages costs more than the call.
+constexpr size_t kSharedMax = 2u << 20;
+constexpr size_t kPieceAlign = 256;  // hipMalloc's own promise
+
+struct Pieces {
+  struct Want {
+    void** p;
+    size_t bytes;
+  };
+  std::vector<Want> want;
+  template <typename T>
+  Pieces& add(T** p, int64_t count) {
+    *p = nullptr;
+    want.push_back({(void**)p, sizeof(T) * (size_t)std::max<int64_t>(count, 1)});
+    return *this;
+  }
+  int32_t alloc(mfixdem_handle* h) {
+    size_t shared = 0;
+    int live = 0;
+    for (const Want& w : want)
+      if (w.bytes <= kSharedMax) {
+        shared += (w.bytes + kPieceAlign - 1) / kPieceAlign * kPieceAlign;
+        live++;
+      }
+    char* at = nullptr;
+    if (live) {
+      if (hipMalloc((void**)&at, shared) != hipSuccess) return MFIXDEM_ERR_OOM;
+      h->blocks.push_back({at, shared, live});
+    }
+    int32_t rc = MFIXDEM_OK;
+    for (const Want& w : want)
+      if (w.bytes <= kSharedMax) {
+        *w.p = at;
+        at += (w.bytes + kPieceAlign - 1) / kPieceAlign * kPieceAlign;
+      } else if (rc == MFIXDEM_OK && hipMalloc(w.p, w.bytes) != hipSuccess) {
+        *w.p = nullptr;
+        rc = MFIXDEM_ERR_OOM;
+      }
+    return rc;
+  }
+};
+
+// the shared allocation that holds p, or -1
+int shared_block(const mfixdem_handle* h, const void* p) {
+  for (size_t b = 0; b < h->blocks.size(); b++) {
+    const char* base = h->blocks[b].base;
+    if ((const char*)p >= base && (const char*)p < base + h->blocks[b].bytes) return (int)b;
+  }
+  return -1;
 }
+
 template <typename T>
-void dfree(T*& p) {
-  if (p) (void)hipFree((void*)p);
+void dfree(mfixdem_handle* h, T*& p) {
+  if (!p) return;
+  const int b = shared_block(h, p);
+  if (b < 0) {
+    (void)hipFree((void*)p);
+  } else if (--h->blocks[b].live == 0) {
+    (void)hipFree(h->blocks[b].base);
+    h->blocks.erase(h->blocks.begin() + b);
+  }
   p = nullptr;
 }
 
@@ -417,12 +480,12 @@ int32_t launch_step(mfixdem_handle* h) {
 int32_t ensure_list_capacity(mfixdem_handle* h, int nl, int64_t entries) {
   if (h->nbr_cap[nl] >= entries) return MFIXDEM_OK;
   const int64_t cap = std::max<int64_t>(entries + entries / 4, 1024);
-  dfree(h->nbr[nl]);
-  dfree(h->nbr_pid[nl]);
-  dfree(h->nbr_row[nl]);
-  CHECKRC(dalloc(&h->nbr[nl], cap));
-  CHECKRC(dalloc(&h->nbr_pid[nl], cap));
-  CHECKRC(dalloc(&h->nbr_row[nl], cap));
+  h->nbr_cap[nl] = 0;
+  dfree(h, h->nbr[nl]);
+  dfree(h, h->nbr_pid[nl]);
+  dfree(h, h->nbr_row[nl]);
+  CHECKRC(Pieces().add(&h->nbr[nl], cap).add(&h->nbr_pid[nl], cap).add(&h->nbr_row[nl], cap)
+              .alloc(h));
   h->nbr_cap[nl] = cap;
   return MFIXDEM_OK;
 }
@@ -431,10 +494,9 @@ int32_t ensure_list_capacity(mfixdem_handle* h, int nl, int64_t entries) {
 int32_t ensure_pft_capacity(mfixdem_handle* h, int b, int64_t pairs) {
   if (h->pft_cap[b] >= pairs && h->pft[b]) return MFIXDEM_OK;
   const int64_t cap = std::max<int64_t>(pairs + pairs / 4, 1024);
-  dfree(h->pft[b]);
-  dfree(h->pfl[b]);
-  CHECKRC(dalloc(&h->pft[b], 3 * cap));
-  CHECKRC(dalloc(&h->pfl[b], cap));
+  dfree(h, h->pft[b]);
+  dfree(h, h->pfl[b]);
+  CHECKRC(Pieces().add(&h->pft[b], 3 * cap).add(&h->pfl[b], cap).alloc(h));
   h->pft_cap[b] = cap;
   return MFIXDEM_OK;
 }
@@ -442,8 +504,8 @@ int32_t ensure_pft_capacity(mfixdem_handle* h, int b, int64_t pairs) {
 int32_t ensure_in_capacity(mfixdem_handle* h, int64_t pairs) {
   if (h->in_cap >= pairs && h->in_tmp) return MFIXDEM_OK;
   const int64_t cap = std::max<int64_t>(pairs + pairs / 4, 1024);
-  dfree(h->in_tmp);
-  CHECKRC(dalloc(&h->in_tmp, cap));
+  dfree(h, h->in_tmp);
+  CHECKRC(Pieces().add(&h->in_tmp, cap).alloc(h));
   h->in_cap = cap;
   return MFIXDEM_OK;
 }
@@ -717,10 +779,9 @@ int32_t do_neighbour(mfixdem_handle* h) {
       continue;
     }
     const int mr = fl[kFlagOwnOverflow] + 16;
-    dfree(h->own_tmp);
-    dfree(h->own_key);
-    CHECKRC(dalloc(&h->own_tmp, (int64_t)n * mr));
-    CHECKRC(dalloc(&h->own_key, (int64_t)n * mr));
+    dfree(h, h->own_tmp);
+    dfree(h, h->own_key);
+    CHECKRC(Pieces().add(&h->own_tmp, (int64_t)n * mr).add(&h->own_key, (int64_t)n * mr).alloc(h));
     h->maxrow = mr;
   }
   CHECKRC(fatal_flags(fl));
@@ -1145,15 +1206,16 @@ int32_t upload_facets(mfixdem_handle* h, const std::vector<const Setup*>& sys) {
       fmask.push_back(m);
     }
   }
-  dfree(h->fac);
-  dfree(h->dg_foff);
-  dfree(h->dg_fids);
-  dfree(h->cell_fmask);
-  int32_t rc;
-  if ((rc = dalloc(&h->fac, (int64_t)fac.size())) || (rc = dalloc(&h->dg_foff, (int64_t)foff.size())) ||
-      (rc = dalloc(&h->dg_fids, (int64_t)fids.size())) ||
-      (rc = dalloc(&h->cell_fmask, (int64_t)fmask.size())))
-    return rc;
+  dfree(h, h->fac);
+  dfree(h, h->dg_foff);
+  dfree(h, h->dg_fids);
+  dfree(h, h->cell_fmask);
+  CHECKRC(Pieces()
+              .add(&h->fac, (int64_t)fac.size())
+              .add(&h->dg_foff, (int64_t)foff.size())
+              .add(&h->dg_fids, (int64_t)fids.size())
+              .add(&h->cell_fmask, (int64_t)fmask.size())
+              .alloc(h));
   if (!fmask.empty())
     HIPOK(hipMemcpy(h->cell_fmask, fmask.data(), fmask.size(), hipMemcpyHostToDevice));
   if (!fac.empty())
@@ -1287,11 +1349,14 @@ void morton_ranks(const int fn[3], int x, int y, int z, int size, int* rank, int
 // Search cells for the counting sort: the rank of each cell (x fastest) in
 // the Morton order of its (fx, fy, fz), so that the binned particles lie in
 // Morton order, system after system, each followed by the place of its
-// nonexistent particles; zeroed counts.
+// nonexistent particles; zeroed counts.  All that a finer or coarser search
+// grid replaces is made here.
 int32_t setup_fine_cells(mfixdem_handle* h) {
-  dfree(h->fine_rank);
-  dfree(h->fine_cnt);
-  dfree(h->fine_off);
+  dfree(h, h->fstart);
+  dfree(h, h->fend);
+  dfree(h, h->fine_rank);
+  dfree(h, h->fine_cnt);
+  dfree(h, h->fine_off);
   const int nf = h->n_fine, ns = h->nsys;
   std::vector<int> rank((size_t)nf);
   int64_t cell = 0;
@@ -1306,9 +1371,13 @@ int32_t setup_fine_cells(mfixdem_handle* h) {
     cell += cells;
   }
   if (cell != nf) return MFIXDEM_ERR_ARG;
-  CHECKRC(dalloc(&h->fine_rank, nf));
-  CHECKRC(dalloc(&h->fine_cnt, (int64_t)nf + ns));
-  CHECKRC(dalloc(&h->fine_off, (int64_t)nf + ns + 1));
+  CHECKRC(Pieces()
+              .add(&h->fstart, nf)
+              .add(&h->fend, nf)
+              .add(&h->fine_rank, nf)
+              .add(&h->fine_cnt, (int64_t)nf + ns)
+              .add(&h->fine_off, (int64_t)nf + ns + 1)
+              .alloc(h));
   HIPOK(hipMemcpy(h->fine_rank, rank.data(), sizeof(int) * nf, hipMemcpyHostToDevice));
   HIPOK(hipMemset(h->fine_cnt, 0, sizeof(int) * ((size_t)nf + ns)));
   return MFIXDEM_OK;
@@ -1326,53 +1395,38 @@ int32_t alloc_buffers(mfixdem_handle* h) {
   auto fail = [&](int32_t r) { return r; };
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess)
     return fail(MFIXDEM_ERR_HIP);
-  for (int b = 0; b < 2; b++) {
-    if ((rc = dalloc(&h->pos[b], 3 * S)) || (rc = dalloc(&h->vel[b], 3 * S)) ||
-        (rc = dalloc(&h->omega[b], 3 * S)) || (rc = dalloc(&h->radius[b], S)) ||
-        (rc = dalloc(&h->pmass[b], S)) || (rc = dalloc(&h->acc[b], 3 * S)) ||
-        (rc = dalloc(&h->racc[b], 3 * S)) || (rc = dalloc(&h->gid[b], S)) ||
-        (rc = dalloc(&h->fcell[b], S)) || (rc = dalloc(&h->dgc[b], S)) ||
-        (rc = dalloc(&h->state[b], S)) || (rc = dalloc(&h->phase[b], S)) ||
-        (rc = dalloc(&h->wmask[b], S)) || (rc = dalloc(&h->wfid[b], kWallSlots * S)) ||
-        (rc = dalloc(&h->wpft[b], 3 * kWallSlots * S)) ||
-        (rc = dalloc(&h->vals[b], n)) ||
-        (rc = dalloc(&h->nbr_start[b], n + 1)) || (rc = dalloc(&h->nbr_split[b], n)) ||
-        (rc = dalloc(&h->pair_base[b], n + 1)))
-      return fail(rc);
-  }
-  if ((rc = dalloc(&h->fc, 3 * S)) || (rc = dalloc(&h->tow, 3 * S)) ||
-      (rc = dalloc(&h->xr_pack, 4 * S)) || (rc = dalloc(&h->place, n)) ||
-      (rc = dalloc(&h->fc_id, 3 * S)) || (rc = dalloc(&h->tow_id, 3 * S)) ||
-      (rc = dalloc(&h->fstart, h->n_fine)) || (rc = dalloc(&h->fend, h->n_fine)) ||
-      (rc = dalloc(&h->own_cnt, n)) || (rc = dalloc(&h->own_tmp, n * h->maxrow)) ||
-      (rc = dalloc(&h->own_key, n * h->maxrow)) || (rc = dalloc(&h->in_cnt, n)) ||
-      (rc = dalloc(&h->in_cur, n)) || (rc = dalloc(&h->tot_cnt, n)) ||
-      (rc = dalloc(&h->scan_bsum64, n / kScanTile + 2)) ||
-      (rc = dalloc(&h->scan_bsum,
-                   std::max<int64_t>(std::max<int64_t>(n, nc), (int64_t)h->n_fine + h->nsys) /
-                           kScanTile + 2)) ||
-      (rc = dalloc(&h->flags, kFlagCount)) || (rc = dalloc(&h->xe, h->S.ni + 1)) ||
-      (rc = dalloc(&h->csz, h->S.ni + h->S.nj + h->S.nk)) ||
-      (rc = dalloc(&h->yn, h->S.nj + 1)) || (rc = dalloc(&h->zt, h->S.nk + 1)) ||
-      (rc = dalloc(&h->vnode, 3 * nc)) || (rc = dalloc(&h->p_force, 3 * nc)) ||
-      (rc = dalloc(&h->ugc, 3 * nc)) || (rc = dalloc(&h->gas_stage, 3 * nc)) ||
-      (rc = dalloc(&h->ep_g, nc)) || (rc = dalloc(&h->rop_s, nc * h->S.p.nphases)) ||
-      (rc = dalloc(&h->rops_node, nc * h->S.p.nphases)) || (rc = dalloc(&h->vol, nc)) ||
-      (rc = dalloc(&h->vol_surr, nc)) || (rc = dalloc(&h->ro_s, MFIXDEM_MAX_PHASES)) ||
-      (rc = dalloc(&h->fluid, nc)) || (rc = dalloc(&h->pic_cnt, nc)) ||
-      (rc = dalloc(&h->pic_off, nc + 1)) || (rc = dalloc(&h->pic_cur, nc)) ||
-      (rc = dalloc(&h->pic, n)) ||
-      (rc = dalloc(&h->stage, std::max<int64_t>(3 * n, (73 * max_cap + 7) / 8))) ||
-      (rc = dalloc(&h->rops_fix[0], nc * h->S.p.nphases)) ||
-      (rc = dalloc(&h->rops_fix[1], nc * h->S.p.nphases)) || (rc = dalloc(&h->rm_cnt, 2)) ||
-      (rc = dalloc(&h->rm_list, n)))
-    return fail(rc);
+  Pieces a;
+  for (int b = 0; b < 2; b++)
+    a.add(&h->pos[b], 3 * S).add(&h->vel[b], 3 * S).add(&h->omega[b], 3 * S).add(&h->radius[b], S)
+        .add(&h->pmass[b], S).add(&h->acc[b], 3 * S).add(&h->racc[b], 3 * S).add(&h->gid[b], S)
+        .add(&h->fcell[b], S).add(&h->dgc[b], S).add(&h->state[b], S).add(&h->phase[b], S)
+        .add(&h->wmask[b], S).add(&h->wfid[b], kWallSlots * S)
+        .add(&h->wpft[b], 3 * kWallSlots * S).add(&h->vals[b], n).add(&h->nbr_start[b], n + 1)
+        .add(&h->nbr_split[b], n).add(&h->pair_base[b], n + 1);
+  a.add(&h->fc, 3 * S).add(&h->tow, 3 * S).add(&h->xr_pack, 4 * S).add(&h->place, n)
+      .add(&h->fc_id, 3 * S).add(&h->tow_id, 3 * S).add(&h->own_cnt, n)
+      .add(&h->own_tmp, n * h->maxrow)
+      .add(&h->own_key, n * h->maxrow).add(&h->in_cnt, n).add(&h->in_cur, n).add(&h->tot_cnt, n)
+      .add(&h->scan_bsum64, n / kScanTile + 2)
+      .add(&h->scan_bsum,
+           std::max<int64_t>(std::max<int64_t>(n, nc), (int64_t)h->n_fine + h->nsys) / kScanTile + 2)
+      .add(&h->flags, kFlagCount).add(&h->xe, h->S.ni + 1)
+      .add(&h->csz, h->S.ni + h->S.nj + h->S.nk).add(&h->yn, h->S.nj + 1).add(&h->zt, h->S.nk + 1)
+      .add(&h->vnode, 3 * nc).add(&h->p_force, 3 * nc).add(&h->ugc, 3 * nc)
+      .add(&h->gas_stage, 3 * nc).add(&h->ep_g, nc).add(&h->rop_s, nc * h->S.p.nphases)
+      .add(&h->rops_node, nc * h->S.p.nphases).add(&h->vol, nc).add(&h->vol_surr, nc)
+      .add(&h->ro_s, MFIXDEM_MAX_PHASES).add(&h->fluid, nc).add(&h->pic_cnt, nc)
+      .add(&h->pic_off, nc + 1).add(&h->pic_cur, nc).add(&h->pic, n)
+      .add(&h->stage, std::max<int64_t>(3 * n, (73 * max_cap + 7) / 8))
+      .add(&h->rops_fix[0], nc * h->S.p.nphases).add(&h->rops_fix[1], nc * h->S.p.nphases)
+      .add(&h->rm_cnt, 2).add(&h->rm_list, n);
+  if (h->S.p.des_explicitly_coupled) a.add(&h->f_gp, n).add(&h->drag_fc, 3 * n);
+  if ((rc = a.alloc(h))) return fail(rc);
   for (int b = 0; b < 2; b++)
     if (hipMemset(h->rops_fix[b], 0, sizeof(unsigned long long) * nc * h->S.p.nphases) != hipSuccess)
       return fail(MFIXDEM_ERR_HIP);
   if (hipMemset(h->rm_cnt, 0, 2 * sizeof(int)) != hipSuccess) return fail(MFIXDEM_ERR_HIP);
   if (h->S.p.des_explicitly_coupled) {
-    if ((rc = dalloc(&h->f_gp, n)) || (rc = dalloc(&h->drag_fc, 3 * n))) return fail(rc);
     if (hipMemset(h->f_gp, 0, sizeof(double) * n) != hipSuccess ||
         hipMemset(h->drag_fc, 0, sizeof(double) * 3 * n) != hipSuccess)
       return fail(MFIXDEM_ERR_HIP);
@@ -1494,7 +1548,7 @@ int32_t mfixdem_create(const mfixdem_params* p, mfixdem_handle** out) {
 int32_t mfixdem_destroy(mfixdem_handle* h) {
   if (!h) return MFIXDEM_ERR_ARG;
   if (h->stream) (void)sync_stream(h);
-  for_each_buffer(h, [](auto*& p) { dfree(p); });
+  for_each_buffer(h, [h](auto*& p) { dfree(h, p); });
   if (h->host_flags) (void)hipHostFree(h->host_flags);
   if (h->ring) (void)hipHostFree(h->ring);
   for (auto& e : h->ring_ev)
@@ -1663,18 +1717,20 @@ int32_t mfixdem_set_dem_bcs(mfixdem_handle* h, int32_t n, const mfixdem_dem_bc* 
   D.rng = seed;
   CHECKRC(setup_dem_bcs(h->S, D));
   HIPOK(sync_stream(h));
-  for (auto** q : {&h->slot_of_gid, &h->del_cnt, &h->del_list}) dfree(*q);
-  dfree(h->d_bcs);
-  dfree(h->d_seeds);
+  for (auto** q : {&h->slot_of_gid, &h->del_cnt, &h->del_list}) dfree(h, *q);
+  dfree(h, h->d_bcs);
+  dfree(h, h->d_seeds);
   h->dbc = DemBoundaries{};
   h->P.nbc = 0;
   if (n == 0) return MFIXDEM_OK;
   const int64_t N = h->n;
-  CHECKRC(dalloc(&h->d_bcs, n));
-  CHECKRC(dalloc(&h->d_seeds, std::max(D.max_seeds, 1)));
-  CHECKRC(dalloc(&h->slot_of_gid, N));
-  CHECKRC(dalloc(&h->del_cnt, 1));
-  CHECKRC(dalloc(&h->del_list, N));
+  CHECKRC(Pieces()
+              .add(&h->d_bcs, n)
+              .add(&h->d_seeds, D.max_seeds)
+              .add(&h->slot_of_gid, N)
+              .add(&h->del_cnt, 1)
+              .add(&h->del_list, N)
+              .alloc(h));
   const std::vector<BcDev> bd = bcs_dev(h->S, D);
   HIPOK(hipMemcpy(h->d_bcs, bd.data(), sizeof(BcDev) * n, hipMemcpyHostToDevice));
   h->dbc = std::move(D);
@@ -1885,12 +1941,13 @@ int32_t ensure_gas_drag(mfixdem_handle* h) {
                       volf(i + 1, j, k + 1));
         vn[cell(i, j, k)] = a;
       }
-  int32_t rc;
-  if ((rc = dalloc(&h->gd_fgp, (int64_t)kGasRec * h->stride)) ||
-      (rc = dalloc(&h->gd_vol_node, nc)) ||
-      (rc = dalloc(&h->gd_am, nc)) || (rc = dalloc(&h->gd_bm, 3 * (int64_t)nc)) ||
-      (rc = dalloc(&h->gd_fgds, nc)))
-    return rc;
+  CHECKRC(Pieces()
+              .add(&h->gd_fgp, (int64_t)kGasRec * h->stride)
+              .add(&h->gd_vol_node, nc)
+              .add(&h->gd_am, nc)
+              .add(&h->gd_bm, 3 * (int64_t)nc)
+              .add(&h->gd_fgds, nc)
+              .alloc(h));
   HIPOK(hipMemcpy(h->gd_vol_node, vn.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
   return MFIXDEM_OK;
 }
@@ -2237,11 +2294,15 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
     h->rogue_init[2 * s] = INT_MAX;
     h->rogue_init[2 * s + 1] = 0;
   }
-  if (rc == MFIXDEM_OK &&
-      ((rc = dalloc(&h->d_sys, h->stride)) || (rc = dalloc(&h->d_ptab, nsys)) ||
-       (rc = dalloc(&h->d_gtab, nsys)) || (rc = dalloc(&h->d_cell_off, nsys + 1)) ||
-       (rc = dalloc(&h->d_dg_off, nsys + 1)) || (rc = dalloc(&h->d_rogue, 2 * nsys))))
-    rc = MFIXDEM_ERR_OOM;
+  if (rc == MFIXDEM_OK)
+    rc = Pieces()
+             .add(&h->d_sys, h->stride)
+             .add(&h->d_ptab, nsys)
+             .add(&h->d_gtab, nsys)
+             .add(&h->d_cell_off, nsys + 1)
+             .add(&h->d_dg_off, nsys + 1)
+             .add(&h->d_rogue, 2 * nsys)
+             .alloc(h);
   if (rc == MFIXDEM_OK &&
       (hipMemcpy(h->d_sys, sys.data(), sizeof(uint16_t) * h->stride, hipMemcpyHostToDevice) ||
        hipMemcpy(h->d_ptab, ptab.data(), sizeof(DevParams) * nsys, hipMemcpyHostToDevice) ||
@@ -2339,10 +2400,6 @@ int32_t mfixdem_set_tuning(mfixdem_handle* h, double cell_scale, int32_t row_ker
     h->sys_grid = gt;
     h->G = gt[0];
   }
-  dfree(h->fstart);
-  dfree(h->fend);
-  CHECKRC(dalloc(&h->fstart, n_fine));
-  CHECKRC(dalloc(&h->fend, n_fine));
   h->n_fine = n_fine;
   CHECKRC(setup_fine_cells(h));
   h->cell_scale = cell_scale;
@@ -2356,11 +2413,12 @@ int32_t mfixdem_get_device_bytes(mfixdem_handle* h, int64_t* bytes) {
   int64_t total = 0;
   int32_t rc = MFIXDEM_OK;
   for_each_buffer(h, [&](auto*& p) {
-    if (!p) return;
+    if (!p || shared_block(h, p) >= 0) return;
     size_t sz = 0;
     if (hipMemPtrGetInfo((void*)p, &sz) != hipSuccess) rc = MFIXDEM_ERR_HIP;
     total += (int64_t)sz;
   });
+  for (const auto& b : h->blocks) total += (int64_t)b.bytes;
   *bytes = total;
   return rc;
 }
