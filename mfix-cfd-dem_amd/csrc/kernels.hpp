@@ -2488,8 +2488,19 @@ struct BcPtrs {
   const uint8_t* phase;
   const BcDev* bcs;
   int nbc, n, S;
-  int* del_cnt;   // deleted particles: count and global ids
-  int* del_list;
+  int* del_cnt;   // particles deleted so far and blocks done, both left at 0
+  int* del_list;  // their global ids
+  struct BcHost* host;
+  int seq;
+};
+
+// What the host needs of a step with inlets and outlets before it can queue
+// the next one, in pinned memory: the sequence number of the step is written
+// last.  Ids beyond kBcHostGids are read from del_list.
+constexpr int kBcHostGids = 256;
+struct BcHost {
+  int seq, count;
+  int gid[kBcHostGids];
 };
 
 // The checks MASS_INFLOW_DEM (mass_inflow_dem.f:68-139) and MASS_OUTFLOW_DEM
@@ -2505,11 +2516,10 @@ struct BcPtrs {
 //           gives it the outlet's velocity, other outlets keep only its
 //           outward normal velocity, and only while it moves outwards);
 //           deleted (DELETE_PARTICLE, :201-280) once the centre is out.
-__global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= b.n) return;
+// True if the particle was deleted.
+__device__ inline bool particle_bcs(const BcPtrs& b, int i) {
   const int st0 = b.state[i];
-  if (st0 == kNonexistent || st0 == kSeeded) return;
+  if (st0 == kNonexistent || st0 == kSeeded) return false;
   const int S = b.S, dc = b.dgc[i];
   int st = st0;
   double x[3], v[3];
@@ -2554,11 +2564,32 @@ __global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
     b.pmass[i] = 3.4028234663852886e38;  // HUGE(0.0) as DELETE_PARTICLE sets it
     b.wmask[i] = 0;
     b.state[i] = kNonexistent;
-    b.del_list[atomicAdd(b.del_cnt, 1)] = b.gid[i];
-    return;
+    const int at = atomicAdd(b.del_cnt, 1), g = b.gid[i];
+    b.del_list[at] = g;
+    if (at < kBcHostGids) b.host->gid[at] = g;
+    return true;
   }
   if (st != st0) b.state[i] = (uint8_t)st;
   if (vset) store3(b.vel, S, i, v);
+  return false;
+}
+
+// One particle per thread; the block that ends last hands the count and the
+// ids to the host and clears the counters for the next step.  A fill before
+// the kernel, a copy of the count and a wait for the stream took 24 us of a
+// 53 us step at 30,000 particles.
+__global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
+  const int i = blockIdx.x * kBS + threadIdx.x;
+  const bool gone = i < b.n && particle_bcs(b, i);
+  if (gone) __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x) return;
+  const int done = __hip_atomic_fetch_add(b.del_cnt + 1, 1, __ATOMIC_ACQ_REL,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+  if (done != (int)gridDim.x - 1) return;
+  b.host->count = __hip_atomic_load(b.del_cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  b.del_cnt[0] = b.del_cnt[1] = 0;
+  __hip_atomic_store(&b.host->seq, b.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 struct SeedPtrs {

@@ -165,11 +165,14 @@ struct mfixdem_handle {
   // walk's candidates during a rebuild
   double* stage = nullptr;
   // DEM mass inlets / outlets (mfixdem_set_dem_bcs): host schedule and
-  // layout, the device table, this step's seeds, the slot of each global id
+  // layout, the device table, the slot of each global id
   // (rewritten at every binning) and the particles deleted in a step
   DemBoundaries dbc;
   BcDev* d_bcs = nullptr;
-  SeedDev* d_seeds = nullptr;
+  // pinned: the end of a step's checks, and the seeds of two steps (one is
+  // filled while the other may still be read)
+  BcHost* bc_host = nullptr;
+  int bc_seq = 0;
   int *slot_of_gid = nullptr, *del_cnt = nullptr, *del_list = nullptr;
   // status
   mfixdem_status st{};
@@ -300,14 +303,13 @@ int32_t scan_rows(mfixdem_handle* h, const int* own, const int* in, int* pair_ba
   return MFIXDEM_OK;
 }
 
-// Waits until the last scan_rows has written its flags to the host, without
-// waiting for what is queued behind it (a copy and a wait for the stream cost
-// 23 us and left the stream empty).  Ends with an error if the stream ends
-// first, which a failed launch or a device error makes it do.
-int32_t wait_flags(mfixdem_handle* h, int fl[kFlagCount]) {
-  auto seen = [&] {
-    return __atomic_load_n(&h->host_flags->seq, __ATOMIC_ACQUIRE) == h->flags_seq;
-  };
+// Waits until a kernel of the handle's stream has written `want` to a word of
+// pinned memory, without waiting for what is queued behind it (a copy and a
+// wait for the stream cost 23 us and left the stream empty).  Ends with an
+// error if the stream ends first, which a failed launch or a device error
+// makes it do.
+int32_t wait_seq(mfixdem_handle* h, const int* seq, int want) {
+  auto seen = [&] { return __atomic_load_n(seq, __ATOMIC_ACQUIRE) == want; };
   for (int spin = 0; !seen(); spin++) {
     if ((spin & 1023) != 1023) {
       __builtin_ia32_pause();
@@ -318,6 +320,11 @@ int32_t wait_flags(mfixdem_handle* h, int fl[kFlagCount]) {
     HIPOK(e);
     if (!seen()) return MFIXDEM_ERR_HIP;
   }
+  return MFIXDEM_OK;
+}
+// the flags of the last scan_rows
+int32_t wait_flags(mfixdem_handle* h, int fl[kFlagCount]) {
+  CHECKRC(wait_seq(h, &h->host_flags->seq, h->flags_seq));
   std::memcpy(fl, h->host_flags->fl, sizeof(int) * kFlagCount);
   return MFIXDEM_OK;
 }
@@ -996,7 +1003,6 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
   h->cur = 1 - h->cur;
   h->pcur = 1 - h->pcur;
   const int c = h->cur, t = h->tw;
-  CHECKRC(fill_i32(h->stream, h->del_cnt, 1, 0));
   BcPtrs b{};
   b.pos = h->pos[c]; b.vel = h->vel[c]; b.omega = h->omega[c];
   b.radius = h->radius[t]; b.pmass = h->pmass[t];
@@ -1004,30 +1010,39 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
   b.phase = h->phase[t];
   b.bcs = h->d_bcs; b.nbc = (int)D.b.size(); b.n = n; b.S = h->stride;
   b.del_cnt = h->del_cnt; b.del_list = h->del_list;
+  b.host = h->bc_host; b.seq = ++h->bc_seq;
   hipLaunchKernelGGL(k_dem_bcs, dim3(nblk(n)), dim3(kBS), 0, h->stream, b);
   HIPOK(hipGetLastError());
-  CHECKRC(plan_seeds(h->S, D));
+  if (const int32_t rc = plan_seeds(h->S, D)) {
+    CHECKRC(wait_seq(h, &h->bc_host->seq, h->bc_seq));
+    return rc;
+  }
   const int ns = (int)D.seeds.size();
   if (ns > 0) {
-    HIPOK(hipMemcpyAsync(h->d_seeds, D.seeds.data(), sizeof(SeedDev) * ns,
-                         hipMemcpyHostToDevice, h->stream));
+    // the kernel reads the records where the host writes them: those of the
+    // step before last are free, their step's end has been waited for
+    SeedDev* seeds = (SeedDev*)(h->bc_host + 1) + (size_t)(h->bc_seq & 1) * D.max_seeds;
+    std::memcpy(seeds, D.seeds.data(), sizeof(SeedDev) * ns);
     SeedPtrs sp{};
     sp.pos = h->pos[c]; sp.vel = h->vel[c]; sp.omega = h->omega[c];
     sp.radius = h->radius[t]; sp.pmass = h->pmass[t];
     sp.dgc = h->dgc[t]; sp.fcell = h->fcell[t];
     sp.state = h->state[t]; sp.phase = h->phase[t]; sp.wmask = h->wmask[t];
     sp.slot_of_gid = h->slot_of_gid; sp.S = h->stride;
-    hipLaunchKernelGGL(k_seed, dim3(nblk(ns)), dim3(kBS), 0, h->stream, ns, h->d_seeds, sp);
+    hipLaunchKernelGGL(k_seed, dim3(nblk(ns)), dim3(kBS), 0, h->stream, ns, seeds, sp);
     HIPOK(hipGetLastError());
   }
-  int nd = 0;
-  HIPOK(hipMemcpyAsync(&nd, h->del_cnt, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-  HIPOK(sync_stream(h));  // also frees the seed records for the next step
+  CHECKRC(wait_seq(h, &h->bc_host->seq, h->bc_seq));
+  const int nd = h->bc_host->count;
   if (nd > 0) {
     std::vector<int> gone(nd);
-    HIPOK(hipMemcpyAsync(gone.data(), h->del_list, sizeof(int) * nd, hipMemcpyDeviceToHost,
-                         h->stream));
-    HIPOK(sync_stream(h));
+    if (nd <= kBcHostGids) {
+      std::memcpy(gone.data(), h->bc_host->gid, sizeof(int) * nd);
+    } else {
+      HIPOK(hipMemcpyAsync(gone.data(), h->del_list, sizeof(int) * nd, hipMemcpyDeviceToHost,
+                           h->stream));
+      HIPOK(sync_stream(h));
+    }
     for (int g : gone) D.free_gids.insert(g);
     rebuild = true;  // FORCE_NSEARCH (mass_outflow_dem.f:178)
   }
@@ -1325,7 +1340,7 @@ void for_each_buffer(mfixdem_handle* h, F f) {
   f(h->gd_fgp); f(h->gd_vol_node); f(h->gd_am); f(h->gd_bm); f(h->gd_fgds);
   f(h->fac); f(h->dg_foff); f(h->dg_fids); f(h->cell_fmask); f(h->stage);
   f(h->d_sys); f(h->d_ptab); f(h->d_gtab); f(h->d_cell_off); f(h->d_dg_off); f(h->d_rogue);
-  f(h->d_bcs); f(h->d_seeds); f(h->slot_of_gid); f(h->del_cnt); f(h->del_list);
+  f(h->d_bcs); f(h->slot_of_gid); f(h->del_cnt); f(h->del_list);
 }
 
 void fill_devparams(mfixdem_handle* h) {
@@ -1551,6 +1566,7 @@ int32_t mfixdem_destroy(mfixdem_handle* h) {
   for_each_buffer(h, [h](auto*& p) { dfree(h, p); });
   if (h->host_flags) (void)hipHostFree(h->host_flags);
   if (h->ring) (void)hipHostFree(h->ring);
+  if (h->bc_host) (void)hipHostFree(h->bc_host);
   for (auto& e : h->ring_ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : h->ev)
@@ -1719,18 +1735,24 @@ int32_t mfixdem_set_dem_bcs(mfixdem_handle* h, int32_t n, const mfixdem_dem_bc* 
   HIPOK(sync_stream(h));
   for (auto** q : {&h->slot_of_gid, &h->del_cnt, &h->del_list}) dfree(h, *q);
   dfree(h, h->d_bcs);
-  dfree(h, h->d_seeds);
+  if (h->bc_host) (void)hipHostFree(h->bc_host);
+  h->bc_host = nullptr;
+  h->bc_seq = 0;
   h->dbc = DemBoundaries{};
   h->P.nbc = 0;
   if (n == 0) return MFIXDEM_OK;
   const int64_t N = h->n;
   CHECKRC(Pieces()
               .add(&h->d_bcs, n)
-              .add(&h->d_seeds, D.max_seeds)
               .add(&h->slot_of_gid, N)
-              .add(&h->del_cnt, 1)
+              .add(&h->del_cnt, 2)
               .add(&h->del_list, N)
               .alloc(h));
+  if (hipHostMalloc((void**)&h->bc_host, sizeof(BcHost) + 2 * sizeof(SeedDev) * D.max_seeds,
+                    hipHostMallocDefault) != hipSuccess)
+    return MFIXDEM_ERR_OOM;
+  h->bc_host->seq = 0;
+  CHECKRC(fill_i32(h->stream, h->del_cnt, 2, 0));
   const std::vector<BcDev> bd = bcs_dev(h->S, D);
   HIPOK(hipMemcpy(h->d_bcs, bd.data(), sizeof(BcDev) * n, hipMemcpyHostToDevice));
   h->dbc = std::move(D);
