@@ -2,9 +2,10 @@
 //
 // Layout in HBM (all per-particle arrays in the current Morton order of the
 // neighbour-search grid; component c of particle i at [c*stride + i]):
-//   pos/vel/omega      double, double-buffered (read one, write the other)
-//   radius/pmass, gid, state, phase, dgc (DES cell), fcell (fluid
-//   cell), wall mask + per-facet wall history, AB2 accelerations
+//   pos                Sphere records (x, y, z, radius), and vel/omega, double:
+//                      all double-buffered (read one, write the other)
+//   pmass, gid, state, phase, dgc (DES cell), fcell (fluid cell), wall mask
+//   + per-facet wall history, AB2 accelerations
 //   neighbour rows     full rows: [incoming (owner has lower id) | own]
 //                      nbr_start[i] .. nbr_split[i] .. nbr_start[i+1]
 //                      nbr = neighbour slot, nbr_pid = pair id (history slot)
@@ -60,10 +61,28 @@ struct SeedDev {
   int gid, dgc, fcell, phase;
 };
 
+// Position and radius of a particle (x, y, z, w = radius) in one 32-byte
+// record: the contact test gathers two 16-byte pieces of one cache line per
+// neighbour instead of a piece of four lines.  The address and tag units of
+// the vector cache bound the step of a large bed (62 % busy at 3M spheres,
+// with 2 TB/s of HBM traffic).  Per step, with component planes and then with
+// records: 3M uneven systems 287 and 276 us, 301,057 spheres at 0.60 70.7 and
+// 66.2, 1M coupled at 0.30 91.0 and 88.6.
+typedef double Sphere __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ double load_sphere(const Sphere* p, int i, double x[3]) {
+  const Sphere s = p[i];
+  x[0] = s.x;
+  x[1] = s.y;
+  x[2] = s.z;
+  return s.w;
+}
+
 struct StepPtrs {
-  const double *pos, *vel, *omega;
-  double *pos_o, *vel_o, *omega_o;
-  const double *radius, *pmass;
+  const Sphere* pos;
+  Sphere* pos_o;
+  const double *vel, *omega;
+  double *vel_o, *omega_o;
+  const double* pmass;
   const int* gid;
   uint8_t* state;
   const uint8_t* phase;
@@ -336,19 +355,19 @@ __device__ __forceinline__ void add_drag_des1(const DevParams& P, const StepPtrs
   }
   if (lepg < 1.0e-6) lepg = a.ep_g[c0];
   if (!fluid_at(P, ci, cj, ck)) return;
-  const double pvol = sphere_volume(a.radius[i]);
+  const double pvol = sphere_volume(a.pos[i].w);
   if (!MIXED) {
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
     const double fgp = drag_fgp_fp64(P.drag_type, lepg, P.mu_g0, P.ro_g0, vrel,
-                                     2.0 * a.radius[i], pvol);
+                                     2.0 * a.pos[i].w, pvol);
     for (int d = 0; d < 3; d++) fc[d] = fc[d] + fgp * (velfp[d] - vel[d]);
   } else {
     const float vs[3] = {(float)(velfp[0] - vel[0]), (float)(velfp[1] - vel[1]),
                          (float)(velfp[2] - vel[2])};
     const float vrel = fsqrt(dot3f(vs, vs));
     const float fgp = drag_fgp_fp32(P.drag_type, (float)lepg, (float)P.mu_g0, (float)P.ro_g0,
-                                    vrel, (float)(2.0 * a.radius[i]), (float)pvol);
+                                    vrel, (float)(2.0 * a.pos[i].w), (float)pvol);
     for (int d = 0; d < 3; d++) fc[d] = fc[d] + (double)(fgp * vs[d]);
   }
   for (int d = 0; d < 3; d++) fc[d] = fc[d] + lpf[d] * pvol;
@@ -389,19 +408,19 @@ __device__ __forceinline__ void add_drag(const DevParams& P, const StepPtrs& a, 
         const double* vn = a.vnode + 3 * (base + jj + ii * P.nj + kk * P.nj * P.ni);
         for (int d = 0; d < 3; d++) velfp[d] = velfp[d] + vn[d] * w;
       }
-  const double pvol = sphere_volume(a.radius[i]);
+  const double pvol = sphere_volume(a.pos[i].w);
   if (!MIXED) {
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
     const double fgp = drag_fgp_fp64(P.drag_type, a.ep_g[c], P.mu_g0, P.ro_g0, vrel,
-                                     2.0 * a.radius[i], pvol);
+                                     2.0 * a.pos[i].w, pvol);
     for (int d = 0; d < 3; d++) fc[d] = fc[d] + fgp * (velfp[d] - vel[d]);
   } else {
     const float vs[3] = {(float)(velfp[0] - vel[0]), (float)(velfp[1] - vel[1]),
                          (float)(velfp[2] - vel[2])};
     const float vrel = fsqrt(dot3f(vs, vs));
     const float fgp = drag_fgp_fp32(P.drag_type, (float)a.ep_g[c], (float)P.mu_g0,
-                                    (float)P.ro_g0, vrel, (float)(2.0 * a.radius[i]), (float)pvol);
+                                    (float)P.ro_g0, vrel, (float)(2.0 * a.pos[i].w), (float)pvol);
     for (int d = 0; d < 3; d++) fc[d] = fc[d] + (double)(fgp * vs[d]);
   }
   for (int d = 0; d < 3; d++) fc[d] = fc[d] + a.p_force[3 * c + d] * pvol;
@@ -532,8 +551,7 @@ constexpr unsigned kRowOwn = 64u;
 __device__ __forceinline__ bool pair_touches(const StepPtrs& a, int S, const double xp[3],
                                              double rp, int j, int pid, bool owner) {
   double xj[3];
-  load3(a.pos, S, j, xj);
-  const double rj = a.radius[j];
+  const double rj = load_sphere(a.pos, j, xj);
   // IF(IS_NONEXISTENT(I)) CYCLE: history kept.  A nonexistent particle has
   // radius 0 (set with its state), so the state is read only then.
   if (rj == 0.0 && a.state[j] == 0) {
@@ -570,8 +588,7 @@ __device__ __forceinline__ void pair_contact(const DevParams& P0, const PT& P, c
   const int S = P0.stride;
   PairIn in;
   double xj[3], vj[3], wj[3], vp[3], wp[3];
-  load3(a.pos, S, j, xj);
-  const double rj = a.radius[j];
+  const double rj = load_sphere(a.pos, j, xj);
   load3(a.vel, S, j, vj);
   load3(a.omega, S, j, wj);
   load3(a.vel, S, ip, vp);
@@ -738,7 +755,7 @@ struct DepIn {
 // LDS that the step no longer uses), then one global atomic per non-zero
 // node; a larger box or a multi-phase system adds straight to fix.  A
 // particle that left the grid is queued (slot id) for the next kernel,
-// which sets its state and radius to 0: other lanes of this launch may
+// which sets its state to 0: other lanes of this launch may
 // still read them as a partner's.  Every thread of the workgroup calls
 // this (it holds barriers).
 __device__ __forceinline__ void fused_deposit(const DevParams& P, const StepPtrs& a, int i,
@@ -866,8 +883,8 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
   const int S = P0.stride;
   if (st == 0) {
     if (MODE == kModeFused || MODE == kModeIntegrate) {
+      a.pos_o[i] = a.pos[i];
       for (int c = 0; c < 3; c++) {
-        a.pos_o[c * S + i] = a.pos[c * S + i];
         a.vel_o[c * S + i] = a.vel[c * S + i];
         a.omega_o[c * S + i] = a.omega[c * S + i];
       }
@@ -880,7 +897,7 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
     return;
   }
   double pos[3], vel[3], om[3];
-  load3(a.pos, S, i, pos);
+  const double ri = load_sphere(a.pos, i, pos);
   load3(a.vel, S, i, vel);
   load3(a.omega, S, i, om);
   const double mi = a.pmass[i];
@@ -911,7 +928,7 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
 
   // ---- CFNEWVALUES (cfnewvalues.f:700-811)
   const double dt = P.dt;
-  const double omoi = sphere_omoi(mi, a.radius[i]);
+  const double omoi = sphere_omoi(mi, ri);
   if (!P.ab2) {
     // entering and exiting particles move at their velocity (:492, :593)
     const bool normal = st == kNormal;
@@ -957,17 +974,17 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
     a.fcell[i] = pc;
   }
   if (kEarlyDrag && P0.fuse_dep && pc < 0) {
-    // PARTICLES_IN_CELL deletion (particles_in_cell.f:175-184): state and
-    // radius follow in the next kernel
+    // PARTICLES_IN_CELL deletion (particles_in_cell.f:175-184): the state
+    // follows in the next kernel
     const double z[3] = {0.0, 0.0, 0.0};
-    store3(a.pos_o, S, i, z);
+    a.pos_o[i] = Sphere{0.0, 0.0, 0.0, 0.0};
     store3(a.vel_o, S, i, z);
     store3(a.omega_o, S, i, z);
     a.wmask[i] = 0;
     dep.remove = true;
     return;
   }
-  store3(a.pos_o, S, i, pos);
+  a.pos_o[i] = Sphere{pos[0], pos[1], pos[2], ri};
   store3(a.vel_o, S, i, vel);
   store3(a.omega_o, S, i, om);
   if (kEarlyDrag && P0.fuse_dep && fluid_at(P, I, J, K)) {
@@ -1019,10 +1036,10 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
     double xr[4] = {0.0, 0.0, 0.0, -1.0};
     if (live && st != 0) {
       double pos[3], vel[3], om[3];
-      load3(a.pos, S, i, pos);
+      const double ri = load_sphere(a.pos, i, pos);
       load3(a.vel, S, i, vel);
       load3(a.omega, S, i, om);
-      const double ri = a.radius[i], mi = a.pmass[i];
+      const double mi = a.pmass[i];
       for (int c = 0; c < 3; c++) xr[c] = pos[c];
       xr[3] = ri;
       const int phi = a.phase[i];
@@ -1128,18 +1145,18 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
 struct Removal {
   uint8_t* state;
   uint8_t* wmask;
-  double *pos, *vel, *omega, *radius;
+  Sphere* pos;
+  double *vel, *omega;
   int* flags;
 };
 __device__ __forceinline__ void remove_outside(const Removal& r, int S, int i) {
   r.state[i] = 0;
   r.wmask[i] = 0;
+  r.pos[i] = Sphere{0.0, 0.0, 0.0, 0.0};
   for (int d = 0; d < 3; d++) {
-    r.pos[d * S + i] = 0.0;
     r.vel[d * S + i] = 0.0;
     r.omega[d * S + i] = 0.0;
   }
-  r.radius[i] = 0.0;
   atomicAdd(&r.flags[kFlagOutOfDomain], 1);
 }
 
@@ -1159,7 +1176,7 @@ __device__ __forceinline__ void remove_outside(const Removal& r, int S, int i) {
 constexpr int kDepPPT = 2;
 constexpr int kDepCap = 4096;
 __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* list,
-                                                      const double* pos, const double* pmass,
+                                                      const Sphere* pos, const double* pmass,
                                                       const uint8_t* phase, const uint8_t* state,
                                                       const int* fcell, const uint8_t* fluid,
                                                       const double* xe, const double* yn,
@@ -1183,9 +1200,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* li
   for (int u = 0; u < kDepPPT; u++) {
     const int i = pi[u] < 0 ? 0 : pi[u];
     pph[u] = phase[i];
-    px[u][0] = pos[i];
-    px[u][1] = pos[S + i];
-    px[u][2] = pos[2 * S + i];
+    load_sphere(pos, i, px[u]);
     pm[u] = pmass[i];
   }
 #pragma unroll
@@ -1317,7 +1332,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* li
 // order (list null) or list order; the workgroup's cells are summed in an LDS tile over
 // the bounding box of its targets (up to kDepCap cells), else directly.
 __global__ __launch_bounds__(kBS) void k_deposit_filter(DevParams P, const int* list,
-                                                        const double* pos, const double* radius,
+                                                        const Sphere* pos,
                                                         const uint8_t* phase, const uint8_t* state,
                                                         const int* fcell, const double* xe,
                                                         const double* yn, const double* zt,
@@ -1370,7 +1385,8 @@ __global__ __launch_bounds__(kBS) void k_deposit_filter(DevParams P, const int* 
   __syncthreads();
   if (pc >= 0) {
     const int ph = phase[i];
-    const double vol_wt = sphere_volume(radius[i]);
+    double x[3];
+    const double vol_wt = sphere_volume(load_sphere(pos, i, x));
     const double sc = P.dep_scale[ph];
     unsigned long long* f = fix + (size_t)ph * P.ncell;
     auto add = [&](int I, int J, int K, double w) {
@@ -1381,7 +1397,6 @@ __global__ __launch_bounds__(kBS) void k_deposit_filter(DevParams P, const int* 
       else atomicAdd(&f[lin_ijk(I, J, K, P.ni, P.nj)], qv);
     };
     if (filter_scheme(P.interp)) {
-      const double x[3] = {pos[i], pos[S + i], pos[2 * S + i]};
       for_filter(P, xe, yn, zt, csz, ci, cj, ck, x, add);
     } else {
       add(ci, cj, ck, 1.0);
@@ -1640,7 +1655,7 @@ __device__ __forceinline__ int absent_cell(const BatchDev& B, int s, int nfine) 
   return BATCH ? B.cell_off[s + 1] + s : nfine;
 }
 template <bool BATCH>
-__global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G0, const double* pos,
+__global__ __launch_bounds__(kBS) void k_bin_count(int n, GridDev G0, const Sphere* pos,
                                                    uint8_t* state, const int* gid,
                                                    int* dgc, const int* cell_rank,
                                                    int* cell_cnt, int nfine, uint64_t* place,
@@ -1656,7 +1671,8 @@ __global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G0, con
     if constexpr (BATCH) Gs = load_uniform(B.gtab + s);
     const GridDev& G = BATCH ? Gs : G0;
     if (state[i] == kSeeded) state[i] = kEntering;  // binned now: in a DES cell list
-    const double x[3] = {pos[i], pos[S + i], pos[2 * S + i]};
+    double x[3];
+    load_sphere(pos, i, x);
     const int nn[3] = {G.dg_ni, G.dg_nj, G.dg_nk};
     int c3[3], f3[3];
 #pragma unroll
@@ -1704,8 +1720,7 @@ __global__ __launch_bounds__(kBS) void k_bin_count(int n, int S, GridDev G0, con
 // The counts go back to zero for the next binning.
 struct BinPack {               // k_bin_place's packing of the row walk's candidates
   GridDev G;
-  int S;
-  const double *pos, *radius;
+  const Sphere* pos;
   const uint8_t* state;
   double* xr;
   float4* xf;
@@ -1728,8 +1743,9 @@ __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, int nsys,
     GridDev Gs;
     if constexpr (BATCH)
       Gs = load_uniform(B.gtab + wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(i)));
-    const double x[3] = {bp.pos[i], bp.pos[bp.S + i], bp.pos[2 * bp.S + i]};
-    pack_candidate(BATCH ? Gs : bp.G, x, bp.radius[i], bp.state[i] != 0, bp.xr, bp.xf, np);
+    double x[3];
+    const double r = load_sphere(bp.pos, i, x);
+    pack_candidate(BATCH ? Gs : bp.G, x, r, bp.state[i] != 0, bp.xr, bp.xf, np);
     zero0[i] = 0;  // the row counters of the neighbour build that follows
     zero1[i] = 0;
     zero2[i] = 0;
@@ -1745,10 +1761,12 @@ __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, int nsys,
 
 struct PermPtrs {
   const int* perm;
-  const double *pos, *vel, *omega;
-  double *pos_o, *vel_o, *omega_o;
-  const double *radius, *pmass, *acc, *racc;
-  double *radius_o, *pmass_o, *acc_o, *racc_o;
+  const Sphere* pos;
+  Sphere* pos_o;
+  const double *vel, *omega;
+  double *vel_o, *omega_o;
+  const double *pmass, *acc, *racc;
+  double *pmass_o, *acc_o, *racc_o;
   const int *gid, *fcell, *dgc;
   int *gid_o, *fcell_o, *dgc_o;
   const uint8_t *state, *phase, *wmask;
@@ -1764,12 +1782,11 @@ __global__ __launch_bounds__(kBS) void k_permute(int n, int S, PermPtrs p) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
   const int o = p.perm[i];
+  p.pos_o[i] = p.pos[o];
   for (int c = 0; c < 3; c++) {
-    p.pos_o[c * S + i] = p.pos[c * S + o];
     p.vel_o[c * S + i] = p.vel[c * S + o];
     p.omega_o[c * S + i] = p.omega[c * S + o];
   }
-  p.radius_o[i] = p.radius[o];
   p.pmass_o[i] = p.pmass[o];
   p.gid_o[i] = p.gid[o];
   p.fcell_o[i] = p.fcell[o];
@@ -1792,7 +1809,7 @@ __global__ __launch_bounds__(kBS) void k_permute(int n, int S, PermPtrs p) {
 }
 
 struct BuildPtrs {
-  const double *pos, *radius;
+  const Sphere* pos;
   const double* xr;             // [4*i + c]: x, y, z, radius (k_pack_xr), read per candidate
   const float4* xf;             // the same in single precision about GridDev::pf_c (radius
                                 // < 0: outside the prefilter's range)
@@ -1854,7 +1871,8 @@ __device__ __forceinline__ void own_row_hit(const GridDev& G, const BuildPtrs& b
   int ci, cj, ck, li, lj, lk;
   dg_decode(G, b.dgc[own], ci, cj, ck);
   if (dg_ghost(G, ci, cj, ck)) return;
-  const double xo[3] = {b.pos[own], b.pos[S + own], b.pos[2 * S + own]};
+  double xo[3];
+  load_sphere(b.pos, own, xo);
   int slo[3], shi[3];
   stencil_off(G, xo, slo, shi);
   dg_decode(G, b.dgc[oth], li, lj, lk);
@@ -1917,8 +1935,8 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
   const GridDev& G = BATCH ? Gs : G0;
   const int cbase = BATCH ? B.cell_off[s] : 0;
   const int g_r = BATCH ? B.rogue[2 * s] : b.flags[kFlagRogueGid];
-  const double x[3] = {b.pos[h], b.pos[S + h], b.pos[2 * S + h]};
-  const double r = b.radius[h];
+  double x[3];
+  const double r = load_sphere(b.pos, h, x);
   const int gh = b.gid[h];
   int f3[3];
   for (int d = 0; d < 3; d++) {
@@ -2048,15 +2066,16 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
 // nonexistent particle gets a position no cut-off reaches, so the walk
 // needs no state load; the hit path checks the state itself.
 template <bool BATCH>
-__global__ __launch_bounds__(kBS) void k_pack_xr(int n, int S, GridDev G0, const int* idx,
-                                                 const double* pos, const double* radius,
+__global__ __launch_bounds__(kBS) void k_pack_xr(int n, GridDev G0, const int* idx,
+                                                 const Sphere* pos,
                                                  const uint8_t* state, double* xr, float4* xf,
                                                  BatchDev B) {
   const int k = blockIdx.x * kBS + threadIdx.x;  // position in the search-cell order
   if (k >= n) return;
   const int i = idx ? idx[k] : k;
-  const double p[3] = {pos[i], pos[S + i], pos[2 * S + i]};
-  pack_candidate(BATCH ? B.gtab[B.sys[i]] : G0, p, radius[i], state[i] != 0, xr, xf, k);
+  double p[3];
+  const double r = load_sphere(pos, i, p);
+  pack_candidate(BATCH ? B.gtab[B.sys[i]] : G0, p, r, state[i] != 0, xr, xf, k);
 }
 
 // Own rows, one wavefront per search-grid cell.  The candidates of the 27
@@ -2128,10 +2147,11 @@ __global__ __launch_bounds__(kBS) void k_own_rows_wave(int S, GridDev G0, BuildP
     if (t < staged) {
       const uint8_t st = b.state[j];
       const int g = b.gid[j];
-      s_x[wv][t] = b.pos[j];
-      s_y[wv][t] = b.pos[S + j];
-      s_z[wv][t] = b.pos[2 * S + j];
-      s_r[wv][t] = b.radius[j];
+      const Sphere p = b.pos[j];
+      s_x[wv][t] = p.x;
+      s_y[wv][t] = p.y;
+      s_z[wv][t] = p.z;
+      s_r[wv][t] = p.w;
       int li, lj, lk;
       dg_decode(G, b.dgc[j], li, lj, lk);
       s_d[wv][t] = (lk * 1024 + lj) * 1024 + li;
@@ -2155,8 +2175,8 @@ __global__ __launch_bounds__(kBS) void k_own_rows_wave(int S, GridDev G0, BuildP
       if (lane == 0) b.own_cnt[h] = 0;
       continue;
     }
-    const double x[3] = {b.pos[h], b.pos[S + h], b.pos[2 * S + h]};
-    const double r = b.radius[h];
+    double x[3];
+    const double r = load_sphere(b.pos, h, x);
     int lo[3], hi[3];
     stencil_off(G, x, lo, hi);
     int cnt = 0;
@@ -2181,10 +2201,11 @@ __global__ __launch_bounds__(kBS) void k_own_rows_wave(int S, GridDev G0, BuildP
         if (t < total) {
           j = js;
           gj = b.state[j] != 0 ? b.gid[j] : INT_MIN;
-          xj = b.pos[j];
-          yj = b.pos[S + j];
-          zj = b.pos[2 * S + j];
-          rj = b.radius[j];
+          const Sphere p = b.pos[j];
+          xj = p.x;
+          yj = p.y;
+          zj = p.z;
+          rj = p.w;
           int li, lj, lk;
           dg_decode(G, b.dgc[j], li, lj, lk);
           dj = (lk * 1024 + lj) * 1024 + li;
@@ -2256,10 +2277,7 @@ __global__ __launch_bounds__(kBS) void k_own_rows_nsquare(int n, int S, double f
   double xi[3] = {0.0, 0.0, 0.0}, ri = 0.0;
   int gi = INT_MAX;
   if (home) {
-    xi[0] = b.pos[i];
-    xi[1] = b.pos[S + i];
-    xi[2] = b.pos[2 * S + i];
-    ri = b.radius[i];
+    ri = load_sphere(b.pos, i, xi);
     gi = b.gid[i];
   }
   int cnt = 0;
@@ -2269,10 +2287,11 @@ __global__ __launch_bounds__(kBS) void k_own_rows_nsquare(int n, int S, double f
   for (int base = 0; base < n; base += kBS) {
     const int j = base + threadIdx.x;
     if (j < n) {
-      s_x[threadIdx.x] = b.pos[j];
-      s_y[threadIdx.x] = b.pos[S + j];
-      s_z[threadIdx.x] = b.pos[2 * S + j];
-      s_r[threadIdx.x] = b.radius[j];
+      const Sphere p = b.pos[j];
+      s_x[threadIdx.x] = p.x;
+      s_y[threadIdx.x] = p.y;
+      s_z[threadIdx.x] = p.z;
+      s_r[threadIdx.x] = p.w;
       s_g[threadIdx.x] = b.state[j] != 0 ? b.gid[j] : INT_MIN;
     } else {
       s_g[threadIdx.x] = INT_MIN;
@@ -2461,9 +2480,8 @@ __global__ __launch_bounds__(kBS) void k_sort_in(int n, const int* pair_base,
 // DELETE_PARTICLE of rogue particles (mass_outflow_dem.f:201-280)
 template <bool BATCH = false>
 __global__ __launch_bounds__(kBS) void k_delete_rogue(int n, int S, GridDev G0, const int* dgc,
-                                                      uint8_t* state, uint8_t* wmask, double* pos,
-                                                      double* vel, double* omega, double* radius,
-                                                      BatchDev B) {
+                                                      uint8_t* state, uint8_t* wmask, Sphere* pos,
+                                                      double* vel, double* omega, BatchDev B) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n || state[i] != 1) return;
   const GridDev& G = sys_grid<BATCH>(G0, B, BATCH ? B.sys[i] : 0);
@@ -2472,17 +2490,17 @@ __global__ __launch_bounds__(kBS) void k_delete_rogue(int n, int S, GridDev G0, 
   if (!dg_ghost(G, ci, cj, ck)) return;
   state[i] = 0;
   wmask[i] = 0;
+  pos[i] = Sphere{0.0, 0.0, 0.0, 0.0};
   for (int c = 0; c < 3; c++) {
-    pos[c * S + i] = 0.0;
     vel[c * S + i] = 0.0;
     omega[c * S + i] = 0.0;
   }
-  radius[i] = 0.0;
 }
 
 // ------------------------------------------------- DEM inlets / outlets
 struct BcPtrs {
-  double *pos, *vel, *omega, *radius, *pmass;
+  Sphere* pos;
+  double *vel, *omega, *pmass;
   const int *gid, *dgc;
   uint8_t *state, *wmask;
   const uint8_t* phase;
@@ -2523,9 +2541,8 @@ __device__ inline bool particle_bcs(const BcPtrs& b, int i) {
   const int S = b.S, dc = b.dgc[i];
   int st = st0;
   double x[3], v[3];
-  load3(b.pos, S, i, x);
+  const double r = load_sphere(b.pos, i, x);
   load3(b.vel, S, i, v);
-  const double r = b.radius[i];
   bool vset = false;
   for (int k = 0; k < b.nbc; k++) {
     const BcDev& B = b.bcs[k];
@@ -2557,10 +2574,9 @@ __device__ inline bool particle_bcs(const BcPtrs& b, int i) {
   }
   if (st == kNonexistent) {
     const double z[3] = {0.0, 0.0, 0.0};
-    store3(b.pos, S, i, z);
+    b.pos[i] = Sphere{0.0, 0.0, 0.0, 0.0};
     store3(b.vel, S, i, z);
     store3(b.omega, S, i, z);
-    b.radius[i] = 0.0;
     b.pmass[i] = 3.4028234663852886e38;  // HUGE(0.0) as DELETE_PARTICLE sets it
     b.wmask[i] = 0;
     b.state[i] = kNonexistent;
@@ -2593,7 +2609,8 @@ __global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
 }
 
 struct SeedPtrs {
-  double *pos, *vel, *omega, *radius, *pmass;
+  Sphere* pos;
+  double *vel, *omega, *pmass;
   int *dgc, *fcell;
   uint8_t *state, *phase, *wmask;
   const int* slot_of_gid;
@@ -2607,10 +2624,9 @@ __global__ __launch_bounds__(kBS) void k_seed(int ns, const SeedDev* sd, SeedPtr
   const SeedDev d = sd[k];
   const int i = p.slot_of_gid[d.gid], S = p.S;
   const double z[3] = {0.0, 0.0, 0.0};
-  store3(p.pos, S, i, d.pos);
+  p.pos[i] = Sphere{d.pos[0], d.pos[1], d.pos[2], d.radius};
   store3(p.vel, S, i, d.vel);
   store3(p.omega, S, i, z);
-  p.radius[i] = d.radius;
   p.pmass[i] = d.pmass;
   p.dgc[i] = d.dgc;
   p.fcell[i] = d.fcell;
@@ -2643,10 +2659,11 @@ __global__ __launch_bounds__(kBS) void k_locate(int n, int S, FaceGrid f, const 
     fcell[i] = -1;
     return;
   }
-  double x0, x1;
-  const int I = locate_cell(xe, f.n[0], f.lo[0], f.hi[0], f.inv[0], rm.pos[i], x0, x1);
-  const int J = locate_cell(yn, f.n[1], f.lo[1], f.hi[1], f.inv[1], rm.pos[S + i], x0, x1);
-  const int K = locate_cell(zt, f.n[2], f.lo[2], f.hi[2], f.inv[2], rm.pos[2 * S + i], x0, x1);
+  double x[3], x0, x1;
+  load_sphere(rm.pos, i, x);
+  const int I = locate_cell(xe, f.n[0], f.lo[0], f.hi[0], f.inv[0], x[0], x0, x1);
+  const int J = locate_cell(yn, f.n[1], f.lo[1], f.hi[1], f.inv[1], x[1], x0, x1);
+  const int K = locate_cell(zt, f.n[2], f.lo[2], f.hi[2], f.inv[2], x[2], x0, x1);
   const bool in = I && J && K;
   fcell[i] = in ? pack_ijk(I, J, K) : -1;
   if (kDelete && !in) remove_outside(rm, S, i);
@@ -2654,8 +2671,8 @@ __global__ __launch_bounds__(kBS) void k_locate(int n, int S, FaceGrid f, const 
 
 // PIC counts; deletes particles outside the fluid grid (particles_in_cell.f:175-184)
 __global__ __launch_bounds__(kBS) void k_pic_count(int n, int S, int ni, int nj, const int* fcell,
-                                                   uint8_t* state, uint8_t* wmask, double* pos,
-                                                   double* vel, double* omega, double* radius,
+                                                   uint8_t* state, uint8_t* wmask, Sphere* pos,
+                                                   double* vel, double* omega,
                                                    int* cnt, int* flags) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n || state[i] == 0) return;
@@ -2663,12 +2680,11 @@ __global__ __launch_bounds__(kBS) void k_pic_count(int n, int S, int ni, int nj,
   if (pc < 0) {
     state[i] = 0;
     wmask[i] = 0;
+    pos[i] = Sphere{0.0, 0.0, 0.0, 0.0};
     for (int d = 0; d < 3; d++) {
-      pos[d * S + i] = 0.0;
       vel[d * S + i] = 0.0;
       omega[d * S + i] = 0.0;
     }
-    radius[i] = 0.0;
     atomicAdd(&flags[kFlagOutOfDomain], 1);
     return;
   }
@@ -2714,7 +2730,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_nodes(int imax, int jmax, int k
                                                        const double* xe, const double* yn,
                                                        const double* zt, const uint8_t* fluid,
                                                        const int* off, const int* pic,
-                                                       const double* pos, const double* pmass,
+                                                       const Sphere* pos, const double* pmass,
                                                        const uint8_t* phase, double* rops_node,
                                                        int ncell) {
   const int t = blockIdx.x * kBS + threadIdx.x;
@@ -2737,10 +2753,11 @@ __global__ __launch_bounds__(kBS) void k_deposit_nodes(int imax, int jmax, int k
         const double dxx = xe[ci] - x0, dyy = yn[cj] - y0, dzz = zt[ck] - z0;
         for (int q = s; q < e; q++) {
           const int p = pic[q];
-          double zx = pos[p] - x0, zy = pos[S + p] - y0;
+          const Sphere sp = pos[p];
+          double zx = sp.x - x0, zy = sp.y - y0;
           zx = zx / dxx;
           zy = zy / dyy;
-          double zz = pos[2 * S + p] - z0;
+          double zz = sp.z - z0;
           zz = zz / dzz;
           // this node is corner (1-a, 1-b, 1-c) of the cell
           const double xv = a ? 1.0 - zx : zx;
@@ -2774,7 +2791,7 @@ __global__ __launch_bounds__(kBS) void k_gas_fgp(DevParams P, StepPtrs a, double
     const int c = lin_ijk(ci, cj, ck, P.ni, P.nj);
     if (a.fluid[c]) {
       double pos[3], vel[3];
-      load3(a.pos, S, i, pos);
+      const double ri = load_sphere(a.pos, i, pos);
       load3(a.vel, S, i, vel);
       const double x0 = a.xe[ci - 1], y0 = a.yn[cj - 1], z0 = a.zt[ck - 1];
       const double dxx = a.xe[ci] - x0, dyy = a.yn[cj] - y0, dzz = a.zt[ck] - z0;
@@ -2796,7 +2813,7 @@ __global__ __launch_bounds__(kBS) void k_gas_fgp(DevParams P, StepPtrs a, double
       const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
       const double vrel = sqrt(dot3(vs, vs));
       const double f = drag_fgp_fp64(P.drag_type, a.ep_g[c], P.mu_g0, P.ro_g0, vrel,
-                                     2.0 * a.radius[i], sphere_volume(a.radius[i]));
+                                     2.0 * ri, sphere_volume(ri));
       r[0] = zx;
       r[1] = zy;
       r[2] = zz;
@@ -2902,7 +2919,7 @@ __global__ __launch_bounds__(kBS) void k_gas_filter(DevParams P, StepPtrs a, con
     const int c0 = lin_ijk(ci, cj, ck, P.ni, P.nj);
     const int S = P.stride;
     double pos[3], vel[3];
-    load3(a.pos, S, i, pos);
+    const double ri = load_sphere(a.pos, i, pos);
     load3(a.vel, S, i, vel);
     const bool filt = P.interp_on && filter_scheme(P.interp);
     double lepg = 0.0, velfp[3] = {0.0, 0.0, 0.0};
@@ -2919,8 +2936,8 @@ __global__ __launch_bounds__(kBS) void k_gas_filter(DevParams P, StepPtrs a, con
     if (lepg < 1.0e-6) lepg = a.ep_g[c0];
     const double vs[3] = {velfp[0] - vel[0], velfp[1] - vel[1], velfp[2] - vel[2]};
     const double vrel = sqrt(dot3(vs, vs));
-    const double f = drag_fgp_fp64(P.drag_type, lepg, P.mu_g0, P.ro_g0, vrel, 2.0 * a.radius[i],
-                                   sphere_volume(a.radius[i]));
+    const double f = drag_fgp_fp64(P.drag_type, lepg, P.mu_g0, P.ro_g0, vrel, 2.0 * ri,
+                                   sphere_volume(ri));
     if (a.f_gp) a.f_gp[a.gid[i]] = f;  // F_GP(NP) for explicit coupling
     const double lbm[3] = {f * vel[0], f * vel[1], f * vel[2]};
     auto add = [&](int I, int J, int K, double w) {
@@ -2972,7 +2989,7 @@ __global__ __launch_bounds__(kBS) void k_drag_fc(DevParams P, StepPtrs a) {
   }
   const int S = P.stride;
   double pos[3], vel[3];
-  load3(a.pos, S, i, pos);
+  const double ri = load_sphere(a.pos, i, pos);
   load3(a.vel, S, i, vel);
   double velfp[3] = {0.0, 0.0, 0.0}, lpf[3] = {0.0, 0.0, 0.0};
   if (P.interp_on && filter_scheme(P.interp)) {
@@ -2985,7 +3002,7 @@ __global__ __launch_bounds__(kBS) void k_drag_fc(DevParams P, StepPtrs a) {
     for (int d = 0; d < 3; d++) velfp[d] = a.ugc[3 * c0 + d];
     for (int d = 0; d < 3; d++) lpf[d] = a.p_force[3 * c0 + d];
   }
-  const double f = a.f_gp[g], pv = sphere_volume(a.radius[i]);
+  const double f = a.f_gp[g], pv = sphere_volume(ri);
   double out[3];
   for (int d = 0; d < 3; d++) out[d] = f * (velfp[d] - vel[d]);
   for (int d = 0; d < 3; d++) out[d] = out[d] + lpf[d] * pv;
@@ -3056,27 +3073,22 @@ struct FieldPtrs {
   int* rm_cnt_clear;
   const int* rm_list;
   uint8_t* state;
-  double* radius;
 };
 
 // Completes the removals the fused step queued (particles that left the
-// fluid grid): NONEXISTENT state and zero radius.  Grid-stride over the
-// queue; any thread may run it.
+// fluid grid): NONEXISTENT state.  Grid-stride over the queue; any thread
+// may run it.
 __device__ __forceinline__ void apply_removals(const int* cnt, const int* list, uint8_t* state,
-                                               double* radius, int tid, int nthreads) {
+                                               int tid, int nthreads) {
   const int m = *cnt;
-  for (int q = tid; q < m; q += nthreads) {
-    const int i = list[q];
-    state[i] = 0;
-    radius[i] = 0.0;
-  }
+  for (int q = tid; q < m; q += nthreads) state[list[q]] = 0;
 }
 // The same as a kernel of its own, ahead of a neighbour rebuild (which
 // reorders the slots the queue names); one workgroup, which then empties
 // the queue.
 __global__ __launch_bounds__(kBS) void k_apply_removals(int* cnt, const int* list,
-                                                        uint8_t* state, double* radius) {
-  apply_removals(cnt, list, state, radius, threadIdx.x, kBS);
+                                                        uint8_t* state) {
+  apply_removals(cnt, list, state, threadIdx.x, kBS);
   __syncthreads();
   if (threadIdx.x == 0) *cnt = 0;
 }
@@ -3103,7 +3115,7 @@ __global__ __launch_bounds__(kBS) void k_cell_fields(int imax, int jmax, int kma
   __shared__ double s_dens[kNK][kNI][kNJ];
   const int ncell = ni * nj * nk, plane = nj * ni;
   if (FIXED && f.rm_cnt) {
-    apply_removals(f.rm_cnt, f.rm_list, f.state, f.radius, blockIdx.x * kBS + threadIdx.x,
+    apply_removals(f.rm_cnt, f.rm_list, f.state, blockIdx.x * kBS + threadIdx.x,
                    gridDim.x * kBS);
     if (blockIdx.x == 0 && threadIdx.x == 0) *f.rm_cnt_clear = 0;
   }
@@ -3311,17 +3323,25 @@ __global__ __launch_bounds__(kBS) void k_pg_grad(int ni, int nj, int nk, const d
 // copies takes them to the host.  A thread reads its slot coalesced and
 // writes 8 bytes to each plane at its id.
 __global__ __launch_bounds__(kBS) void k_export(int nslots, int n, int S, const int* gid,
-                                                const uint8_t* state, const double* pos,
+                                                const uint8_t* state, const Sphere* pos,
                                                 const double* vel, const double* omega,
                                                 bool want_state, double* out) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= nslots) return;
   const int g = gid[i];
   if (g >= n) return;  // a slot that fills an ensemble member's range up to a multiple of 64
-  const double* src[3] = {pos, vel, omega};
+  const double* src[2] = {vel, omega};
   double* o = out + g;
+  if (pos) {
+    double x[3];
+    load_sphere(pos, i, x);
+    for (int c = 0; c < 3; c++) {
+      *o = x[c];
+      o += n;
+    }
+  }
 #pragma unroll
-  for (int a = 0; a < 3; a++)
+  for (int a = 0; a < 2; a++)
     if (src[a])
       for (int c = 0; c < 3; c++) {
         *o = src[a][(size_t)c * S + i];
@@ -3336,14 +3356,12 @@ __global__ __launch_bounds__(kBS) void k_export(int nslots, int n, int S, const 
 // nonexistent with zero radius and state (slot order = global-id order
 // before the first sort).
 __global__ __launch_bounds__(kBS) void k_set_holes(int n, const int8_t* st, uint8_t* state,
-                                                   double* radius, int S, double* pos,
-                                                   double* vel, double* omega) {
+                                                   int S, Sphere* pos, double* vel, double* omega) {
   const int q = blockIdx.x * kBS + threadIdx.x;
   if (q >= n || st[q] != 0) return;
   state[q] = 0;
-  radius[q] = 0.0;
+  pos[q] = Sphere{0.0, 0.0, 0.0, 0.0};
   for (int d = 0; d < 3; d++) {
-    pos[d * S + q] = 0.0;
     vel[d * S + q] = 0.0;
     omega[d * S + q] = 0.0;
   }

@@ -75,9 +75,10 @@ struct mfixdem_handle {
   int n = 0, stride = 0;
   int cur = 0, pcur = 0, tw = 0, lt = 0;
   // particles (cur / tw twins)
-  double *pos[2]{}, *vel[2]{}, *omega[2]{};
+  Sphere* pos[2]{};  // position and radius
+  double *vel[2]{}, *omega[2]{};
   double* xr_pack = nullptr;  // (x, y, z, radius) per particle, written before each row build
-  double *radius[2]{}, *pmass[2]{};
+  double* pmass[2]{};
   double *acc[2]{}, *racc[2]{};
   int *gid[2]{}, *fcell[2]{}, *dgc[2]{};
   uint8_t *state[2]{}, *phase[2]{}, *wmask[2]{};
@@ -334,7 +335,7 @@ StepPtrs step_ptrs(mfixdem_handle* h) {
   const int c = h->cur, t = h->tw, l = h->lt, p = h->pcur;
   a.pos = h->pos[c]; a.vel = h->vel[c]; a.omega = h->omega[c];
   a.pos_o = h->pos[1 - c]; a.vel_o = h->vel[1 - c]; a.omega_o = h->omega[1 - c];
-  a.radius = h->radius[t]; a.pmass = h->pmass[t];
+  a.pmass = h->pmass[t];
   a.gid = h->gid[t]; a.state = h->state[t]; a.phase = h->phase[t]; a.dgc = h->dgc[t];
   a.cell_fmask = h->cell_fmask;
   a.fac = h->fac; a.dg_foff = h->dg_foff; a.dg_fids = h->dg_fids;
@@ -551,15 +552,13 @@ int32_t do_bin(mfixdem_handle* h) {
   const int nf = h->n_fine;
   BinPack bp{};
   bp.G = h->G;
-  bp.S = S;
   bp.pos = h->pos[c];
-  bp.radius = h->radius[t];
   bp.state = h->state[t];
   bp.xr = h->xr_pack;
   bp.xf = reinterpret_cast<float4*>(h->stage);
   auto bin = [&](auto many) -> int32_t {
     constexpr bool kB = decltype(many)::value;
-    hipLaunchKernelGGL(k_bin_count<kB>, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G,
+    hipLaunchKernelGGL(k_bin_count<kB>, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->G,
                        h->pos[c], h->state[t], h->gid[t], h->dgc[t], h->fine_rank, h->fine_cnt,
                        nf, h->place, h->flags, h->B);
     HIPOK(hipGetLastError());
@@ -578,9 +577,9 @@ int32_t do_bin(mfixdem_handle* h) {
   p.perm = h->vals[1];
   p.pos = h->pos[c]; p.vel = h->vel[c]; p.omega = h->omega[c];
   p.pos_o = h->pos[1 - c]; p.vel_o = h->vel[1 - c]; p.omega_o = h->omega[1 - c];
-  p.radius = h->radius[t]; p.pmass = h->pmass[t];
+  p.pmass = h->pmass[t];
   p.acc = h->acc[t]; p.racc = h->racc[t];
-  p.radius_o = h->radius[1 - t]; p.pmass_o = h->pmass[1 - t];
+  p.pmass_o = h->pmass[1 - t];
   p.acc_o = h->acc[1 - t]; p.racc_o = h->racc[1 - t];
   p.gid = h->gid[t]; p.fcell = h->fcell[t]; p.dgc = h->dgc[t];
   p.gid_o = h->gid[1 - t]; p.fcell_o = h->fcell[1 - t]; p.dgc_o = h->dgc[1 - t];
@@ -651,7 +650,7 @@ int32_t do_neighbour(mfixdem_handle* h) {
   if (!h->binned) CHECKRC(do_bin(h));
   const int n = h->n, S = h->stride, t = h->tw, c = h->cur;
   BuildPtrs b{};
-  b.pos = h->pos[c]; b.radius = h->radius[t]; b.gid = h->gid[t]; b.dgc = h->dgc[t];
+  b.pos = h->pos[c]; b.gid = h->gid[t]; b.dgc = h->dgc[t];
   b.xr = h->xr_pack;
   // the single-precision copy for the walk's prefilter lives in the export
   // stage (at least 3 doubles per slot), which no call uses during a rebuild
@@ -727,8 +726,8 @@ int32_t do_neighbour(mfixdem_handle* h) {
       }
       if (!packed) {
         auto pack = h->nsys > 1 ? k_pack_xr<true> : k_pack_xr<false>;
-        hipLaunchKernelGGL(pack, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->G, b.idx,
-                           b.pos, b.radius, b.state, h->xr_pack,
+        hipLaunchKernelGGL(pack, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->G, b.idx,
+                           b.pos, b.state, h->xr_pack,
                            reinterpret_cast<float4*>(h->stage), h->B);
       }
       auto rows = [&](auto lanes) {
@@ -826,11 +825,11 @@ int32_t do_neighbour(mfixdem_handle* h) {
     if (h->nsys > 1)
       hipLaunchKernelGGL((k_delete_rogue<true>), dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S,
                          h->G, h->dgc[t], h->state[t], h->wmask[t], h->pos[c], h->vel[c],
-                         h->omega[c], h->radius[t], h->B);
+                         h->omega[c], h->B);
     else
       hipLaunchKernelGGL((k_delete_rogue<false>), dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S,
                          h->G, h->dgc[t], h->state[t], h->wmask[t], h->pos[c], h->vel[c],
-                         h->omega[c], h->radius[t], h->B);
+                         h->omega[c], h->B);
     HIPOK(hipGetLastError());
     h->st.rogue_deleted += fl[kFlagRogueCount];
   }
@@ -845,8 +844,7 @@ int32_t do_pic_lists(mfixdem_handle* h) {
   CHECKRC(fill_i32(h->stream, h->pic_cnt, nc, 0));
   hipLaunchKernelGGL(k_pic_count, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, S, h->S.ni, h->S.nj,
                      h->fcell[t],
-                     h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->radius[t],
-                     h->pic_cnt, h->flags);
+                     h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->pic_cnt, h->flags);
   HIPOK(hipGetLastError());
   CHECKRC(scan_i32(h, h->pic_cnt, h->pic_off, nc));
   CHECKRC(fill_i32(h->stream, h->pic_cur, nc, 0));
@@ -871,7 +869,6 @@ FieldPtrs field_ptrs(mfixdem_handle* h) {
     f.rm_cnt_clear = h->rm_cnt + (1 - h->fb);
     f.rm_list = h->rm_list;
     f.state = h->state[h->tw];
-    f.radius = h->radius[h->tw];
   }
   return f;
 }
@@ -905,8 +902,7 @@ int32_t do_cell_fields(mfixdem_handle* h, bool fixed) {
 
 Removal removal(mfixdem_handle* h) {
   const int t = h->tw, c = h->cur;
-  return Removal{h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->radius[t],
-                 h->flags};
+  return Removal{h->state[t], h->wmask[t], h->pos[c], h->vel[c], h->omega[c], h->flags};
 }
 
 // the fluid cell of every particle, those outside the grid deleted or not
@@ -945,7 +941,7 @@ int32_t deposit_current(mfixdem_handle* h) {
   const Removal rm = removal(h);
   if (h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012) {
     hipLaunchKernelGGL(k_deposit_filter, dim3(nblk(h->n)), dim3(kBS), 0, h->stream, P,
-                       nullptr, h->pos[h->cur], h->radius[h->tw], h->phase[h->tw],
+                       nullptr, h->pos[h->cur], h->phase[h->tw],
                        h->state[h->tw], h->fcell[h->tw], h->xe, h->yn, h->zt, h->csz,
                        h->rops_fix[h->fb], rm);
     HIPOK(hipGetLastError());
@@ -1005,7 +1001,7 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
   const int c = h->cur, t = h->tw;
   BcPtrs b{};
   b.pos = h->pos[c]; b.vel = h->vel[c]; b.omega = h->omega[c];
-  b.radius = h->radius[t]; b.pmass = h->pmass[t];
+  b.pmass = h->pmass[t];
   b.gid = h->gid[t]; b.dgc = h->dgc[t]; b.state = h->state[t]; b.wmask = h->wmask[t];
   b.phase = h->phase[t];
   b.bcs = h->d_bcs; b.nbc = (int)D.b.size(); b.n = n; b.S = h->stride;
@@ -1025,7 +1021,7 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn) {
     std::memcpy(seeds, D.seeds.data(), sizeof(SeedDev) * ns);
     SeedPtrs sp{};
     sp.pos = h->pos[c]; sp.vel = h->vel[c]; sp.omega = h->omega[c];
-    sp.radius = h->radius[t]; sp.pmass = h->pmass[t];
+    sp.pmass = h->pmass[t];
     sp.dgc = h->dgc[t]; sp.fcell = h->fcell[t];
     sp.state = h->state[t]; sp.phase = h->phase[t]; sp.wmask = h->wmask[t];
     sp.slot_of_gid = h->slot_of_gid; sp.S = h->stride;
@@ -1072,7 +1068,7 @@ int32_t one_step(mfixdem_handle* h, int32_t nn) {
     t_begin(h);
     if (fused_dep(h)) {  // the rebuild reorders the slots the removal queue names
       hipLaunchKernelGGL(k_apply_removals, dim3(1), dim3(kBS), 0, h->stream, h->rm_cnt + h->fb,
-                         h->rm_list, h->state[h->tw], h->radius[h->tw]);
+                         h->rm_list, h->state[h->tw]);
       HIPOK(hipGetLastError());
     }
     CHECKRC(do_bin(h));
@@ -1270,7 +1266,8 @@ int32_t upload_setup(mfixdem_handle* h) {
 // particles set, NONEXISTENT for the rest of the system's slots.
 int32_t upload_ensemble(mfixdem_handle* h) {
   const int64_t N = h->n, S = h->stride;
-  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38);
+  std::vector<Sphere> X(S, Sphere{0.0, 0.0, 0.0, 0.0});
+  std::vector<double> M(S, 3.4028234663852886e38);
   std::vector<int> G(S, 0), FC(S, -1), DG(S, 0);
   std::vector<uint8_t> ST(S, 0), PH(S, 0), WM(S, 0);
   for (int s = 0; s < h->nsys; s++) {
@@ -1278,7 +1275,7 @@ int32_t upload_ensemble(mfixdem_handle* h) {
     for (int q = off; q < h->sys_off[s + 1]; q++) G[q] = q - off;
     for (int q = off; q < off + h->sys_n[s]; q++) {
       const double r = h->st_r[q];
-      R[q] = r;
+      X[q] = Sphere{h->st_pos[q], h->st_pos[S + q], h->st_pos[2 * S + q], r};
       M[q] = (4.0 / 3.0) * kPi * (r * r * r) * h->st_rho[q];
       PH[q] = (uint8_t)(h->st_phase[q] - 1);
       ST[q] = 1;
@@ -1286,10 +1283,9 @@ int32_t upload_ensemble(mfixdem_handle* h) {
   }
   h->cur = h->pcur = h->tw = h->lt = 0;
   CHECKRC(reset_deposit(h));
-  HIPOK(hipMemcpy(h->pos[0], h->st_pos.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
+  HIPOK(hipMemcpy(h->pos[0], X.data(), sizeof(Sphere) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->vel[0], h->st_vel.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->omega[0], h->st_om.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->radius[0], R.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->pmass[0], M.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->gid[0], G.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->fcell[0], FC.data(), sizeof(int) * S, hipMemcpyHostToDevice));
@@ -1321,7 +1317,7 @@ int32_t upload_ensemble(mfixdem_handle* h) {
 template <class F>
 void for_each_buffer(mfixdem_handle* h, F f) {
   for (int b = 0; b < 2; b++) {
-    f(h->pos[b]); f(h->vel[b]); f(h->omega[b]); f(h->radius[b]);
+    f(h->pos[b]); f(h->vel[b]); f(h->omega[b]);
     f(h->pmass[b]); f(h->acc[b]);
     f(h->racc[b]); f(h->gid[b]); f(h->fcell[b]); f(h->dgc[b]);
     f(h->state[b]); f(h->phase[b]); f(h->wmask[b]); f(h->wfid[b]); f(h->wpft[b]);
@@ -1412,7 +1408,7 @@ int32_t alloc_buffers(mfixdem_handle* h) {
     return fail(MFIXDEM_ERR_HIP);
   Pieces a;
   for (int b = 0; b < 2; b++)
-    a.add(&h->pos[b], 3 * S).add(&h->vel[b], 3 * S).add(&h->omega[b], 3 * S).add(&h->radius[b], S)
+    a.add(&h->pos[b], S).add(&h->vel[b], 3 * S).add(&h->omega[b], 3 * S)
         .add(&h->pmass[b], S).add(&h->acc[b], 3 * S).add(&h->racc[b], 3 * S).add(&h->gid[b], S)
         .add(&h->fcell[b], S).add(&h->dgc[b], S).add(&h->state[b], S).add(&h->phase[b], S)
         .add(&h->wmask[b], S).add(&h->wfid[b], kWallSlots * S)
@@ -1588,19 +1584,19 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
   if (h && h->nsys > 1) return MFIXDEM_ERR_ARG;  // single-system call
   if (!h || n < 0 || n > h->n || ld < n || !pos || !radius || !ro_sol) return MFIXDEM_ERR_ARG;
   const int64_t N = h->n, S = h->stride;
-  std::vector<double> P3((size_t)3 * S, 0.0), V3((size_t)3 * S, 0.0), W3((size_t)3 * S, 0.0);
-  std::vector<double> R(S, 0.0), M(S, 3.4028234663852886e38);
+  std::vector<double> V3((size_t)3 * S, 0.0), W3((size_t)3 * S, 0.0);
+  std::vector<Sphere> X(S, Sphere{0.0, 0.0, 0.0, 0.0});
+  std::vector<double> M(S, 3.4028234663852886e38);
   std::vector<int> G(S, 0), FC(S, -1), DG(S, 0);
   std::vector<uint8_t> ST(S, 0), PH(S, 0), WM(S, 0);
   for (int64_t q = 0; q < N; q++) G[q] = (int)q;
   for (int64_t q = 0; q < n; q++) {
     for (int c = 0; c < 3; c++) {
-      P3[c * S + q] = pos[c * ld + q];
       V3[c * S + q] = vel ? vel[c * ld + q] : 0.0;
       W3[c * S + q] = omega ? omega[c * ld + q] : 0.0;
     }
     const double r = radius[q];
-    R[q] = r;
+    X[q] = Sphere{pos[q], pos[ld + q], pos[2 * ld + q], r};
     // make_arrays_des.f:288-291
     M[q] = (4.0 / 3.0) * kPi * (r * r * r) * ro_sol[q];
     const int ph = phase ? phase[q] - 1 : 0;
@@ -1628,10 +1624,9 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
   HIPOK(sync_stream(h));  // steps already queued still use the buffers
   h->cur = h->pcur = h->tw = h->lt = 0;
   CHECKRC(reset_deposit(h));
-  HIPOK(hipMemcpy(h->pos[0], P3.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
+  HIPOK(hipMemcpy(h->pos[0], X.data(), sizeof(Sphere) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->vel[0], V3.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->omega[0], W3.data(), sizeof(double) * 3 * S, hipMemcpyHostToDevice));
-  HIPOK(hipMemcpy(h->radius[0], R.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->pmass[0], M.data(), sizeof(double) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->gid[0], G.data(), sizeof(int) * S, hipMemcpyHostToDevice));
   HIPOK(hipMemcpy(h->fcell[0], FC.data(), sizeof(int) * S, hipMemcpyHostToDevice));
@@ -1676,7 +1671,7 @@ int32_t mfixdem_set_particle_state(mfixdem_handle* h, const int8_t* state, int64
   HIPOK(sync_stream(h));
   HIPOK(hipMemcpy(h->stage, state, (size_t)n, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_set_holes, dim3(nblk(n)), dim3(kBS), 0, h->stream, (int)n,
-                     (const int8_t*)h->stage, h->state[0], h->radius[0], h->stride, h->pos[0],
+                     (const int8_t*)h->stage, h->state[0], h->stride, h->pos[0],
                      h->vel[0], h->omega[0]);
   HIPOK(hipGetLastError());
   HIPOK(sync_stream(h));
