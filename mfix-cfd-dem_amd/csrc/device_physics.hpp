@@ -95,48 +95,63 @@ __device__ __forceinline__ void cross3f(const float x[3], const float y[3], floa
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float fdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 
+// A pair seen from particle p of it, with partner j.  The reference forms it
+// with p as L where p owns the pair (owner) and as I otherwise: x_I - x_L,
+// v_L - v_I, the normal, the slip and the tangential history then all have the
+// other sign, and every operation of the law rounds the same for negated
+// operands or leaves two terms whose order does not matter.  Only what is not
+// symmetric in L and I (the two lever arms, the phase pair) is exchanged, 4
+// values instead of 22.  With the shared reciprocals (div_by) a step took 15.0
+// us instead of 15.4 at 20,000 settled spheres, 64.4 instead of 66.2 at 301,057.
 struct PairIn {
-  double xL[3], xI[3], vL[3], vI[3], wL[3], wI[3];
-  double rL, rI, mL, mI;
+  double xp[3], xj[3], vp[3], vj[3], wp[3], wj[3];
+  double rp, rj, mp, mj;
   int phL, phI;
+  bool owner;
 };
 struct PairOut {
-  double fct[3];    // FN + FT on L (I receives -fct)
-  double tl[3];     // torque increment of L (DIST_CL * n x FT)
-  double ti[3];     // torque increment of I (DIST_CI * n x FT)
-  double pft[3];    // new tangential history
+  double f[3];      // FN + FT on p
+  double t[3];      // torque increment of p (DIST_CL or DIST_CI * n x FT)
+  double pft[3];    // new tangential history, in p's orientation as the old one
 };
 
-// CALC_FORCE_DEM pair body (calc_force_dem.f:210-412) with CFRELVEL
-// (cfrelvel.f:54-77).  Returns 0 no contact, 1 contact, 2 zero distance.
+// a / b for several a: y is 1 / b correctly rounded, and one residual step
+// then gives the correctly rounded quotient (Markstein, IBM J. Res. Dev. 34,
+// 1990), in 3 operations instead of the 10 of a division of its own.  For |a|
+// above 1e-290 and b and 1 / b in the normal range.
+__device__ __forceinline__ double div_by(double a, double b, double y) {
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// CALC_FORCE_DEM pair body (calc_force_dem.f:263-412) with CFRELVEL
+// (cfrelvel.f:54-77) of a pair in contact (pair_touches).
 template <class PT>
-__device__ __forceinline__ int pair_force_fp64(const PT& P, const PairIn& a,
-                                               const double pft_in[3], PairOut& o) {
-  const double r_lm = a.rL + a.rI;
-  double dist[3] = {a.xI[0] - a.xL[0], a.xI[1] - a.xL[1], a.xI[2] - a.xL[2]};
-  double dm = dot3(dist, dist);
-  const double rs = r_lm - kSmall;
-  if (dm > rs * rs) return 0;
-  if (dm == 0.0) return 2;
-  dm = sqrt(dm);
+__device__ __forceinline__ void pair_force_fp64(const PT& P, const PairIn& a,
+                                                const double pft_in[3], PairOut& o) {
+  const double dist[3] = {a.xj[0] - a.xp[0], a.xj[1] - a.xp[1], a.xj[2] - a.xp[2]};
+  const double dm = sqrt(dot3(dist, dist));
+  const double rdm = 1.0 / dm;  // and 1 / (2 dm) is half of it, exactly
   double nrm[3];
-  for (int c = 0; c < 3; c++) nrm[c] = dist[c] / dm;
-  const double ovl = r_lm - dm;
+  for (int c = 0; c < 3; c++) nrm[c] = div_by(dist[c], dm, rdm);
+  const double ovl = a.rp + a.rj - dm;
   double vrel[3];
-  for (int c = 0; c < 3; c++) vrel[c] = a.vL[c] - a.vI[c];
-  const double dcl = (dm * dm + a.rL * a.rL - a.rI * a.rI) / (2.0 * dm);
+  for (int c = 0; c < 3; c++) vrel[c] = a.vp[c] - a.vj[c];
+  const double rL = a.owner ? a.rp : a.rj, rI = a.owner ? a.rj : a.rp;
+  const double dcl = div_by(dm * dm + rL * rL - rI * rI, 2.0 * dm, 0.5 * rdm);
   const double dci = dm - dcl;
+  const double dcp = a.owner ? dcl : dci, dcj = a.owner ? dci : dcl;
   double osum[3], vrot[3];
-  for (int c = 0; c < 3; c++) osum[c] = a.wL[c] * dcl + a.wI[c] * dci;
+  for (int c = 0; c < 3; c++) osum[c] = a.wp[c] * dcp + a.wj[c] * dcj;
   cross3(osum, nrm, vrot);
   for (int c = 0; c < 3; c++) vrel[c] = vrel[c] + vrot[c];
   const double vrn = dot3(vrel, nrm);
   double vs[3];
   for (int c = 0; c < 3; c++) vs[c] = vrel[c] - vrn * nrm[c];
-  const double reff = (a.rL * a.rI) / (a.rL + a.rI);
-  const double meff = (a.mL * a.mI) / (a.mL + a.mI);
+  const double meff = (a.mp * a.mj) / (a.mp + a.mj);
   double kn, kt, etan, etat;
   if (P.hertz) {
+    const double reff = (a.rp * a.rj) / (a.rp + a.rj);
     double sqo = sqrt(ovl);
     kn = P.hkn[a.phL][a.phI] * sqo * sqrt(reff);
     kt = P.hkt[a.phL][a.phI] * sqo * sqrt(reff);
@@ -159,7 +174,8 @@ __device__ __forceinline__ int pair_force_fp64(const PT& P, const PairIn& a,
     const double fnmd = P.mew * sqrt(dot3(fn, fn));
     if (ftmd > fnmd) {
       double tg[3];
-      for (int c = 0; c < 3; c++) tg[c] = ot[c] / mag;
+      const double rmag = 1.0 / mag;
+      for (int c = 0; c < 3; c++) tg[c] = div_by(ot[c], mag, rmag);
       for (int c = 0; c < 3; c++) ft[c] = -fnmd * tg[c];
       for (int c = 0; c < 3; c++) ot[c] = (fnmd / kt) * tg[c];
     }
@@ -167,48 +183,44 @@ __device__ __forceinline__ int pair_force_fp64(const PT& P, const PairIn& a,
     ft[0] = ft[1] = ft[2] = 0.0;
   }
   for (int c = 0; c < 3; c++) o.pft[c] = ot[c];
-  const double dist_cl = dm / 2.0 + (a.rL * a.rL - a.rI * a.rI) / (2.0 * dm);
-  const double dist_ci = dm - dist_cl;
+  const double dist_cl = dm / 2.0 + div_by(rL * rL - rI * rI, 2.0 * dm, 0.5 * rdm);
+  const double arm = a.owner ? dist_cl : dm - dist_cl;
   double tf[3];
   cross3(nrm, ft, tf);
-  for (int c = 0; c < 3; c++) o.fct[c] = 0.0 + fn[c] + ft[c];
-  for (int c = 0; c < 3; c++) o.tl[c] = dist_cl * tf[c];
-  for (int c = 0; c < 3; c++) o.ti[c] = dist_ci * tf[c];
-  return 1;
+  for (int c = 0; c < 3; c++) o.f[c] = 0.0 + fn[c] + ft[c];
+  for (int c = 0; c < 3; c++) o.t[c] = arm * tf[c];
 }
 
 // Mixed precision: contact geometry test in FP64 (same contact set as the
 // FP64 path), everything after it in FP32 except the history update.
 template <class PT>
-__device__ __forceinline__ int pair_force_mixed(const PT& P, const PairIn& a,
-                                                const double pft_in[3], PairOut& o) {
-  const double r_lm = a.rL + a.rI;
-  const double dist[3] = {a.xI[0] - a.xL[0], a.xI[1] - a.xL[1], a.xI[2] - a.xL[2]};
+__device__ __forceinline__ void pair_force_mixed(const PT& P, const PairIn& a,
+                                                 const double pft_in[3], PairOut& o) {
+  const double r_lm = a.rp + a.rj;
+  const double dist[3] = {a.xj[0] - a.xp[0], a.xj[1] - a.xp[1], a.xj[2] - a.xp[2]};
   const double dm2 = dot3(dist, dist);
-  const double rs = r_lm - kSmall;
-  if (dm2 > rs * rs) return 0;
-  if (dm2 == 0.0) return 2;
   const float dmf = fsqrt((float)dm2);
   const float inv = __builtin_amdgcn_rcpf(dmf);
   float nrm[3];
   for (int c = 0; c < 3; c++) nrm[c] = (float)dist[c] * inv;
   // overlap from the FP64 squared distance: r_lm - |d| = (r_lm^2 - |d|^2) / (r_lm + |d|)
   const float ovl = (float)((r_lm * r_lm - dm2)) * __builtin_amdgcn_rcpf((float)r_lm + dmf);
-  const float rL = (float)a.rL, rI = (float)a.rI;
+  const float rL = (float)(a.owner ? a.rp : a.rj), rI = (float)(a.owner ? a.rj : a.rp);
   float vrel[3];
-  for (int c = 0; c < 3; c++) vrel[c] = (float)(a.vL[c] - a.vI[c]);
+  for (int c = 0; c < 3; c++) vrel[c] = (float)(a.vp[c] - a.vj[c]);
   const float dcl = (dmf * dmf + rL * rL - rI * rI) * (0.5f * inv);
   const float dci = dmf - dcl;
   float osum[3], vrot[3];
-  for (int c = 0; c < 3; c++) osum[c] = (float)a.wL[c] * dcl + (float)a.wI[c] * dci;
+  const float dcp = a.owner ? dcl : dci, dcj = a.owner ? dci : dcl;
+  for (int c = 0; c < 3; c++) osum[c] = (float)a.wp[c] * dcp + (float)a.wj[c] * dcj;
   cross3f(osum, nrm, vrot);
   for (int c = 0; c < 3; c++) vrel[c] += vrot[c];
   const float vrn = dot3f(vrel, nrm);
   float vs[3];
   for (int c = 0; c < 3; c++) vs[c] = vrel[c] - vrn * nrm[c];
   const float reff = fdiv(rL * rI, rL + rI);
-  const float mL = (float)a.mL, mI = (float)a.mI;
-  const float meff = fdiv(mL * mI, mL + mI);
+  const float mp = (float)a.mp, mj = (float)a.mj;
+  const float meff = fdiv(mp * mj, mp + mj);
   float kn, kt, etan, etat;
   if (P.hertz) {
     const float sr = fsqrt(reff);
@@ -249,13 +261,11 @@ __device__ __forceinline__ int pair_force_mixed(const PT& P, const PairIn& a,
   }
   for (int c = 0; c < 3; c++) o.pft[c] = ot[c];
   const float dist_cl = 0.5f * dmf + (rL * rL - rI * rI) * (0.5f * inv);
-  const float dist_ci = dmf - dist_cl;
+  const float arm = a.owner ? dist_cl : dmf - dist_cl;
   float tf[3];
   cross3f(nrm, ft, tf);
-  for (int c = 0; c < 3; c++) o.fct[c] = (double)(fn[c] + ft[c]);
-  for (int c = 0; c < 3; c++) o.tl[c] = (double)(dist_cl * tf[c]);
-  for (int c = 0; c < 3; c++) o.ti[c] = (double)(dist_ci * tf[c]);
-  return 1;
+  for (int c = 0; c < 3; c++) o.f[c] = (double)(fn[c] + ft[c]);
+  for (int c = 0; c < 3; c++) o.t[c] = (double)(arm * tf[c]);
 }
 
 // ClosestPtPointTriangle, stl_functions_des_mod.f:25-160.

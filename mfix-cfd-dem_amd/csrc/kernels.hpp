@@ -587,31 +587,22 @@ __device__ __forceinline__ void pair_contact(const DevParams& P0, const PT& P, c
                                              int pid, bool owner, double d[6]) {
   const int S = P0.stride;
   PairIn in;
-  double xj[3], vj[3], wj[3], vp[3], wp[3];
-  const double rj = load_sphere(a.pos, j, xj);
-  load3(a.vel, S, j, vj);
-  load3(a.omega, S, j, wj);
-  load3(a.vel, S, ip, vp);
-  load3(a.omega, S, ip, wp);
-  const double mj = a.pmass[j], mp = a.pmass[ip];
+  in.rj = load_sphere(a.pos, j, in.xj);
+  load3(a.vel, S, j, in.vj);
+  load3(a.omega, S, j, in.wj);
+  load3(a.vel, S, ip, in.vp);
+  load3(a.omega, S, ip, in.wp);
+  in.mj = a.pmass[j];
+  in.mp = a.pmass[ip];
   const int phj = a.phase[j], php = a.phase[ip];
-  for (int c = 0; c < 3; c++) {
-    in.xL[c] = owner ? xp[c] : xj[c];
-    in.xI[c] = owner ? xj[c] : xp[c];
-    in.vL[c] = owner ? vp[c] : vj[c];
-    in.vI[c] = owner ? vj[c] : vp[c];
-    in.wL[c] = owner ? wp[c] : wj[c];
-    in.wI[c] = owner ? wj[c] : wp[c];
-  }
-  in.rL = owner ? rp : rj;
-  in.rI = owner ? rj : rp;
-  in.mL = owner ? mp : mj;
-  in.mI = owner ? mj : mp;
   in.phL = owner ? php : phj;
   in.phI = owner ? phj : php;
+  for (int c = 0; c < 3; c++) in.xp[c] = xp[c];
+  in.rp = rp;
+  in.owner = owner;
   double hin[3] = {0.0, 0.0, 0.0};
-  if (a.pfl_in[pid])
-    for (int c = 0; c < 3; c++) hin[c] = a.pft_in[3 * pid + c];
+  if (a.pfl_in[pid])  // kept in the owner's orientation
+    for (int c = 0; c < 3; c++) hin[c] = owner ? a.pft_in[3 * pid + c] : -a.pft_in[3 * pid + c];
   PairOut o;
   if (MIXED) pair_force_mixed(P, in, hin, o);
   else pair_force_fp64(P, in, hin, o);
@@ -620,9 +611,8 @@ __device__ __forceinline__ void pair_contact(const DevParams& P0, const PT& P, c
     a.pfl_out[pid] = 1;
     if (P0.store_forces) atomicAdd(&a.flags[kFlagContacts], 1);
   }
-  // FC(I) = FC(I) - FC_pair: adding the negation rounds the same
-  for (int c = 0; c < 3; c++) d[c] = owner ? o.fct[c] : -o.fct[c];
-  for (int c = 0; c < 3; c++) d[3 + c] = owner ? o.tl[c] : o.ti[c];
+  for (int c = 0; c < 3; c++) d[c] = o.f[c];
+  for (int c = 0; c < 3; c++) d[3 + c] = o.t[c];
 }
 
 // Orders the LDS accesses of a wavefront's lanes: no barrier is needed
