@@ -78,6 +78,7 @@ __device__ __forceinline__ double load_sphere(const Sphere* p, int i, double x[3
 }
 
 struct StepPtrs {
+  const int* stop;  // systems with inlets and outlets: BcPtrs::del_cnt[kBcStop]
   const Sphere* pos;
   Sphere* pos_o;
   const double *vel, *omega;
@@ -1005,6 +1006,7 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
   constexpr bool kPairs = MODE == kModeFused || MODE == kModeForce;
   constexpr bool kEarlyDrag = MODE == kModeFused && !FILTER && !BATCH;
   __shared__ double s_drag[kEarlyDrag ? 6 : 1][kBS];
+  if (MODE == kModeFused && !BATCH && a.stop && *a.stop) return;  // queued too early
   // a wavefront holds 2^lgw consecutive particles, one per lane of its first
   // 2^lgw lanes (lgw = 6 in the modes without pairs)
   const int wbase = (xcd_tile(blockIdx.x, gridDim.x) * (kBS / 64) + (int)(threadIdx.x >> 6)) << lgw;
@@ -2504,7 +2506,9 @@ struct BcPtrs {
   const uint8_t* phase;
   const BcDev* bcs;
   int nbc, n, S;
-  int* del_cnt;   // particles deleted so far and blocks done, both left at 0
+  // particles deleted so far, blocks done (both left at 0), and whether the
+  // neighbour search a deletion forces is due
+  int* del_cnt;
   int* del_list;  // their global ids
   struct BcHost* host;
   int seq;
@@ -2513,6 +2517,11 @@ struct BcPtrs {
 // What the host needs of a step with inlets and outlets before it can queue
 // the next one, in pinned memory: the sequence number of the step is written
 // last.  Ids beyond kBcHostGids are read from del_list.
+// There is one for each of two steps, since a step may be queued while the
+// one before it still runs: kernels of a step that a deletion has overtaken
+// (the neighbour search comes first) find the word at del_cnt[kBcStop] set
+// and do nothing, and the host queues them again after the search.
+constexpr int kBcStop = 2, kBcWords = 3;
 constexpr int kBcHostGids = 256;
 struct BcHost {
   int seq, count;
@@ -2593,16 +2602,22 @@ __device__ inline bool particle_bcs(const BcPtrs& b, int i) {
 // the kernel, a copy of the count and a wait for the stream took 24 us of a
 // 53 us step at 30,000 particles.
 __global__ __launch_bounds__(kBS) void k_dem_bcs(BcPtrs b) {
+  if (b.del_cnt[kBcStop]) return;
   const int i = blockIdx.x * kBS + threadIdx.x;
   const bool gone = i < b.n && particle_bcs(b, i);
   if (gone) __threadfence_system();
-  __syncthreads();
+  const bool any = __syncthreads_or(gone);
   if (threadIdx.x) return;
-  const int done = __hip_atomic_fetch_add(b.del_cnt + 1, 1, __ATOMIC_ACQ_REL,
+  if (any) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // a block without one has
+                                                               // nothing to order
+  const int done = __hip_atomic_fetch_add(b.del_cnt + 1, 1, __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT);
   if (done != (int)gridDim.x - 1) return;
-  b.host->count = __hip_atomic_load(b.del_cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const int nd = __hip_atomic_load(b.del_cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  b.host->count = nd;
   b.del_cnt[0] = b.del_cnt[1] = 0;
+  b.del_cnt[kBcStop] = nd > 0;
   __hip_atomic_store(&b.host->seq, b.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

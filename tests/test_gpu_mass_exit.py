@@ -12,8 +12,7 @@ from test_gpu_parity import assert_same_pairs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 255, 256, 257, 900])
-def test_layer_leaves_at_once(n):
+def layer(n):
     box = (0.05, 0.016, 0.05)
     p = params(box, (10, 8, 10), grav=(0.0, 0.0, 0.0), max_pip=n + 400)
     q = np.arange(n)
@@ -24,7 +23,12 @@ def test_layer_leaves_at_once(n):
                         vel=[(0.0, -0.5, 0.0)])
     inlet = abi.dem_bc(abi.BC_MASS_INFLOW, abi.PLANE_S, (0.02, box[1], 0.02),
                        (0.03, box[1], 0.03), vel=[(0.0, -0.5, 0.0)], ep_s=[0.2])
-    g, o = start(p, [outlet, inlet], parts)
+    return start(p, [outlet, inlet], parts)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 900])
+def test_layer_leaves_at_once(n):
+    g, o = layer(n)
     nn = 1
     for k in (200, 39, 1, 1, 1, 58, 100):
         g.run(nn, k)
@@ -33,6 +37,23 @@ def test_layer_leaves_at_once(n):
         assert_same(g, o, f"after step {nn - 1}")
         # the layer is there before step 240 and gone after it
         assert (o.get_particles()[3] == 3).sum() == (n if nn <= 240 else 0)
+    assert_same_pairs(g, o)
+    g.close()
+    o.close()
+
+
+@pytest.mark.parametrize("last", [239, 240, 241, 400])
+@pytest.mark.parametrize("n", [1, 257, 900])
+def test_layer_leaves_within_one_call(n, last):
+    """The deletions (step 240) overtake a step that is already queued, unless
+    the call ends there."""
+    g, o = layer(n)
+    for s in (g, o):
+        s.run(1, last)
+    assert_same(g, o, f"after step {last}")
+    for s in (g, o):
+        s.run(last + 1, 60)
+    assert_same(g, o, f"after step {last + 60}")
     assert_same_pairs(g, o)
     g.close()
     o.close()
