@@ -442,12 +442,14 @@ void t_end(mfixdem_handle* h, int slot) {
 // particles): 2,003 settled spheres, r = 11.5, 44 / 34 / 28 / 24 us; 20,000,
 // r = 12.6, 43 / 32 / 28 / 28; 301,057, r = 13, 129 / 121 / 133 / 172;
 // 120,000 mixed, r = 8, 33 / 32 / 36 / 45; 150,000 coupled, r = 5, 75 / 81 /
-// 96 / 128 (with the transfers of its fluid step).
+// 96 / 128 (with the transfers of its fluid step).  Fewer than 8 pay only
+// while the chip is not full, one wavefront per SIMD at most (8 / 4 / 2): 2,003
+// spheres 13.0 / 11.7 / 11.1, 20,000 14.8 / 18.9 / 26.5.
 int step_lgw(const mfixdem_handle* h) {
   const double r = 0.5 * (double)h->n_pairs / std::max(h->n, 1);  // r / 4
   const double room = 1024.0 * std::max(1.0, r * r);
   int lgw = 6;
-  while (lgw > 3 && (double)(h->n >> (lgw - 1)) <= room) lgw--;
+  while (lgw > 1 && (double)(h->n >> (lgw - 1)) <= (lgw > 3 ? room : 1024.0)) lgw--;
   return lgw;
 }
 
