@@ -1165,7 +1165,8 @@ __device__ __forceinline__ void remove_outside(const Removal& r, int S, int i) {
 // deposits itself).  The particles are visited in slot order (list null,
 // the Morton order of their search cells) or in list order, kDepPPT
 // consecutive ones per thread (2 measured fastest at 1M spheres, against 1
-// and 4): a run of particles in the same fluid cell
+// and 4; at 25,013, where 2 make only 49 workgroups, 1 takes 7.6 us and 2 8.9):
+// a run of particles in the same fluid cell
 // is summed in registers, each run adds its 8 corner values into an int64
 // tile in LDS covering the bounding box of the workgroup's nodes (up to
 // kDepCap nodes), and each touched tile node then costs one global atomic.
@@ -1173,12 +1174,12 @@ __device__ __forceinline__ void remove_outside(const Removal& r, int S, int i) {
 // to global memory.  Particles that changed fluid cell since the rebuild
 // only widen the box.  Weights are rounded to fixed point per particle and
 // summed as integers, so the result does not depend on the order.
-constexpr int kDepPPT = 2;
 constexpr int kDepCap = 4096;
+template <int kDepPPT>
 __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* list,
                                                       const Sphere* pos, const double* pmass,
                                                       const uint8_t* phase, const uint8_t* state,
-                                                      const int* fcell, const uint8_t* fluid,
+                                                      const int* fcell,
                                                       const double* xe, const double* yn,
                                                       const double* zt, unsigned long long* fix,
                                                       Removal rm) {
@@ -1215,7 +1216,7 @@ __global__ __launch_bounds__(kBS) void k_deposit_list(DevParams P, const int* li
     }
     int I, J, K;
     unpack_ijk(pc, I, J, K);
-    if (!fluid[lin_ijk(I, J, K, P.ni, P.nj)]) continue;
+    if (!fluid_at(P, I, J, K)) continue;
     pcell[u] = pc;
     lo0 = min(lo0, I); lo1 = min(lo1, J); lo2 = min(lo2, K);
     hi0 = max(hi0, I); hi1 = max(hi1, J); hi2 = max(hi2, K);

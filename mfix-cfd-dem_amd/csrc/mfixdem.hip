@@ -951,10 +951,14 @@ int32_t deposit_current(mfixdem_handle* h) {
     HIPOK(hipGetLastError());
     return do_cell_fields(h, true);
   }
-  hipLaunchKernelGGL(k_deposit_list, dim3(nblk(((int64_t)h->n + kDepPPT - 1) / kDepPPT)),
-                     dim3(kBS), 0, h->stream, P, nullptr, h->pos[h->cur], h->pmass[h->tw],
-                     h->phase[h->tw], h->state[h->tw], h->fcell[h->tw], h->fluid, h->xe, h->yn,
-                     h->zt, h->rops_fix[h->fb], rm);
+  // two particles per thread once each of the 256 CUs still gets a workgroup
+  // of its own (k_deposit_list has both sides)
+  const int ppt = h->n >= 2 * 256 * kBS ? 2 : 1;
+  auto k = ppt == 2 ? k_deposit_list<2> : k_deposit_list<1>;
+  hipLaunchKernelGGL(k, dim3(nblk(((int64_t)h->n + ppt - 1) / ppt)), dim3(kBS), 0, h->stream, P,
+                     nullptr, h->pos[h->cur], h->pmass[h->tw], h->phase[h->tw],
+                     h->state[h->tw], h->fcell[h->tw], h->xe, h->yn, h->zt,
+                     h->rops_fix[h->fb], rm);
   HIPOK(hipGetLastError());
   return do_cell_fields(h, true);
 }
