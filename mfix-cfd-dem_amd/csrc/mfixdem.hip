@@ -437,8 +437,10 @@ void t_end(mfixdem_handle* h, int slot) {
 // (r = 2 pairs / particle) in r windows of 64, one after another.  Fewer
 // particles shorten that walk and spread it over more wavefronts, at the
 // price of idle lanes in the per-particle part, which pays while the chip
-// (1,024 SIMDs) has room: always up to one wavefront per SIMD, and beyond
-// that the more the longer the rows are.  Measured per step (64 / 32 / 16 / 8
+// (1,024 SIMDs) has room: always up to one wavefront per SIMD, two where no
+// gas makes that part long (33,778 slots of a hopper 15.2 -> 13.6 us with 32
+// particles, 24,001 loose spheres 9.8 -> 9.0 with 16, but 40,009 coupled 22.9 ->
+// 24.2 with 32), and beyond that the more the longer the rows are.  Measured per step (64 / 32 / 16 / 8
 // particles): 2,003 settled spheres, r = 11.5, 44 / 34 / 28 / 24 us; 20,000,
 // r = 12.6, 43 / 32 / 28 / 28; 301,057, r = 13, 129 / 121 / 133 / 172;
 // 120,000 mixed, r = 8, 33 / 32 / 36 / 45; 150,000 coupled, r = 5, 75 / 81 /
@@ -447,7 +449,7 @@ void t_end(mfixdem_handle* h, int slot) {
 // spheres 13.0 / 11.7 / 11.1, 20,000 14.8 / 18.9 / 26.5.
 int step_lgw(const mfixdem_handle* h) {
   const double r = 0.5 * (double)h->n_pairs / std::max(h->n, 1);  // r / 4
-  const double room = 1024.0 * std::max(1.0, r * r);
+  const double room = std::max(h->S.p.coupled ? 1024.0 : 2048.0, 1024.0 * r * r);
   int lgw = 6;
   while (lgw > 1 && (double)(h->n >> (lgw - 1)) <= (lgw > 3 ? room : 1024.0)) lgw--;
   return lgw;
