@@ -994,11 +994,6 @@ int32_t refresh_free_gids(mfixdem_handle* h) {
   return MFIXDEM_OK;
 }
 
-// DES_TIME_STEP with DEM boundaries (des_time_march.f:354-380): the step
-// kernel (with UPDATE_EXIT_DES_VEL), then MASS_INFLOW_DEM and
-// MASS_OUTFLOW_DEM, and the neighbour search, which a deleted particle
-// forces.  Launched directly (the seeds differ from step to step), with one
-// wait for the count of deleted particles.
 // The kernels of a step that its inlets and outlets may not have decided yet:
 // the step itself and the checks of the boundaries (k_dem_bcs).
 int32_t queue_bc_step(mfixdem_handle* h) {
@@ -1022,14 +1017,45 @@ int32_t queue_bc_step(mfixdem_handle* h) {
   return MFIXDEM_OK;
 }
 
-// One step of a system with inlets and outlets.  The host must know which
-// particles a step deleted before it can place the next step's seeds, and
-// whether a neighbour search comes first; waiting for that with nothing
-// queued left the GPU idle for half of the time.  So where the call has
-// another step to take (more) and no search is due, the next step's kernels
-// are queued before the wait, and undone in the few cases that the step
-// deletes something (they find the stop word set and do nothing): 50 steps of
-// a draining hopper of 30,011 particles 2.0-2.3 -> 1.5 ms.
+// The particles that a step's checks (out) deleted: their global ids are free
+// again, and the kernels queued after the checks, which found the stop word
+// set, are queued anew by the next step.
+int32_t take_deleted(mfixdem_handle* h, const BcHost* out) {
+  const int nd = out->count;
+  std::vector<int> gone(nd);
+  if (nd <= kBcHostGids) {
+    std::memcpy(gone.data(), out->gid, sizeof(int) * nd);
+  } else {
+    HIPOK(hipMemcpyAsync(gone.data(), h->del_list, sizeof(int) * nd, hipMemcpyDeviceToHost,
+                         h->stream));
+    HIPOK(sync_stream(h));
+  }
+  for (int g : gone) h->dbc.free_gids.insert(g);
+  return fill_i32(h->stream, h->del_cnt + kBcStop, 1, 0);
+}
+
+// the neighbour search of a system with inlets and outlets
+int32_t bc_rebuild(mfixdem_handle* h) {
+  const int64_t rogue0 = h->st.rogue_deleted;
+  t_begin(h);
+  CHECKRC(do_bin(h));
+  CHECKRC(do_neighbour(h));
+  t_end(h, kTimeRebuild);
+  if (h->st.rogue_deleted != rogue0) CHECKRC(refresh_free_gids(h));
+  return MFIXDEM_OK;
+}
+
+// DES_TIME_STEP with DEM boundaries (des_time_march.f:354-380): the step
+// kernel (with UPDATE_EXIT_DES_VEL), then MASS_INFLOW_DEM and
+// MASS_OUTFLOW_DEM, and the neighbour search, which a deleted particle
+// forces.  The host must know which particles a step deleted before it can
+// place the next step's seeds, and whether a neighbour search comes first;
+// waiting for that with nothing queued left the GPU idle for half of the
+// time.  So where the call has another step to take (more) and no search is
+// due, the next step's kernels are queued before the wait, and undone in the
+// few cases that the step deletes something (they find the stop word set and
+// do nothing): 50 steps of a draining hopper of 30,011 particles 2.0-2.3 ->
+// 1.5 ms.
 int32_t bc_step(mfixdem_handle* h, int32_t nn, bool more) {
   DemBoundaries& D = h->dbc;
   bool rebuild = (nn == 1) || (nn % h->S.p.neighbor_search_n == 0);
@@ -1038,7 +1064,13 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn, bool more) {
   const int seq = h->bc_seq, c = h->cur, t = h->tw;
   BcHost* out = h->bc_host + (seq & 1);
   if (const int32_t rc = plan_seeds(h->S, D)) {
+    // no slot for a seed: the step's deletions stand, with the search they
+    // force, and the slots they free are there for the next step
     CHECKRC(wait_seq(h, &out->seq, seq));
+    if (out->count > 0) {
+      CHECKRC(take_deleted(h, out));
+      CHECKRC(bc_rebuild(h));
+    }
     return rc;
   }
   const int ns = (int)D.seeds.size();
@@ -1062,17 +1094,7 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn, bool more) {
     h->bc_ahead = true;
   }
   CHECKRC(wait_seq(h, &out->seq, seq));
-  const int nd = out->count;
-  if (nd > 0) {
-    std::vector<int> gone(nd);
-    if (nd <= kBcHostGids) {
-      std::memcpy(gone.data(), out->gid, sizeof(int) * nd);
-    } else {
-      HIPOK(hipMemcpyAsync(gone.data(), h->del_list, sizeof(int) * nd, hipMemcpyDeviceToHost,
-                           h->stream));
-      HIPOK(sync_stream(h));
-    }
-    for (int g : gone) D.free_gids.insert(g);
+  if (out->count > 0) {
     rebuild = true;  // FORCE_NSEARCH (mass_outflow_dem.f:178)
     if (h->bc_ahead) {  // as if the next step had not been queued
       h->bc_ahead = false;
@@ -1080,16 +1102,9 @@ int32_t bc_step(mfixdem_handle* h, int32_t nn, bool more) {
       h->pcur = 1 - h->pcur;
       h->bc_seq--;
     }
-    CHECKRC(fill_i32(h->stream, h->del_cnt + kBcStop, 1, 0));
+    CHECKRC(take_deleted(h, out));
   }
-  if (rebuild) {
-    const int64_t rogue0 = h->st.rogue_deleted;
-    t_begin(h);
-    CHECKRC(do_bin(h));
-    CHECKRC(do_neighbour(h));
-    t_end(h, kTimeRebuild);
-    if (h->st.rogue_deleted != rogue0) CHECKRC(refresh_free_gids(h));
-  }
+  if (rebuild) CHECKRC(bc_rebuild(h));
   D.s_time = D.s_time + h->S.d.dtsolid;
   h->st.steps++;
   return MFIXDEM_OK;
@@ -1341,6 +1356,8 @@ int32_t upload_ensemble(mfixdem_handle* h) {
   }
   HIPOK(hipMemsetAsync(h->flags, 0, sizeof(int) * kFlagCount, h->stream));
   h->flags_set = false;
+  // an error may have left the last run in the middle of a step
+  if (h->del_cnt) CHECKRC(fill_i32(h->stream, h->del_cnt, kBcWords, 0));
   h->st = mfixdem_status{};
   h->n_pairs = 0;
   h->first_pass = true;
@@ -1683,6 +1700,8 @@ int32_t mfixdem_set_particles(mfixdem_handle* h, int64_t n, const double* pos, c
   // on the handle's stream, which every later call on the handle waits for
   HIPOK(hipMemsetAsync(h->flags, 0, sizeof(int) * kFlagCount, h->stream));
   h->flags_set = false;
+  // an error may have left the last run in the middle of a step
+  if (h->del_cnt) CHECKRC(fill_i32(h->stream, h->del_cnt, kBcWords, 0));
   HIPOK(hipMemsetAsync(h->fc_id, 0, sizeof(double) * 3 * S, h->stream));
   HIPOK(hipMemsetAsync(h->tow_id, 0, sizeof(double) * 3 * S, h->stream));
   if (h->f_gp) {  // des_init_arrays.f:143
@@ -1873,6 +1892,8 @@ int32_t mfixdem_init(mfixdem_handle* h) {
   if (h->nsys > 1) CHECKRC(upload_ensemble(h));
   HIPOK(hipMemsetAsync(h->flags, 0, sizeof(int) * kFlagCount, h->stream));
   h->flags_set = false;
+  // an error may have left the last run in the middle of a step
+  if (h->del_cnt) CHECKRC(fill_i32(h->stream, h->del_cnt, kBcWords, 0));
   if (h->S.p.coupled) CHECKRC(do_locate(h, false));
   CHECKRC(do_bin(h));
   CHECKRC(do_neighbour(h));
