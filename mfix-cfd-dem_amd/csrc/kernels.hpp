@@ -1470,10 +1470,32 @@ __device__ __forceinline__ T block_sum(const T* a, int m, T* lds) {
   return s;
 }
 
+// The totals of a scan's tiles: tile[b], and, where there are more than
+// kScanDirect tiles, also pre[b], the sum of those before b in b's group of
+// kScanTile tiles, and group[g], the total of group g (pre null: neither).
+template <typename T>
+struct TileSums {
+  T *tile, *pre, *group;
+};
+
+// The sum of the totals of the tiles before this workgroup's.  Up to
+// kScanDirect tiles every workgroup adds them up itself, nb^2 / 2 loads in
+// all, which saves a launch; beyond it k_scan_groups leaves at most 1,024
+// group totals to add (a scan of 2^30 elements).  Per step with a rebuild in
+// each, 5,000 spheres in a box of 1,024 nb search cells, without and with
+// k_scan_groups: nb = 1,380 62 and 67 us, 2,750 79 and 81, 4,120 96 and 96,
+// 5,500 117 and 115, 22,000 433 and 371, 88,000 2,302 and 1,335.
+constexpr int kScanDirect = 4096;
+template <typename T>
+__device__ __forceinline__ T sum_before(const TileSums<T>& t, T* lds) {
+  const int b = blockIdx.x;
+  return t.pre ? t.pre[b] + block_sum(t.group, b / kScanTile, lds) : block_sum(t.tile, b, lds);
+}
+
 // Exclusive scan of in[0..n) into out[0..n], out[n] = total, in two launches
-// of one workgroup per tile: each tile scanned by itself, then every
-// workgroup sums the totals of the tiles before its own (a launch of its own
-// for those took 4.5 us a rebuild, this sum nothing that shows).
+// of one workgroup per tile, each tile scanned by itself and then the totals
+// of the tiles before it added, with k_scan_groups between them where there
+// are more than kScanDirect tiles.
 __global__ __launch_bounds__(kBS) void k_scan_tiles(const int* in, int* out, int n, int* bsum) {
   __shared__ int lds[kBS / 64 + 1];
   const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
@@ -1491,14 +1513,32 @@ __global__ __launch_bounds__(kBS) void k_scan_tiles(const int* in, int* out, int
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(kBS) void k_scan_add(int* out, int n, const int* bsum) {
+template <typename T>
+__global__ __launch_bounds__(kBS) void k_scan_groups(int nb, TileSums<T> t) {
+  __shared__ T lds[kBS / 64 + 1];
+  const int base = blockIdx.x * kScanTile + threadIdx.x * kScanPer;
+  T v[kScanPer], s = 0;
+  for (int q = 0; q < kScanPer; q++) {
+    v[q] = base + q < nb ? t.tile[base + q] : 0;
+    s += v[q];
+  }
+  T tot;
+  T pre = block_excl_scan(s, &tot, lds);
+  for (int q = 0; q < kScanPer; q++) {
+    if (base + q < nb) t.pre[base + q] = pre;
+    pre += v[q];
+  }
+  if (threadIdx.x == 0) t.group[blockIdx.x] = tot;
+}
+
+__global__ __launch_bounds__(kBS) void k_scan_add(int* out, int n, TileSums<int> t) {
   __shared__ int lds[kBS / 64];
-  const int pre = block_sum(bsum, blockIdx.x, lds);
+  const int pre = sum_before(t, lds);
   for (int q = 0; q < kScanPer; q++) {
     const int i = blockIdx.x * kScanTile + q * kBS + threadIdx.x;
     if (i < n) out[i] += pre;
   }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = pre + bsum[blockIdx.x];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = pre + t.tile[blockIdx.x];
 }
 
 // The offsets of the neighbour rows in one scan: each particle's own and
@@ -1536,10 +1576,10 @@ struct HostFlags {
 };
 
 __global__ __launch_bounds__(kBS) void k_scan_rows_add(int* pair_base, int* row_start, int n,
-                                                       const long long* bsum, int* flags,
+                                                       TileSums<long long> sums, int* flags,
                                                        HostFlags* host, int seq) {
   __shared__ long long lds[kBS / 64];
-  const long long pre = block_sum(bsum, blockIdx.x, lds);
+  const long long pre = sum_before(sums, lds);
   const int ph = (int)(pre >> 32), pl = (int)(pre & 0xffffffffll);
   for (int q = 0; q < kScanPer; q++) {
     const int i = blockIdx.x * kScanTile + q * kBS + threadIdx.x;
@@ -1549,7 +1589,7 @@ __global__ __launch_bounds__(kBS) void k_scan_rows_add(int* pair_base, int* row_
     }
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-    const long long t = pre + bsum[blockIdx.x];
+    const long long t = pre + sums.tile[blockIdx.x];
     pair_base[n] = (int)(t >> 32);
     row_start[n] = (int)(t >> 32) + (int)(t & 0xffffffffll);
     flags[kFlagPairs] = (int)(t >> 32);  // read back with the other flags

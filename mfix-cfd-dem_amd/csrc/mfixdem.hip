@@ -282,12 +282,32 @@ int32_t fill_i32(hipStream_t s, int* a, int64_t n, int v) {
   return MFIXDEM_OK;
 }
 
+// Words a scan of at most n elements needs for the sums of its tiles.
+int64_t scan_words(int64_t n) {
+  const int64_t nb = n / kScanTile + 2;
+  return 2 * nb + nb / kScanTile + 1;
+}
+inline int scan_tiles(int64_t n) { return std::max((int)((n + kScanTile - 1) / kScanTile), 1); }
+// the sums of nb tiles in a buffer of scan_words
+template <typename T>
+TileSums<T> tile_sums(T* buf, int nb) {
+  if (nb <= kScanDirect) return {buf, nullptr, nullptr};
+  return {buf, buf + nb, buf + 2 * (int64_t)nb};
+}
+// the group sums of a scan of nb tiles, between its two passes
+template <typename T>
+void sum_groups(mfixdem_handle* h, int nb, const TileSums<T>& t) {
+  if (t.pre)
+    hipLaunchKernelGGL(k_scan_groups<T>, dim3(scan_tiles(nb)), dim3(kBS), 0, h->stream, nb, t);
+}
+
 // exclusive scan of in[0..n) -> out[0..n]; out[n] = total
 int32_t scan_i32(mfixdem_handle* h, const int* in, int* out, int64_t n) {
-  const int nb = std::max((int)((n + kScanTile - 1) / kScanTile), 1);
-  hipLaunchKernelGGL(k_scan_tiles, dim3(nb), dim3(kBS), 0, h->stream, in, out, (int)n,
-                     h->scan_bsum);
-  hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kBS), 0, h->stream, out, (int)n, h->scan_bsum);
+  const int nb = scan_tiles(n);
+  const TileSums<int> t = tile_sums(h->scan_bsum, nb);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(nb), dim3(kBS), 0, h->stream, in, out, (int)n, t.tile);
+  sum_groups(h, nb, t);
+  hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kBS), 0, h->stream, out, (int)n, t);
   HIPOK(hipGetLastError());
   return MFIXDEM_OK;
 }
@@ -296,11 +316,13 @@ int32_t scan_i32(mfixdem_handle* h, const int* in, int* out, int64_t n) {
 // incoming counts (k_scan_rows_tiles); the flags go to the host with it.
 int32_t scan_rows(mfixdem_handle* h, const int* own, const int* in, int* pair_base,
                   int* row_start, int64_t n) {
-  const int nb = std::max((int)((n + kScanTile - 1) / kScanTile), 1);
+  const int nb = scan_tiles(n);
+  const TileSums<long long> t = tile_sums(h->scan_bsum64, nb);
   hipLaunchKernelGGL(k_scan_rows_tiles, dim3(nb), dim3(kBS), 0, h->stream, own, in, pair_base,
-                     row_start, (int)n, h->scan_bsum64);
+                     row_start, (int)n, t.tile);
+  sum_groups(h, nb, t);
   hipLaunchKernelGGL(k_scan_rows_add, dim3(nb), dim3(kBS), 0, h->stream, pair_base, row_start,
-                     (int)n, h->scan_bsum64, h->flags, h->host_flags, ++h->flags_seq);
+                     (int)n, t, h->flags, h->host_flags, ++h->flags_seq);
   HIPOK(hipGetLastError());
   return MFIXDEM_OK;
 }
@@ -1475,9 +1497,9 @@ int32_t alloc_buffers(mfixdem_handle* h) {
       .add(&h->fc_id, 3 * S).add(&h->tow_id, 3 * S).add(&h->own_cnt, n)
       .add(&h->own_tmp, n * h->maxrow)
       .add(&h->own_key, n * h->maxrow).add(&h->in_cnt, n).add(&h->in_cur, n).add(&h->tot_cnt, n)
-      .add(&h->scan_bsum64, n / kScanTile + 2)
-      .add(&h->scan_bsum,
-           std::max<int64_t>(std::max<int64_t>(n, nc), (int64_t)h->n_fine + h->nsys) / kScanTile + 2)
+      .add(&h->scan_bsum64, scan_words(n))
+      .add(&h->scan_bsum, scan_words(std::max<int64_t>(std::max<int64_t>(n, nc),
+                                                       (int64_t)h->n_fine + h->nsys)))
       .add(&h->flags, kFlagCount).add(&h->xe, h->S.ni + 1)
       .add(&h->csz, h->S.ni + h->S.nj + h->S.nk).add(&h->yn, h->S.nj + 1).add(&h->zt, h->S.nk + 1)
       .add(&h->vnode, 3 * nc).add(&h->p_force, 3 * nc).add(&h->ugc, 3 * nc)
