@@ -405,7 +405,8 @@ int32_t mfixdem_get_status(mfixdem_handle* h, mfixdem_status* out);
    cut-off FACTOR_RLM*2*MAX_RADIUS, and the kernel that builds the
    neighbour rows: one thread per particle over a half stencil (default),
    or one wavefront per search cell with an LDS tile of 128, 192 or 256
-   candidates.  The pair sets
+   candidates.  A dilute member of an ensemble takes larger cells, 16 per
+   slot at most.  The pair sets
    and every result are the same for all choices; FACTOR_RLM itself (the
    neighbour-list skin) is a model parameter and stays as given.  May be
    called at any time outside a step. */

@@ -2372,7 +2372,10 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
     const Setup& S = h->sys_setup[s];
     fill_params(S, h->n, h->stride, ptab[s], gtab[s]);
     int nfine = 0;
-    if (search_grid(S.p, S.p.max_pip, gtab[s], nfine) != MFIXDEM_OK) {
+    const int slots = h->sys_off[s + 1] - h->sys_off[s];
+    if ((nsys > 1 ? member_grid(S.p, slots, gtab[s], nfine)
+                  : search_grid(S.p, slots, gtab[s], nfine)) != MFIXDEM_OK ||
+        nfine > INT_MAX / 2 - cell_off[s]) {
       delete h;
       return MFIXDEM_ERR_UNSUPPORTED;
     }
@@ -2488,8 +2491,8 @@ int32_t mfixdem_set_tuning(mfixdem_handle* h, double cell_scale, int32_t row_ker
     std::vector<int> off(h->nsys + 1, 0);
     for (int s = 0; s < h->nsys; s++) {
       int nf = 0;
-      if (search_grid(h->sys_setup[s].p, h->sys_setup[s].p.max_pip, gt[s], nf, cell_scale) !=
-          MFIXDEM_OK)
+      if (member_grid(h->sys_setup[s].p, h->sys_off[s + 1] - h->sys_off[s], gt[s], nf,
+                      cell_scale) != MFIXDEM_OK)
         return MFIXDEM_ERR_UNSUPPORTED;
       off[s + 1] = off[s] + nf;
     }
