@@ -1668,6 +1668,39 @@ __device__ __forceinline__ int cell_system(const BatchDev& B, int c) {
   return lo;
 }
 
+// The rank of each search cell (x fastest) in the Morton order of its (fx, fy,
+// fz), the order that the binned particles lie in: the cells of the grid that
+// an octree over it visits before this one, which are, level by level, the
+// cells in the octants before the cell's own.  Ensembles rank system after
+// system, each followed by the place of its nonexistent particles.  Run once
+// per search grid (on the host, octant by octant, it took 4 ns a cell: 60 of
+// the 190 ms that 64 members of 40,000 spheres took to set up).
+template <bool BATCH>
+__global__ __launch_bounds__(kBS) void k_cell_ranks(int nfine, GridDev G0, int* rank,
+                                                    BatchDev B) {
+  const int c = blockIdx.x * kBS + threadIdx.x;
+  if (c >= nfine) return;
+  const int s = BATCH ? cell_system(B, c) : 0;
+  const GridDev& G = sys_grid<BATCH>(G0, B, s);
+  const int base = BATCH ? B.cell_off[s] : 0;
+  const int nx = G.fn[0], ny = G.fn[1], nz = G.fn[2];
+  const int x = (c - base) % nx, y = (c - base) / nx % ny, z = (c - base) / (nx * ny);
+  int before = base + s;
+  // the octree's cubes have sides of 1024, 512, ... cells (an axis has 1022 at
+  // most); e0, e1, e2: cells of the cube around (x, y, z) inside the grid
+  int e0 = nx, e1 = ny, e2 = nz;
+  for (int h = 512; h > 0; h >>= 1) {
+    const int l0 = min(e0, h), l1 = min(e1, h), l2 = min(e2, h);  // of its lower halves
+    if (z & h) before += e0 * e1 * l2;
+    e2 = z & h ? e2 - l2 : l2;
+    if (y & h) before += e0 * l1 * e2;
+    e1 = y & h ? e1 - l1 : l1;
+    if (x & h) before += l0 * e1 * e2;
+    e0 = x & h ? e0 - l0 : l0;
+  }
+  rank[c] = before;
+}
+
 // The single-precision copy is relative to G.pf_c; a particle beyond
 // pf_xmax on some axis gets radius -1 there (every test with it is then
 // made in double precision), a nonexistent one a position no cut-off

@@ -1423,24 +1423,9 @@ void fill_devparams(mfixdem_handle* h) {
   h->P.nbc = (int)h->dbc.b.size();
 }
 
-// Walks the cells of a grid in Morton order (octants of a cube that covers
-// the grid, those outside it skipped): rank[cell] = next place.
-void morton_ranks(const int fn[3], int x, int y, int z, int size, int* rank, int& next) {
-  if (x >= fn[0] || y >= fn[1] || z >= fn[2]) return;
-  if (size == 1) {
-    rank[x + fn[0] * (y + fn[1] * z)] = next++;
-    return;
-  }
-  const int s = size / 2;
-  for (int o = 0; o < 8; o++)
-    morton_ranks(fn, x + (o & 1) * s, y + ((o >> 1) & 1) * s, z + (o >> 2) * s, s, rank, next);
-}
-
-// Search cells for the counting sort: the rank of each cell (x fastest) in
-// the Morton order of its (fx, fy, fz), so that the binned particles lie in
-// Morton order, system after system, each followed by the place of its
-// nonexistent particles; zeroed counts.  All that a finer or coarser search
-// grid replaces is made here.
+// Search cells for the counting sort: the rank of each cell (k_cell_ranks),
+// zeroed counts.  All that a finer or coarser search grid replaces is made
+// here; an ensemble's tables (h->B) are up to date.
 int32_t setup_fine_cells(mfixdem_handle* h) {
   dfree(h, h->fstart);
   dfree(h, h->fend);
@@ -1448,19 +1433,6 @@ int32_t setup_fine_cells(mfixdem_handle* h) {
   dfree(h, h->fine_cnt);
   dfree(h, h->fine_off);
   const int nf = h->n_fine, ns = h->nsys;
-  std::vector<int> rank((size_t)nf);
-  int64_t cell = 0;
-  int next = 0;
-  for (int s = 0; s < ns; s++, next++) {
-    const int* fn = ns > 1 ? h->sys_grid[s].fn : h->G.fn;
-    int size = 1;
-    while (size < std::max(fn[0], std::max(fn[1], fn[2]))) size *= 2;
-    const int64_t cells = (int64_t)fn[0] * fn[1] * fn[2];
-    if (cell + cells > nf) return MFIXDEM_ERR_ARG;
-    morton_ranks(fn, 0, 0, 0, size, rank.data() + cell, next);
-    cell += cells;
-  }
-  if (cell != nf) return MFIXDEM_ERR_ARG;
   CHECKRC(Pieces()
               .add(&h->fstart, nf)
               .add(&h->fend, nf)
@@ -1468,9 +1440,11 @@ int32_t setup_fine_cells(mfixdem_handle* h) {
               .add(&h->fine_cnt, (int64_t)nf + ns)
               .add(&h->fine_off, (int64_t)nf + ns + 1)
               .alloc(h));
-  HIPOK(hipMemcpy(h->fine_rank, rank.data(), sizeof(int) * nf, hipMemcpyHostToDevice));
-  HIPOK(hipMemset(h->fine_cnt, 0, sizeof(int) * ((size_t)nf + ns)));
-  return MFIXDEM_OK;
+  auto ranks = ns > 1 ? k_cell_ranks<true> : k_cell_ranks<false>;
+  hipLaunchKernelGGL(ranks, dim3(nblk(nf)), dim3(kBS), 0, h->stream, nf, h->G, h->fine_rank,
+                     h->B);
+  HIPOK(hipGetLastError());
+  return fill_i32(h->stream, h->fine_cnt, (int64_t)nf + ns, 0);
 }
 
 // Device buffers, stream and events of a handle whose set-up (S, P, G,
@@ -1521,7 +1495,7 @@ int32_t alloc_buffers(mfixdem_handle* h) {
         hipMemset(h->drag_fc, 0, sizeof(double) * 3 * n) != hipSuccess)
       return fail(MFIXDEM_ERR_HIP);
   }
-  if ((rc = upload_setup(h)) || (rc = setup_fine_cells(h))) return fail(rc);
+  if ((rc = upload_setup(h))) return fail(rc);
   if (hipMemset(h->flags, 0, sizeof(int) * kFlagCount) != hipSuccess) return fail(MFIXDEM_ERR_HIP);
   if (hipHostMalloc((void**)&h->host_flags, sizeof(HostFlags), hipHostMallocDefault) != hipSuccess)
     return fail(MFIXDEM_ERR_OOM);
@@ -1627,7 +1601,7 @@ int32_t mfixdem_create(const mfixdem_params* p, mfixdem_handle** out) {
     delete h;
     return MFIXDEM_ERR_UNSUPPORTED;
   }
-  if ((rc = alloc_buffers(h)) || (rc = bind_scratch(h))) {
+  if ((rc = alloc_buffers(h)) || (rc = setup_fine_cells(h)) || (rc = bind_scratch(h))) {
     mfixdem_destroy(h);
     return rc;
   }
@@ -2419,10 +2393,6 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
     for (int s = 0; s < nsys; s++) sp.push_back(&h->sys_setup[s]);
     rc = upload_facets(h, sp);
   }
-  if (rc != MFIXDEM_OK) {
-    mfixdem_destroy(h);
-    return rc;
-  }
   h->B.sys = h->d_sys;
   h->B.ptab = h->d_ptab;
   h->B.gtab = h->d_gtab;
@@ -2430,6 +2400,11 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
   h->B.dg_off = h->d_dg_off;
   h->B.rogue = h->d_rogue;
   h->B.nsys = nsys;
+  if (rc == MFIXDEM_OK) rc = setup_fine_cells(h);
+  if (rc != MFIXDEM_OK) {
+    mfixdem_destroy(h);
+    return rc;
+  }
   const size_t S = h->stride;
   h->st_pos.assign(3 * S, 0.0);
   h->st_vel.assign(3 * S, 0.0);
