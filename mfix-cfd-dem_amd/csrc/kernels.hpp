@@ -148,15 +148,18 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 }
 
 // Ensembles: many independent systems in one set of particle arrays.  The
-// slots of system s are a fixed range that starts at a multiple of 64 (the
+// slots of system s are a fixed range.  It starts at a multiple of 64 (the
 // slots between a system's capacity and that multiple stay NONEXISTENT), so
 // that the particles of a wavefront belong to one system and its parameters
 // are read through the scalar cache (read per lane, the step of 3M spheres in
-// 64 systems took 419 us, so 301).  Each slot carries its system id, and
+// 64 systems took 419 us, so 301); where thousands of systems are smaller than
+// a wavefront (pack_slots) it starts where the one before it ends, and the
+// lanes read their own system's.  Each slot carries its system id, and
 // parameters, grids, search-grid cell offsets, DES-cell offsets and rogue
 // flags are per-system tables, none of which a kernel writes except the
-// flags.  The BATCH kernel variants read them; with BATCH = false the kernels
-// take the single system's blocks by value.
+// flags.  The BATCH kernel variants read them; kernels of one system take
+// its blocks by value.
+enum Batch { kOneSystem = 0, kAlignedSystems = 1, kPackedSystems = 2 };
 struct GridDev;
 struct BatchDev {
   const uint16_t* sys;      // system of each slot
@@ -168,16 +171,20 @@ struct BatchDev {
   int nsys;
 };
 #define MFIXDEM_CONST __attribute__((address_space(4)))
-// the system of the wavefront whose particles begin at the (uniform) slot i
-template <bool BATCH>
-__device__ __forceinline__ int wave_system(const BatchDev& B, int i) {
-  if constexpr (BATCH) return __builtin_amdgcn_readfirstlane((int)B.sys[i]);
+// the system of slot i: of the wavefront, for which any of its slots will do,
+// or of the lane
+template <int BATCH>
+__device__ __forceinline__ int slot_system(const BatchDev& B, int i) {
+  if constexpr (BATCH == kAlignedSystems)
+    return __builtin_amdgcn_readfirstlane((int)B.sys[__builtin_amdgcn_readfirstlane(i)]);
+  else if constexpr (BATCH == kPackedSystems) return B.sys[i];
   else return 0;
 }
-template <bool BATCH>
+template <int BATCH>
 __device__ __forceinline__ decltype(auto) sys_params(const DevParams& P0, const BatchDev& B,
                                                      int s) {
-  if constexpr (BATCH) return (((const MFIXDEM_CONST DevParams*)B.ptab)[s]);
+  if constexpr (BATCH == kAlignedSystems) return (((const MFIXDEM_CONST DevParams*)B.ptab)[s]);
+  else if constexpr (BATCH == kPackedSystems) return (B.ptab[s]);
   else return (P0);
 }
 // a table entry that is the same in every lane, through the scalar cache
@@ -190,6 +197,13 @@ __device__ __forceinline__ T load_uniform(const T* p) {
 #pragma unroll
   for (int k = 0; k < (int)(sizeof(T) / 4); k++) o[k] = u[k];
   return t;
+}
+
+// what slot_system's kernels need of that system's entry, by value
+template <int BATCH, class T>
+__device__ __forceinline__ T load_entry(const T* tab, int s) {
+  if constexpr (BATCH == kAlignedSystems) return load_uniform(tab + s);
+  else return tab[s];
 }
 
 __device__ __forceinline__ void load3(const double* a, int S, int i, double v[3]) {
@@ -640,10 +654,11 @@ __device__ __forceinline__ void wave_lds_fence() {
 // bit-identical to a per-particle loop.  Rows of a nonexistent particle
 // (xr[3] < 0) only carry their history over.  Every lane of the wavefront
 // must call this; xr is the lane's own position and radius, which the lanes
-// working on its row read from LDS.
-template <bool MIXED, class PT>
-__device__ __forceinline__ void wave_pairs(const DevParams& P0, const PT& P, const StepPtrs& a,
-                                           int lgw, int wbase, int e0, int e1,
+// working on its row read from LDS.  P: the parameters of the wavefront's
+// system; a packed ensemble reads those of the row's.
+template <bool MIXED, int BATCH, class PT>
+__device__ __forceinline__ void wave_pairs(const DevParams& P0, const PT& P, const BatchDev& B,
+                                           const StepPtrs& a, int lgw, int wbase, int e0, int e1,
                                            const double xr[4], double fc[3], double tow[3]) {
   constexpr int kQueue = 128;
   __shared__ double s_xr[kBS / 64][4][64];
@@ -709,8 +724,12 @@ __device__ __forceinline__ void wave_pairs(const DevParams& P0, const PT& P, con
       p = (int)(rc & rmask);
       const double xp[3] = {s_xr[w][0][p], s_xr[w][1][p], s_xr[w][2][p]};
       double d[6];
-      pair_contact<MIXED>(P0, P, a, wbase + p, xp, s_xr[w][3][p], q_j[w][q], q_pid[w][q],
-                          (rc & kRowOwn) != 0u, d);
+      auto contact = [&](const auto& Pr) {
+        pair_contact<MIXED>(P0, Pr, a, wbase + p, xp, s_xr[w][3][p], q_j[w][q], q_pid[w][q],
+                            (rc & kRowOwn) != 0u, d);
+      };
+      if constexpr (BATCH == kPackedSystems) contact(B.ptab[B.sys[wbase + p]]);
+      else contact(P);
 #pragma unroll
       for (int k = 0; k < 6; k++) s_d[w][k][lane] = d[k];
     }
@@ -1004,7 +1023,7 @@ __device__ __forceinline__ void step_tail(const DevParams& P0, const PT& P,
 // after the pair forces, where CALC_DRAG_DES adds them.  With
 // P0.fuse_dep it also deposits the particles' new positions
 // (COMP_MEAN_FIELDS0 node sums) before it ends.
-template <bool MIXED, int MODE, bool FILTER, bool BATCH = false, bool STL = false>
+template <bool MIXED, int MODE, bool FILTER, int BATCH = kOneSystem, bool STL = false>
 __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev B, int lgw) {
   constexpr bool kPairs = MODE == kModeFused || MODE == kModeForce;
   constexpr bool kEarlyDrag = MODE == kModeFused && !FILTER && !BATCH;
@@ -1018,7 +1037,8 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
   if (!kPairs && !live) return;  // the pair modes keep every lane for the wave passes
   const int S = P0.stride;
   const int w0 = __builtin_amdgcn_readfirstlane(wbase);
-  const int sys = wave_system<BATCH>(B, w0 < P0.n ? w0 : 0);
+  const int sys = slot_system<BATCH>(
+      B, BATCH == kPackedSystems ? (live ? i : 0) : (w0 < P0.n ? w0 : 0));
   decltype(auto) P = sys_params<BATCH>(P0, B, sys);
   const int st = live ? a.state[i] : 0;
   // the first loads do not wait for the state (with pair_contact's history:
@@ -1138,11 +1158,11 @@ __global__ __launch_bounds__(kBS) void k_step(DevParams P0, StepPtrs a, BatchDev
       if (wm != wm0) a.wmask[i] = wm;
     }
     // ---- pairs (calc_force_dem.f:180-412), summed after the walls
-    wave_pairs<MIXED>(P0, P, a, lgw, w0, e0, e1, xr, fc, tow);
+    wave_pairs<MIXED, BATCH>(P0, P, B, a, lgw, w0, e0, e1, xr, fc, tow);
   }
   DepIn dep;
   if (live)
-    step_tail<MIXED, MODE, FILTER, BATCH, kEarlyDrag>(P0, P, a, i, st, fc, tow, drag,
+    step_tail<MIXED, MODE, FILTER, BATCH != kOneSystem, kEarlyDrag>(P0, P, a, i, st, fc, tow, drag,
                                                       &s_drag[0][0], dep);
   if constexpr (kEarlyDrag) {
     // s_drag is read above and free once the first barrier inside has passed
@@ -1736,11 +1756,11 @@ __device__ __forceinline__ void pack_candidate(const GridDev& G, const double p[
 // another, each with its own last cell, so that every system keeps its slot
 // range; there the key sort this replaces took 275 us of kernels at 3M
 // spheres and moved all particle data at every binning.
-template <bool BATCH>
+template <int BATCH>
 __device__ __forceinline__ int absent_cell(const BatchDev& B, int s, int nfine) {
   return BATCH ? B.cell_off[s + 1] + s : nfine;
 }
-template <bool BATCH>
+template <int BATCH>
 __global__ __launch_bounds__(kBS) void k_bin_count(int n, GridDev G0, const Sphere* pos,
                                                    uint8_t* state, const int* gid,
                                                    int* dgc, const int* cell_rank,
@@ -1748,13 +1768,13 @@ __global__ __launch_bounds__(kBS) void k_bin_count(int n, GridDev G0, const Sphe
                                                    int* flags, BatchDev B) {
   const int i = blockIdx.x * kBS + threadIdx.x;
   if (i >= n) return;
-  const int s = wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(i));
+  const int s = slot_system<BATCH>(B, i);
   int r = absent_cell<BATCH>(B, s, nfine);
   if (state[i] == kNonexistent) {
     dgc[i] = 0;
   } else {
     GridDev Gs;
-    if constexpr (BATCH) Gs = load_uniform(B.gtab + s);
+    if constexpr (BATCH) Gs = load_entry<BATCH>(B.gtab, s);
     const GridDev& G = BATCH ? Gs : G0;
     if (state[i] == kSeeded) state[i] = kEntering;  // binned now: in a DES cell list
     double x[3];
@@ -1811,7 +1831,7 @@ struct BinPack {               // k_bin_place's packing of the row walk's candid
   double* xr;
   float4* xf;
 };
-template <bool BATCH>
+template <int BATCH>
 __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, int nsys,
                                                    const uint64_t* place,
                                                    const int* cell_rank, const int* cell_off,
@@ -1827,8 +1847,7 @@ __global__ __launch_bounds__(kBS) void k_bin_place(int n, int nfine, int nsys,
     inv[i] = np;
     // the candidate data of the row walk, at the particle's new place
     GridDev Gs;
-    if constexpr (BATCH)
-      Gs = load_uniform(B.gtab + wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(i)));
+    if constexpr (BATCH) Gs = load_entry<BATCH>(B.gtab, slot_system<BATCH>(B, i));
     double x[3];
     const double r = load_sphere(bp.pos, i, x);
     pack_candidate(BATCH ? Gs : bp.G, x, r, bp.state[i] != 0, bp.xr, bp.xf, np);
@@ -1997,7 +2016,7 @@ __device__ __forceinline__ void own_row_exact(const GridDev& G, const BuildPtrs&
 // takes the cells p, p + kRowLanes, ...): shorter candidate walks per lane,
 // and the range table each lane keeps in LDS shrinks with them, so more
 // wavefronts fit on a CU to hide the walk's dependent loads.
-template <bool BATCH, int kRowLanes>
+template <int BATCH, int kRowLanes>
 __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, BuildPtrs b,
                                                   BatchDev B) {
   constexpr int kCells = (kHalfCells + kRowLanes - 1) / kRowLanes;
@@ -2010,14 +2029,12 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
   if (hp >= n) return;
   const int h = b.idx ? b.idx[hp] : hp;                   // and slot
   if (b.state[h] == 0) return;
-  // a system's positions are its slot range: with two lanes per particle a
-  // wavefront's 32 positions are of one system
-  constexpr bool kUniform = BATCH && kRowLanes == 2;
-  const int s = kUniform ? wave_system<BATCH>(B, __builtin_amdgcn_readfirstlane(hp))
-                         : (BATCH ? B.sys[hp] : 0);
+  // a system's positions are its slot range: with two lanes per particle and
+  // aligned systems a wavefront's 32 positions are of one system
+  static_assert(BATCH != kAlignedSystems || kRowLanes == 2, "");
+  const int s = slot_system<BATCH>(B, hp);
   GridDev Gs;
-  if constexpr (kUniform) Gs = load_uniform(B.gtab + s);
-  else if constexpr (BATCH) Gs = B.gtab[s];
+  if constexpr (BATCH) Gs = load_entry<BATCH>(B.gtab, s);
   const GridDev& G = BATCH ? Gs : G0;
   const int cbase = BATCH ? B.cell_off[s] : 0;
   const int g_r = BATCH ? B.rogue[2 * s] : b.flags[kFlagRogueGid];
@@ -2073,7 +2090,7 @@ __global__ __launch_bounds__(kBS) void k_own_rows(int n, int S, GridDev G0, Buil
     const float e0 = xh.x - uc.x, e1 = xh.y - uc.y, e2 = xh.z - uc.z;
     if (coarse && uc.w >= 0.0f && e0 * e0 + e1 * e1 + e2 * e2 > lim * lim) continue;
     if (nh < kHits) s_hit[nh++][threadIdx.x] = tc;
-    else own_row_exact<BATCH>(G, b, S, g_r, h, gh, x, r, tc);  // a crowded stencil: at once
+    else own_row_exact<BATCH != kOneSystem>(G, b, S, g_r, h, gh, x, r, tc);  // a crowded stencil: at once
   }
   if (nh == 0) return;
   // The waiting candidates, all at once: their loads issued together, the

@@ -58,7 +58,8 @@ struct mfixdem_handle {
   BatchDev B{};
   std::vector<Setup> sys_setup;           // per system (ensembles)
   std::vector<GridDev> sys_grid;          // per-system grids (host copy of d_gtab)
-  std::vector<int> sys_off;               // first slot of each system (+ total), multiples of 64
+  std::vector<int> sys_off;               // first slot of each system (+ total)
+  bool packed = false;                    // the systems' slots follow each other (pack_slots)
   std::vector<int> sys_cap;               // capacity of each system
   std::vector<int> sys_n;                 // particles set per system
   std::vector<int> rogue_init;            // {INT_MAX, 0} per system
@@ -490,18 +491,21 @@ int32_t launch_step(mfixdem_handle* h) {
   const bool mixed = h->S.p.precision == MFIXDEM_MIXED;
   const BatchDev B = h->B;
   if (h->nsys > 1) {  // ensembles: pure DEM, per-system parameter tables
-    if (mixed) hipLaunchKernelGGL((k_step<true, MODE, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
-    else hipLaunchKernelGGL((k_step<false, MODE, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+    auto k = h->packed ? (mixed ? k_step<true, MODE, false, kPackedSystems>
+                                : k_step<false, MODE, false, kPackedSystems>)
+                       : (mixed ? k_step<true, MODE, false, kAlignedSystems>
+                                : k_step<false, MODE, false, kAlignedSystems>);
+    hipLaunchKernelGGL(k, grid, blk, 0, h->stream, P, a, B, lgw);
   } else if (P.nfs == 0) {  // more facets than wall slots: facet table and slot search
     const bool filt = h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012;
     if (filt && mixed)
-      hipLaunchKernelGGL((k_step<true, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+      hipLaunchKernelGGL((k_step<true, MODE, true, kOneSystem, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else if (filt)
-      hipLaunchKernelGGL((k_step<false, MODE, true, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+      hipLaunchKernelGGL((k_step<false, MODE, true, kOneSystem, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else if (mixed)
-      hipLaunchKernelGGL((k_step<true, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+      hipLaunchKernelGGL((k_step<true, MODE, false, kOneSystem, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else
-      hipLaunchKernelGGL((k_step<false, MODE, false, false, true>), grid, blk, 0, h->stream, P, a, B, lgw);
+      hipLaunchKernelGGL((k_step<false, MODE, false, kOneSystem, true>), grid, blk, 0, h->stream, P, a, B, lgw);
   } else if (h->S.p.interp_scheme != MFIXDEM_INTERP_GARG_2012) {
     if (mixed) hipLaunchKernelGGL((k_step<true, MODE, true>), grid, blk, 0, h->stream, P, a, B, lgw);
     else hipLaunchKernelGGL((k_step<false, MODE, true>), grid, blk, 0, h->stream, P, a, B, lgw);
@@ -585,7 +589,7 @@ int32_t do_bin(mfixdem_handle* h) {
   bp.xr = h->xr_pack;
   bp.xf = reinterpret_cast<float4*>(h->stage);
   auto bin = [&](auto many) -> int32_t {
-    constexpr bool kB = decltype(many)::value;
+    constexpr int kB = decltype(many)::value;
     hipLaunchKernelGGL(k_bin_count<kB>, dim3(nblk(n)), dim3(kBS), 0, h->stream, n, h->G,
                        h->pos[c], h->state[t], h->gid[t], h->dgc[t], h->fine_rank, h->fine_cnt,
                        nf, h->place, h->flags, h->B);
@@ -598,7 +602,9 @@ int32_t do_bin(mfixdem_handle* h) {
     HIPOK(hipGetLastError());
     return MFIXDEM_OK;
   };
-  CHECKRC(batch ? bin(std::true_type{}) : bin(std::false_type{}));
+  if (!batch) CHECKRC(bin(std::integral_constant<int, kOneSystem>{}));
+  else if (h->packed) CHECKRC(bin(std::integral_constant<int, kPackedSystems>{}));
+  else CHECKRC(bin(std::integral_constant<int, kAlignedSystems>{}));
   h->counts_zeroed = true;
   h->xr_packed = true;
   PermPtrs p{};
@@ -761,10 +767,13 @@ int32_t do_neighbour(mfixdem_handle* h) {
       auto rows = [&](auto lanes) {
         constexpr int kL = decltype(lanes)::value;
         const dim3 rg(nblk((int64_t)n * kL)), blk(kBS);
-        if (h->nsys > 1)
-          hipLaunchKernelGGL((k_own_rows<true, kL>), rg, blk, 0, h->stream, n, S, h->G, b, h->B);
-        else
-          hipLaunchKernelGGL((k_own_rows<false, kL>), rg, blk, 0, h->stream, n, S, h->G, b, h->B);
+        auto k = k_own_rows<kOneSystem, kL>;
+        if (h->nsys > 1) {
+          k = k_own_rows<kPackedSystems, kL>;
+          if constexpr (kL == 2)
+            if (!h->packed) k = k_own_rows<kAlignedSystems, kL>;
+        }
+        hipLaunchKernelGGL(k, rg, blk, 0, h->stream, n, S, h->G, b, h->B);
       };
       // Lanes per particle: all 14 cells of the half stencil side by side
       // while that leaves the chip room, 7 where rows are long (2 lanes then
@@ -1445,6 +1454,27 @@ int32_t setup_fine_cells(mfixdem_handle* h) {
                      h->B);
   HIPOK(hipGetLastError());
   return fill_i32(h->stream, h->fine_cnt, (int64_t)nf + ns, 0);
+}
+
+// Whether the systems of an ensemble, with these capacities, share wavefronts.
+// Slots aligned to 64 make at least one wavefront of every system, mostly
+// empty where systems are small, and take 1.6 KB of memory for every empty slot;
+// systems that follow each other fill their wavefronts, whose lanes then read
+// the parameters one by one.  Packed where the wavefronts would be half empty
+// and the chip (1,024 SIMDs) full of them.  Measured, 50 steps with 2
+// rebuilds, aligned / packed, loose and dense: 16 spheres in each of 1,024
+// systems 0.52 / 0.55 and 1.20 / 1.36 ms, 1,536 0.58 / 0.54 and 1.35 / 1.36,
+// 2,048 0.61 / 0.55 and 1.53 / 1.35, 8,192 1.68 / 0.87 and 3.80 / 2.26; in
+// 8,192 systems 4 spheres 1.63 / 0.59 and 3.65 / 1.42 (0.86 / 0.09 GB), 32
+// 1.73 / 1.49 and 4.32 / 3.97, 48 1.82 / 1.69 and 5.42 / 5.54, 64 1.76 / 2.21
+// and 6.00 / 8.37; one sphere in each of 40,000 systems 10.2 / 0.92.
+bool pack_slots(const std::vector<int>& cap) {
+  int64_t slots = 0, waves = 0;
+  for (int c : cap) {
+    slots += c;
+    waves += ((int64_t)c + 63) / 64;
+  }
+  return waves >= 1536 && slots <= 32 * waves;
 }
 
 // Device buffers, stream and events of a handle whose set-up (S, P, G,
@@ -2327,13 +2357,16 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
       delete h;
       return rc;
     }
-    const int64_t end = (int64_t)h->sys_off[s] + q.max_pip;
+    h->sys_cap[s] = q.max_pip;
+  }
+  h->packed = nsys > 1 && pack_slots(h->sys_cap);
+  for (int s = 0; s < nsys; s++) {
+    const int64_t end = (int64_t)h->sys_off[s] + h->sys_cap[s];
     if (end > INT_MAX / 4) {
       delete h;
       return MFIXDEM_ERR_ARG;
     }
-    h->sys_off[s + 1] = (int)(nsys > 1 ? (end + 63) / 64 * 64 : end);
-    h->sys_cap[s] = q.max_pip;
+    h->sys_off[s + 1] = (int)(nsys > 1 && !h->packed ? (end + 63) / 64 * 64 : end);
   }
   h->S = h->sys_setup[0];
   h->n = h->sys_off[nsys];
