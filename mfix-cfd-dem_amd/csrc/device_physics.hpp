@@ -117,9 +117,11 @@ struct PairOut {
 
 // a / b for several a: y is 1 / b correctly rounded, and one residual step
 // then gives the correctly rounded quotient (Markstein, IBM J. Res. Dev. 34,
-// 1990), in 3 operations instead of the 10 of a division of its own.  For |a|
-// above 1e-290 and b and 1 / b in the normal range.
-__device__ __forceinline__ double div_by(double a, double b, double y) {
+// 1990), in 3 operations instead of the 10 of a division of its own.  For b, y
+// and a / b in the normal range and |a| above 1e-290 (below that the residual
+// underflows and the last bit of the quotient may differ) or zero, whose
+// quotient is +0 whatever its sign.
+__host__ __device__ __forceinline__ double div_by(double a, double b, double y) {
   const double q = a * y;
   return __builtin_fma(__builtin_fma(-b, q, a), y, q);
 }
