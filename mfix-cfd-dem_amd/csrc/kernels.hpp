@@ -105,7 +105,7 @@ struct StepPtrs {
   const uint8_t* nbr_row;       // per entry: slot of its row mod 64, kRowOwn set for own entries
   const double* pft_in;         // tangential history [3*pair + d], valid where pfl is 1
   double* pft_out;
-  const uint8_t* pfl_in;        // 1: the pair's history is set; 0: it is zero (pft unread)
+  const uint8_t* pfl_in;        // 1: the pair's history is set; 0: it is zero, whatever pft holds
   uint8_t* pfl_out;
   double *fc, *tow;             // FC/TOW in slot order (unfused path)
   double *fc_id, *tow_id;       // FC/TOW in global-id order (inspection)
@@ -3481,14 +3481,6 @@ __global__ __launch_bounds__(kBS) void k_set_holes(int n, const int8_t* st, uint
     vel[d * S + q] = 0.0;
     omega[d * S + q] = 0.0;
   }
-}
-
-// PARTICLE_STATE in global-id order (a seeded particle is ENTERING)
-__global__ void k_scatter_gid_u8(int n, const int* gid, const uint8_t* src, int8_t* dst) {
-  const int i = blockIdx.x * kBS + threadIdx.x;
-  if (i >= n) return;
-  const uint8_t v = src[i];
-  dst[gid[i]] = (int8_t)(v == kSeeded ? kEntering : v);
 }
 
 }  // namespace mfixdem

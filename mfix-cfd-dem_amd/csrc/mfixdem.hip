@@ -181,7 +181,6 @@ struct mfixdem_handle {
   mfixdem_status st{};
   bool inited = false, gas_set = false, first_pass = true, binned = false;
   int debug = 0;
-  // kernel timing
   // kernel timing: a pool of events recorded around each timed launch and
   // read back in one go, so launches queue back to back while timed
   std::vector<hipEvent_t> ev;
@@ -728,7 +727,11 @@ int32_t do_neighbour(mfixdem_handle* h) {
     // 8 lanes to a row where rows are long or the chip has room, else 4.
     // Measured (k_place + k_sort_in, 8 / 4 / 2 lanes): 2,003 settled spheres,
     // 5.7 pairs each, 15 / 25 / 46 us; 301,057, 6.5 pairs, 149 / 181 / 268;
-    // 120,000, 4 pairs, 20 / 20 / 27; 1M, 1.6 pairs, 119 / 89 / 90.
+    // 120,000, 4 pairs, 20 / 20 / 27; 1M, 1.6 pairs, 119 / 89 / 90.  A step
+    // with a rebuild in it, 8 / 4 lanes, spheres loose (25 %) and touching in
+    // a cubic lattice: 24,001 45.8 / 46.5 and 69.9 / 72.9 us, 32,003 48.4 /
+    // 47.5 and 72.7 / 76.0, 40,009 50.3 / 50.3 and 78.1 / 81.7, 48,017 54.6 /
+    // 54.0 and 82.6 / 86.1, 200,003 82.0 / 77.6 and 159 / 164.
     if (h->n_pairs >= 4 * (int64_t)n || n <= 32768) go(std::integral_constant<int, 8>{});
     else go(std::integral_constant<int, 4>{});
     HIPOK(hipGetLastError());
@@ -780,8 +783,13 @@ int32_t do_neighbour(mfixdem_handle* h) {
       // have more hits than their LDS lists hold), else 2.  Measured (2 / 7 /
       // 14 lanes): 2,003 settled spheres 39 / 14 / 11 us; 301,057 211 / 170 /
       // 192; 120,000 at 4 pairs each 30 / 31 / 40; 1M at 1.6, 126 / 181 / 262.
-      // (Ensembles of any size but a small one keep 2, whose wavefronts read one
-      // system's grid.)
+      // A step with a rebuild in it, spheres loose (25 %) and touching in a
+      // cubic lattice: 8,009 49.5 / 43.7 / 43.4 and 71.5 / 66.7 / 65.5 us,
+      // 20,011 50.9 / 43.8 / 44.2 and 73.9 / 70.2 / 70.8, 32,003 52.4 / 47.5 /
+      // 49.8 and 78.7 / 76.0 / 77.9, 65,003 57.5 / 56.0 / 59.9 and 92.9 / 92.7 /
+      // 103, 80,021 60.9 / 61.2 / 63.4 and 106 / 109 / 114.
+      // (Ensembles of any size but a small one keep 2, with which an aligned
+      // system's wavefronts read one grid.)
       if (n <= 20480) rows(std::integral_constant<int, 14>{});
       else if (h->nsys == 1 && (n <= 65536 || (h->n_pairs >= 5 * (int64_t)n && n < (1 << 24))))
         rows(std::integral_constant<int, 7>{});
