@@ -96,3 +96,27 @@ def test_members_of_all_sizes_share_wavefronts(precision):
     e, want = check(variants, 1709, kind)
     assert [w[1].rogue_deleted for w in want] == [int(k in (2, 5)) for k in range(len(caps))]
     e.close()
+
+
+@pytest.mark.parametrize("tuning", [(1.0, abi.ROWS_WAVE128), (1.6, abi.ROWS_WAVE192),
+                                    (2.5, abi.ROWS_THREAD)])
+def test_tuning_choices_of_a_packed_ensemble(tuning):
+    variants = [member(c, c, k) for k, c in enumerate((1, 20, 3, 40, 7, 30))]
+    e = Ensemble([variants[k % 6][0] for k in range(1800)])
+    for k in range(1800):
+        e.set_particles(k, variants[k % 6][1])
+    e.set_tuning(*tuning)
+    e.init()
+    e.run(1, 25)
+    want = []
+    for p, parts in variants:
+        o = OracleSystem(p)
+        o.set_particles(parts)
+        o.init()
+        o.run(1, 25)
+        want.append(o.get_particles())
+        o.close()
+    for k in list(range(0, 1800, 7)) + [1799]:
+        for a, b, what in zip(e.get_particles(k), want[k % 6], ("pos", "vel", "omega", "state")):
+            assert np.array_equal(a, b), (k, what)
+    e.close()
