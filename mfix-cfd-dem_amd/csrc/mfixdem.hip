@@ -2390,7 +2390,7 @@ int32_t mfixdem_ensemble_create(int32_t nsys, const mfixdem_params* p, mfixdem_h
     const int slots = h->sys_off[s + 1] - h->sys_off[s];
     if ((nsys > 1 ? member_grid(S.p, slots, gtab[s], nfine)
                   : search_grid(S.p, slots, gtab[s], nfine)) != MFIXDEM_OK ||
-        nfine > INT_MAX / 2 - cell_off[s]) {
+        nfine > INT_MAX - (1 << 20) - cell_off[s]) {
       delete h;
       return MFIXDEM_ERR_UNSUPPORTED;
     }
